@@ -83,14 +83,17 @@ def csr_flops(name, nw, nnz_spvn, nnz_spvnT):
     return None if c is None else 8.0 * c
 
 
-def contraction_spins_per_launch(M, N, K, nw):
+def contraction_spins_per_launch(M, N, K, nw, mode=None):
     """Spin blocks per launch of the bias-shaped contraction (G against the
-    K Cholesky rows, the bias and the Coulomb term).  The library splits its
+    K Cholesky rows, the bias and the Coulomb term).  In FP64 one launch
+    covers both spins from N*M = 512 on.  Otherwise the library splits its
     k = N*M range into S chunks, S doubling from 1 while 2*S*tiles < 2048
     (tiles = ceil(nw/128) * ceil(K/64)) and N*M/(2S) stays a multiple of 64;
     with S > 1 one launch covers both spins, otherwise each spin is its own
     launch."""
     NM = N * M
+    if mode == "fp64_dense":
+        return 2 if NM >= 512 else 1
     tiles = -(-nw // 128) * -(-K // 64)
     S = 1
     while S < 16 and 2 * S * tiles < 2048 and NM % (2 * S) == 0 and (NM // (2 * S)) % 64 == 0:
@@ -101,7 +104,7 @@ def contraction_spins_per_launch(M, N, K, nw):
 def kernel_flops(name, M, N, K, nw, mode=None):
     """Algorithmic real flops per launch (8 per complex multiply-add).  The
     FP64 CSR mode's dense bias product contracts both spins in one launch."""
-    sp = 2 if mode == "fp64_csr" else contraction_spins_per_launch(M, N, K, nw)
+    sp = 2 if mode == "fp64_csr" else contraction_spins_per_launch(M, N, K, nw, mode)
     c = {
         "vhs_gemm": nw * M * M * K,
         "prop_taylor": 2 * nw * M * M * N,

@@ -14,6 +14,7 @@
 #include "common.hpp"
 #include "gemm.hpp"
 #include "gemm_b16.hpp"
+#include "gemm_f64.hpp"
 #include "kernels.hpp"
 #include "propagate.hpp"
 
@@ -344,13 +345,39 @@ inline int nblk(long n, int t) { return (int)std::min<long>((n + t - 1) / t, 655
 struct TileCfg {
   int BM, BNC, WM, WN;
 };
-// candidates per precision (BKC is 8 complex for FP64/FP32, 16 for BF16)
-constexpr TileCfg kCfgF64[] = {{32, 16, 1, 1}, {64, 32, 2, 2}, {128, 64, 2, 2}};
+// candidates per precision (BKC is 8 complex for FP32, 16 for BF16)
 constexpr TileCfg kCfgF32[] = {{32, 16, 1, 1}, {128, 64, 2, 2}, {128, 128, 2, 2}};
 constexpr TileCfg kCfgB16[] = {{32, 16, 1, 1}, {128, 64, 2, 2}, {128, 128, 2, 2}, {256, 64, 4, 2}, {64, 64, 2, 2}};
 
-template <int CP> constexpr int ncfg() { return CP == CP_F64 ? 3 : (CP == CP_F32 ? 3 : 5); }
-template <int CP> constexpr TileCfg cfg_at(int i) { return CP == CP_F64 ? kCfgF64[i] : (CP == CP_F32 ? kCfgF32[i] : kCfgB16[i]); }
+template <int CP> constexpr int ncfg() { return CP == CP_F32 ? 3 : 5; }
+template <int CP> constexpr TileCfg cfg_at(int i) { return CP == CP_F32 ? kCfgF32[i] : kCfgB16[i]; }
+
+// Time each of n candidates (results are discarded), in two rounds keeping
+// each one's faster round; `best` starts as the default.
+template <class F> int tune_tiles(afqmc_ctx* c, int n, int& best, F&& run)
+{
+  const bool prof = c->prof;
+  c->prof = false;
+  hipEvent_t e0 = get_event(c), e1 = get_event(c);
+  std::vector<float> tms(n, 1e30f);
+  for (int round = 0; round < 2; round++)
+    for (int i = 0; i < n; i++) {
+      RET(run(i));  // warm
+      (void)hipEventRecord(e0, c->stream);
+      for (int rep = 0; rep < 3; rep++) RET(run(i));
+      (void)hipEventRecord(e1, c->stream);
+      (void)hipEventSynchronize(e1);
+      float ms = 0.f;
+      (void)hipEventElapsedTime(&ms, e0, e1);
+      tms[i] = std::min(tms[i], ms);
+    }
+  for (int i = 0; i < n; i++)
+    if (tms[i] < tms[best]) best = i;
+  c->evpool.push_back(e0);
+  c->evpool.push_back(e1);
+  c->prof = prof;
+  return AFQMC_OK;
+}
 
 template <int CP, class AT, class BT, class OT, bool AK, bool BK, int CI>
 int zgemm_cfg(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch)
@@ -406,8 +433,8 @@ int zgemm_run(afqmc_ctx* c, const char* name, const ZGemmArgs& a, int batch, int
 
 template <int CP> int default_cfg(const ZGemmArgs& a)
 {
-  if (a.m >= 96 && a.n >= 48) return CP == CP_F64 ? 2 : 1;  // 128 x 64 tiles
-  return 0;                                                 // one-wave 32 x 16 tiles
+  if (a.m >= 96 && a.n >= 48) return 1;  // 128 x 64 tiles
+  return 0;                              // one-wave 32 x 16 tiles
 }
 
 // Split-BF16 products whose operands are both split-BF16 with k contiguous
@@ -468,28 +495,8 @@ template <class OT, int NP = 2> int zgemm_ring(afqmc_ctx* c, const char* name, c
   auto it = c->tune.find(key);
   if (it != c->tune.end() && !c->tuning) return ring_run<OT, NP>(c, name, a, batch, it->second);
   if (!c->tuning) return ring_run<OT, NP>(c, name, a, batch, ring_default(a));
-  const bool prof = c->prof;
-  c->prof = false;
-  hipEvent_t e0 = get_event(c), e1 = get_event(c);
-  float tms[kNRing];
-  for (int ri = 0; ri < kNRing; ri++) tms[ri] = 1e30f;
-  for (int round = 0; round < 2; round++)
-    for (int ri = 0; ri < kNRing; ri++) {
-      RET((ring_run<OT, NP>(c, name, a, batch, ri)));  // warm
-      (void)hipEventRecord(e0, c->stream);
-      for (int rep = 0; rep < 3; rep++) RET((ring_run<OT, NP>(c, name, a, batch, ri)));
-      (void)hipEventRecord(e1, c->stream);
-      (void)hipEventSynchronize(e1);
-      float ms = 0.f;
-      (void)hipEventElapsedTime(&ms, e0, e1);
-      tms[ri] = std::min(tms[ri], ms);
-    }
   int best = ring_default(a);
-  for (int ri = 0; ri < kNRing; ri++)
-    if (tms[ri] < tms[best]) best = ri;
-  c->evpool.push_back(e0);
-  c->evpool.push_back(e1);
-  c->prof = prof;
+  RET(tune_tiles(c, kNRing, best, [&](int ri) { return ring_run<OT, NP>(c, name, a, batch, ri); }));
   c->tune[key] = best;
   return ring_run<OT, NP>(c, name, a, batch, best);
 }
@@ -511,12 +518,127 @@ bool ring3_ok(const ZGemmArgs& a)
          ((uintptr_t)a.B & 15) == 0 && ((uintptr_t)a.A3 & 15) == 0 && ((uintptr_t)a.B3 & 15) == 0 && !a.conjb;
 }
 
+// FP64 products (zgemm_f64_kernel): every operand order, tile candidates
+// (rows, complex columns, waves, LDS stages).
+struct F64Cfg {
+  int BM, BN, WM, WN, S;
+};
+constexpr F64Cfg kF64[] = {{32, 32, 2, 2, 3}, {64, 64, 2, 2, 2}, {128, 64, 4, 2, 2}};
+constexpr int kNF64 = 3;
+
+F64Args f64args(int m, int n, int k)
+{
+  F64Args a;
+  std::memset(&a, 0, sizeof(a));
+  a.m = a.mi = m;
+  a.n = a.ni = n;
+  a.k = k;
+  a.bdiv = 1;
+  a.ar = 1.0;
+  return a;
+}
+
+// The tile with the least estimated time: padded tiles per CU times their
+// area over the rate each reaches with the CU full (57.4, 62.7 and 63.9
+// TFLOP/s at 2048 x 128 x 128 x 512); a CU with a single workgroup has too
+// few waves to cover the LDS reads and reaches about 0.7 of it.
+int f64_default(const F64Args& a, int batch)
+{
+  constexpr double rate[kNF64] = {57.4, 62.7, 63.9};
+  int best = 0;
+  double tb = 1e300;
+  for (int i = 0; i < kNF64; i++) {
+    const double tiles = (double)((a.m + kF64[i].BM - 1) / kF64[i].BM) * ((a.n + kF64[i].BN - 1) / kF64[i].BN) * batch;
+    const double percu = std::ceil(tiles / 256.0);
+    const double t = percu * kF64[i].BM * kF64[i].BN / (rate[i] * (percu < 2.0 ? 0.7 : 1.0));
+    if (t < tb) {
+      tb = t;
+      best = i;
+    }
+  }
+  return best;
+}
+
+template <class OZ, int CI, bool DMA> int f64_cfg(afqmc_ctx* c, const char* name, F64Args a, int batch)
+{
+  constexpr F64Cfg t = kF64[CI];
+  a.MT = (a.m + t.BM - 1) / t.BM;
+  a.NT = (a.n + t.BN - 1) / t.BN;
+  const long tiles = (long)a.MT * a.NT * batch;
+  if (tiles > 2147483647L) return fail(c, AFQMC_ERR_SHAPE, "GEMM grid too large");
+  return launch(c, name, [&]() {
+    hipLaunchKernelGGL((zgemm_f64_kernel<OZ, t.BM, t.BN, t.WM, t.WN, t.S, DMA>), dim3((unsigned)tiles),
+                       dim3(64 * t.WM * t.WN), 0, c->stream, a);
+  });
+}
+
+template <class OZ> int f64_run(afqmc_ctx* c, const char* name, const F64Args& a, int batch, int ci)
+{
+  // the direct loads move 16 aligned bytes; a caller's own device pointers
+  // (the allocation-free entry point) may hold less
+  if ((((uintptr_t)a.A | (uintptr_t)a.B) & 15) != 0) return f64_cfg<OZ, 0, false>(c, name, a, batch);
+  switch (ci) {
+  case 1: return f64_cfg<OZ, 1, true>(c, name, a, batch);
+  case 2: return f64_cfg<OZ, 2, true>(c, name, a, batch);
+  default: return f64_cfg<OZ, 0, true>(c, name, a, batch);
+  }
+}
+
+template <class OZ> int zgemm64(afqmc_ctx* c, const char* name, const F64Args& a, int batch)
+{
+  if (a.m <= 0 || a.n <= 0 || batch <= 0) return AFQMC_OK;
+  if (c->force_cfg > 0 && c->force_cfg <= kNF64) return f64_run<OZ>(c, name, a, batch, c->force_cfg - 1);
+  if (c->tune.empty() && !c->tuning) return f64_run<OZ>(c, name, a, batch, f64_default(a, batch));
+  char keyb[160];
+  std::snprintf(keyb, sizeof(keyb), "%s/f64/%d/%d/%d/%d", name, a.m, a.n, a.k, batch);
+  const std::string key(keyb);
+  auto it = c->tune.find(key);
+  if (it != c->tune.end() && !c->tuning) return f64_run<OZ>(c, name, a, batch, it->second);
+  int best = f64_default(a, batch);
+  if (!c->tuning) return f64_run<OZ>(c, name, a, batch, best);
+  RET(tune_tiles(c, kNF64, best, [&](int ci) { return f64_run<OZ>(c, name, a, batch, ci); }));
+  c->tune[key] = best;
+  return f64_run<OZ>(c, name, a, batch, best);
+}
+
+// a strided FP64 product as the other precisions' call sites state it
+template <class OZ> int zgemm64(afqmc_ctx* c, const char* name, const ZGemmArgs& z, int batch)
+{
+  F64Args a = f64args(z.m, z.n, z.k);
+  a.A = z.A;
+  a.sam = z.sam;
+  a.sak = z.sak;
+  a.sa1 = z.sa1;
+  a.sa2 = z.sa2;
+  a.B = z.B;
+  a.sbn = z.sbn;
+  a.sbk = z.sbk;
+  a.sb1 = z.sb1;
+  a.sb2 = z.sb2;
+  a.conjb = z.conjb;
+  a.C = z.C;
+  a.scm = z.scm;
+  a.scn = z.scn;
+  a.sc1 = z.sc1;
+  a.sc2 = z.sc2;
+  a.bdiv = z.bdiv > 0 ? z.bdiv : 1;
+  a.ar = z.ar;
+  a.ai = z.ai;
+  a.br = z.br;
+  a.bi = z.bi;
+  a.ktri = z.ktri;
+  return zgemm64<OZ>(c, name, a, batch);
+}
+
 template <int CP, class AT, class BT, class OT, bool AK, bool BK>
 int zgemm(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch)
 {
   if (a.m <= 0 || a.n <= 0 || batch <= 0) return AFQMC_OK;
   if (a.bdiv <= 0) a.bdiv = 1;
-  if constexpr (CP == CP_BF16X6) {
+  if constexpr (CP == CP_F64) {
+    static_assert(std::is_same<AT, double>::value && std::is_same<BT, double>::value, "FP64 products take FP64 operands");
+    return zgemm64<typename ztype<OT>::type>(c, name, a, batch);
+  } else if constexpr (CP == CP_BF16X6) {
     static_assert(std::is_same<AT, bfs>::value && std::is_same<BT, bfs>::value && AK && BK,
                   "three-piece products take split operands with k contiguous");
     if (!ring3_ok(a)) return fail(c, AFQMC_ERR_UNSUPPORTED, std::string(name) + ": three-piece operand layout");
@@ -538,31 +660,8 @@ int zgemm(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch)
   auto it = c->tune.find(key);
   if (it != c->tune.end() && !c->tuning) return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, it->second);
   if (!c->tuning) return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, default_cfg<CP>(a));
-  // tuning: time each candidate (results of this call are discarded), in
-  // two rounds keeping each candidate's faster round
-  const bool prof = c->prof;
-  c->prof = false;
-  hipEvent_t e0 = get_event(c), e1 = get_event(c);
-  const int def = default_cfg<CP>(a);
-  float tms[8];
-  for (int ci = 0; ci < ncfg<CP>(); ci++) tms[ci] = 1e30f;
-  for (int round = 0; round < 2; round++)
-    for (int ci = 0; ci < ncfg<CP>(); ci++) {
-      RET((zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, ci)));  // warm
-      (void)hipEventRecord(e0, c->stream);
-      for (int rep = 0; rep < 3; rep++) RET((zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, ci)));
-      (void)hipEventRecord(e1, c->stream);
-      (void)hipEventSynchronize(e1);
-      float ms = 0.f;
-      (void)hipEventElapsedTime(&ms, e0, e1);
-      tms[ci] = std::min(tms[ci], ms);
-    }
-  int best = def;
-  for (int ci = 0; ci < ncfg<CP>(); ci++)
-    if (tms[ci] < tms[best]) best = ci;
-  c->evpool.push_back(e0);
-  c->evpool.push_back(e1);
-  c->prof = prof;
+  int best = default_cfg<CP>(a);
+  RET(tune_tiles(c, ncfg<CP>(), best, [&](int ci) { return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, ci); }));
   c->tune[key] = best;
   return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, best);
   }
@@ -669,32 +768,33 @@ int gj_inverse(afqmc_ctx* c, zd* T, zd* Tinv, zd* det, long dq, long dr)
   return gj_inverse_into(c, T, Tinv, det, dq, dr, c->flags, c->dcache, c->Wl, c->lcache);
 }
 
-// T1[w][s] = W[w][s]^T * trial_s  (N x N, k = M), all walkers and spins
-int overlap_matrices(afqmc_ctx* c)
+// T1[w][s] = W[w][s]^T * trial_s  (N x N, k = M) for nw walkers: the walkers'
+// rows (w, a) of one spin are one tall product against that spin's trial, so
+// only its last row tile is partial
+int overlap_product(afqmc_ctx* c, const zd* W, const zd* trial, zd* T1)
 {
   const int M = c->M, N = c->N;
-  ZGemmArgs a = gargs();
-  a.A = c->W;
+  const long MN = (long)M * N, NN = (long)N * N;
+  F64Args a = f64args(c->nw * N, N, M);
+  a.mi = N;
+  a.A = W;
   a.sam = 1;
+  a.samo = 2 * MN;
   a.sak = N;
-  a.sa1 = 2L * M * N;
-  a.sa2 = (long)M * N;
-  a.B = c->trial;
+  a.sa1 = MN;
+  a.B = trial;
   a.sbn = 1;
   a.sbk = N;
-  a.sb1 = 0;
-  a.sb2 = (long)M * N;
-  a.C = c->T1;
+  a.sb1 = MN;
+  a.C = T1;
   a.scm = N;
+  a.scmo = 2 * NN;
   a.scn = 1;
-  a.sc1 = 2L * N * N;
-  a.sc2 = (long)N * N;
-  a.bdiv = 2;
-  a.m = N;
-  a.n = N;
-  a.k = M;
-  return zgemm<CP_F64, double, double, double, false, false>(c, "ovlp_gemm", a, 2 * c->nw);
+  a.sc1 = NN;
+  return zgemm64<zd>(c, "ovlp_gemm", a, 2);
 }
+
+int overlap_matrices(afqmc_ctx* c) { return overlap_product(c, c->W, c->trial, c->T1); }
 
 // Gc(a,k) = sum_b T1inv(a,b) W(k,b) for every walker-spin pair; output
 // strides are set by the caller.
@@ -717,6 +817,14 @@ ZGemmArgs gc_args(const afqmc_ctx* c)
   a.n = M;
   a.k = N;
   return a;
+}
+
+// G is held walker-first, [nw][2NM], where only GEMMs read it (written in
+// rows of M instead of single values nw apart: gc_gemm 316 -> 105 us at 256
+// walkers of 64 x 256); the CSR products read it walker-last.
+bool g_wfirst(const afqmc_ctx* c)
+{
+  return c->mode != AFQMC_FP64_CSR || (c->sptd && !c->v_rp);
 }
 
 // FP64 copy of G in [nw][2NM] for the energy of the mixed modes: rebuilt
@@ -762,7 +870,7 @@ int do_mdm(afqmc_ctx* c)
   c->g_fresh = true;
   ZGemmArgs a = gc_args(c);
   a.C = c->G;
-  if (c->mode == AFQMC_FP64_CSR) {
+  if (!g_wfirst(c)) {
     // G[(s*N + a)*M + k][w]
     a.scm = (long)M * nw;
     a.scn = nw;
@@ -798,6 +906,60 @@ int do_overlaps(afqmc_ctx* c)
   return AFQMC_OK;
 }
 
+// A workspace of at least `bytes` for the partial sums of split contractions.
+int need_vws(afqmc_ctx* c, size_t bytes)
+{
+  if (c->vws_bytes >= bytes) return AFQMC_OK;
+  dfree(c, c->vws);
+  c->vws_bytes = bytes;
+  return dalloc_bytes(c, &c->vws, bytes);
+}
+
+// Chunks of a k sum of length kt whose output is m x n: enough 64 x 64 tiles
+// for four workgroups per CU, each chunk at least 256 long and a multiple of
+// the k-tile, at most smax of them; the last one may be shorter.
+long f64_chunk(long m, long n, long kt, int items, int smax)
+{
+  const long tiles = ((m + 63) / 64) * ((n + 63) / 64) * items;
+  const long s = std::max<long>(1, std::min<long>(std::min<long>(smax, kt / 256), (1024 + tiles - 1) / tiles));
+  return (((kt + s - 1) / s) + 7) / 8 * 8;
+}
+
+// vbias(w, n) = sum_{s,j} G(w, s, j) Lt(s, n, j) in FP64: the partial
+// products (spin, chunk of j) run as one batch into a workspace, summed in
+// chunk order.  (200 walkers, 999 vectors, N M = 15250: 12.6 ms unsplit in
+// 32 workgroups per spin.)
+int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const char* name, const char* rname)
+{
+  const long NM = (long)c->N * c->M, nw = c->nw, K = c->K;
+  const long chunk = f64_chunk(nw, K, NM, 2, 16);
+  const int S = (int)((NM + chunk - 1) / chunk);
+  RET(need_vws(c, sizeof(zd) * 2 * S * nw * K));
+  F64Args a = f64args((int)nw, (int)K, (int)chunk);
+  a.ktot = NM;
+  a.A = G;  // batch (spin, chunk)
+  a.sam = 2 * NM;
+  a.sak = 1;
+  a.sa1 = NM;
+  a.sa2 = chunk;
+  a.B = Lt;
+  a.sbn = NM;
+  a.sbk = 1;
+  a.sb1 = K * NM;
+  a.sb2 = chunk;
+  a.C = c->vws;
+  a.scm = K;
+  a.scn = 1;
+  a.sc1 = S * nw * K;
+  a.sc2 = nw * K;
+  a.bdiv = S;
+  RET(zgemm64<zd>(c, name, a, 2 * S));
+  return launch(c, rname, [&]() {
+    hipLaunchKernelGGL((zsum_slices_kernel<zd>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const zd*)c->vws,
+                       out, nw * K, 2 * S);
+  });
+}
+
 // vbias(w, n) = sum_{s,j} G(w, s, j) Lt(s, n, j) in dense modes.  With few
 // output tiles (walkers x vectors) the long j sum is split into S chunks:
 // the 2S partial products (spin, chunk) run as one batched GEMM into a
@@ -808,6 +970,9 @@ int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, 
                          const char* rname = "vbias_reduce")
 {
   const long NM = (long)c->N * c->M, nw = c->nw, K = c->K;
+  if constexpr (CP == CP_F64) {
+    if (NM >= 512) return dense_contract_f64(c, (const zd*)Gp, (const zd*)Lt, out, name, rname);
+  }
   const long tiles = ((nw + 127) / 128) * ((K + 63) / 64);
   int S = 1;
   while (S < 16 && 2 * S * tiles < 2048 && NM % (2 * S) == 0 && (NM / (2 * S)) % 64 == 0) S *= 2;
@@ -838,12 +1003,7 @@ int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, 
   // partials in FP32 for the FP32/BF16 contractions, FP64 otherwise
   using PT = typename std::conditional<CP == CP_F64, double, float>::type;
   using PZ = typename ztype<PT>::type;
-  const size_t need = sizeof(PZ) * 2 * S * nw * K;
-  if (c->vws_bytes < need) {
-    dfree(c, c->vws);
-    c->vws_bytes = need;
-    RET(dalloc_bytes(c, &c->vws, need));
-  }
+  RET(need_vws(c, sizeof(PZ) * 2 * S * nw * K));
   const long chunk = NM / S;
   ZGemmArgs a = gargs();
   a.A = Gp;  // batch b = (spin, chunk): A offset spin*NM + chunk*NM/S
@@ -883,27 +1043,21 @@ int do_mdm_full(afqmc_ctx* c)
   const long MM = (long)M * M, MN = (long)M * N;
   if (!c->Gfull) RET(dalloc(c, &c->Gfull, 2 * MM * nw));
   RET(do_mdm(c));
-  ZGemmArgs a = gargs();
+  // columns (k, w) of one spin side by side: one M x M*nw product per spin
+  F64Args a = f64args(M, M * nw, N);
   a.A = c->trial;  // A(i, a) = trialwfn_s[i][a]
   a.sam = N;
   a.sak = 1;
-  a.sa1 = 0;
-  a.sa2 = MN;
-  a.B = c->G;  // B(k, a) = Gc[(s N + a) M + k][w]
-  a.sbn = nw;
+  a.sa1 = MN;
+  a.B = c->G;  // B((k, w), a) = Gc[(s N + a) M + k][w]
+  a.sbn = 1;
   a.sbk = (long)M * nw;
-  a.sb1 = 1;
-  a.sb2 = MN * nw;
-  a.C = c->Gfull;  // C(i, k) = G[(s M + i) M + k][w]
+  a.sb1 = MN * nw;
+  a.C = c->Gfull;  // C(i, (k, w)) = G[(s M + i) M + k][w]
   a.scm = (long)M * nw;
-  a.scn = nw;
-  a.sc1 = 1;
-  a.sc2 = MM * nw;
-  a.bdiv = 2;
-  a.m = M;
-  a.n = M;
-  a.k = N;
-  return zgemm<CP_F64, double, double, double, true, false>(c, "gfull_gemm", a, 2 * nw);
+  a.scn = 1;
+  a.sc1 = MM * nw;
+  return zgemm64<zd>(c, "gfull_gemm", a, 2);
 }
 
 // base::get_vbias(Spvn, G, vbias, false) (vbias.hpp:65-82):
@@ -920,43 +1074,41 @@ int do_vbias_full(afqmc_ctx* c)
   return AFQMC_OK;
 }
 
-// FP64_CSR bias product with SpvnT kept dense: vbias[K][nw] = SpvnT[K][2NM]
-// G[2NM][nw] (walker-last) on FP64 MFMA, the long sum split into S chunks
-// (a batched GEMM into a workspace, then summed in FP64 in chunk order).
+// FP64_CSR bias product with SpvnT kept dense: vbias[K][nw] = SpvnT[K][2NM] G
+// on FP64 MFMA, the long sum split into S chunks (a batched GEMM into a
+// workspace, then summed in FP64 in chunk order).
 int dense_csr_vbias(afqmc_ctx* c)
 {
   const long NAK = 2L * c->N * c->M, nw = c->nw, K = c->K;
-  const long tiles = ((K + 63) / 64) * ((nw + 31) / 32);
-  int S = 1;
-  while (S < 32 && S * tiles < 1024 && NAK % (2 * S) == 0 && (NAK / (2 * S)) % 64 == 0) S *= 2;
-  const long chunk = NAK / S;
-  ZGemmArgs a = gargs();
+  const long chunk = f64_chunk(K, nw, NAK, 1, 32);
+  const int S = (int)((NAK + chunk - 1) / chunk);
+  F64Args a = f64args((int)K, (int)nw, (int)chunk);
+  a.ktot = NAK;
+  a.bdiv = S;
   a.A = c->sptd;
   a.sam = NAK;
   a.sak = 1;
+  a.sa2 = chunk;  // item b: columns b*chunk .. of SpvnT and of G
   a.B = c->G;
-  a.sbn = 1;
-  a.sbk = nw;
-  a.m = (int)K;
-  a.n = (int)nw;
-  a.k = (int)chunk;
+  if (g_wfirst(c)) {
+    a.sbn = NAK;
+    a.sbk = 1;
+    a.sb2 = chunk;
+  } else {
+    a.sbn = 1;
+    a.sbk = nw;
+    a.sb2 = chunk * nw;
+  }
   a.scm = nw;
   a.scn = 1;
   if (S == 1) {
     a.C = c->vbias;
-    return zgemm<CP_F64, double, double, double, true, false>(c, "vbias_gemm", a, 1);
+    return zgemm64<zd>(c, "vbias_gemm", a, 1);
   }
-  const size_t need = sizeof(zd) * S * K * nw;
-  if (c->vws_bytes < need) {
-    dfree(c, c->vws);
-    c->vws_bytes = need;
-    RET(dalloc_bytes(c, &c->vws, need));
-  }
-  a.sa1 = chunk;  // batch b: columns b*chunk .. of SpvnT, rows b*chunk .. of G
-  a.sb1 = chunk * nw;
+  RET(need_vws(c, sizeof(zd) * S * K * nw));
   a.C = c->vws;
-  a.sc1 = K * nw;
-  RET((zgemm<CP_F64, double, double, double, true, false>(c, "vbias_gemm", a, S)));
+  a.sc2 = K * nw;
+  RET(zgemm64<zd>(c, "vbias_gemm", a, S));
   return launch(c, "vbias_reduce", [&]() {
     hipLaunchKernelGGL((zsum_slices_kernel<zd>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const zd*)c->vws,
                        c->vbias, nw * K, S);
@@ -1060,6 +1212,72 @@ int do_vhs(afqmc_ctx* c)
     return zgemm<CP_BF16X6, bfs, bfs, bfs, true, true>(c, "vhs_gemm", a, 1);
   }
   return zgemm<CP_BF16X3, bfs, bfs, bfs, true, true>(c, "vhs_gemm", a, 1);
+}
+
+// The FP64 propagator (see propagate_chain for the series).  S and the Horner
+// terms hold each (walker, spin) M x N block transposed ([N][M]), so both
+// spins of a walker are 2N contiguous rows and every product reads both
+// operands k-contiguous: P W as (w, s, a) rows against P, each Horner step as
+// the walker's 2N rows against V, P U as P against (w, s, a) columns.
+int propagate_f64(afqmc_ctx* c, const zd* V)
+{
+  const int M = c->M, N = c->N, nw = c->nw;
+  const long MN = (long)M * N, MM = (long)M * M;
+  zd* S = (zd*)c->S;
+  {  // S[(w, s, a)][i] = sum_k W[w][s][k][a] P[i][k]
+    F64Args a = f64args(2 * nw * N, M, M);
+    a.mi = N;
+    a.A = c->W;
+    a.sam = 1;
+    a.samo = MN;
+    a.sak = N;
+    a.B = c->propg;
+    a.sbn = M;
+    a.sbk = 1;
+    a.C = S;
+    a.scm = M;
+    a.scmo = MN;
+    a.scn = 1;
+    RET(zgemm64<zd>(c, "prop_pw", a, 1));
+  }
+  const zd* prev = S;
+  zd* bufs[2] = {(zd*)c->Ta, (zd*)c->Tb};
+  for (int k = 6; k >= 1; k--) {
+    // U_k[(s, a)][i] = S[(s, a)][i] + (i/k) sum_j U_{k+1}[(s, a)][j] V[i][j]
+    F64Args a = f64args(2 * N, M, M);
+    a.A = prev;
+    a.sam = M;
+    a.sak = 1;
+    a.sa1 = 2 * MN;
+    a.B = V;
+    a.sbn = M;
+    a.sbk = 1;
+    a.sb1 = MM;
+    a.C = bufs[k & 1];
+    a.F = S;
+    a.scm = a.sfm = M;
+    a.scn = a.sfn = 1;
+    a.sc1 = 2 * MN;
+    a.ar = 0.0;
+    a.ai = 1.0 / (double)k;
+    RET(zgemm64<zd>(c, "prop_taylor", a, nw));
+    prev = bufs[k & 1];
+  }
+  // W[w][s][i][a] = sum_k P[i][k] U_1[(w, s, a)][k]
+  F64Args a = f64args(M, 2 * nw * N, M);
+  a.ni = N;
+  a.A = c->propg;
+  a.sam = M;
+  a.sak = 1;
+  a.B = prev;
+  a.sbn = M;
+  a.sbno = MN;
+  a.sbk = 1;
+  a.C = c->W;
+  a.scm = N;
+  a.scn = 1;
+  a.scno = MN;
+  return zgemm64<zd>(c, "prop_ps", a, 1);
 }
 
 // W <- P * T6(V) * P * W per walker and spin (afqmc_sys.hpp:146-173), T6 the
@@ -1268,9 +1486,8 @@ int do_propagate(afqmc_ctx* c)
   c->g_fresh = false;
   if (c->three & 4) return propagate_three(c);
   if (fused_prop_ok(c)) return propagate_fused(c);
-  if (c->mode == AFQMC_FP64_CSR) return propagate_chain<CP_F64, double, double, double, double>(c, c->propg, c->vHSw);
-  if (c->mode == AFQMC_FP64_DENSE)
-    return propagate_chain<CP_F64, double, double, double, double>(c, c->propg, c->vHS);
+  if (c->mode == AFQMC_FP64_CSR) return propagate_f64(c, c->vHSw);
+  if (c->mode == AFQMC_FP64_DENSE) return propagate_f64(c, (const zd*)c->vHS);
   if (c->mode == AFQMC_MIXED_FP32)
     return propagate_chain<CP_F32, float, float, float, float>(c, c->propg32, c->vHS);
   return propagate_chain<CP_BF16X3, float, bfs, bfs, bfs>(c, c->propg32, c->vHS);
@@ -1552,7 +1769,29 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     if constexpr (CP == CP_BF16X6) {
       return fail(c, AFQMC_ERR_STATE, "three-piece exchange without its dense block");
     } else {
-      RET((zgemm<CP, LT_, GT, YT, true, true>(c, "energy_y_gemm", a, 2 * nw)));
+      if constexpr (CP == CP_F64) {
+        // the walkers' rows b of G side by side as columns (w, b)
+        F64Args f = f64args(cnt * N, nw * N, M);
+        f.ni = N;
+        f.A = a.A;
+        f.sam = M;
+        f.sak = 1;
+        f.sa1 = (long)K * NM;
+        f.B = a.B;
+        f.sbn = M;
+        f.sbno = 2 * NM;
+        f.sbk = 1;
+        f.sb1 = NM;
+        f.C = a.C;
+        f.scm = N;
+        f.scn = 1;
+        f.scno = 2L * cnt * per_item;
+        f.sc1 = (long)cnt * per_item;
+        f.ar = a.ar;
+        RET(zgemm64<typename ztype<YT>::type>(c, "energy_y_gemm", f, 2));
+      } else {
+        RET((zgemm<CP, LT_, GT, YT, true, true>(c, "energy_y_gemm", a, 2 * nw)));
+      }
     }
     RET(launch(c, "energy_trace", [&]() {
       hipLaunchKernelGGL((trace_sq_kernel<typename ztype<YT>::type>), dim3(2 * nw), dim3(256), 0, c->stream,
@@ -1584,27 +1823,22 @@ template <class OT> int build_vx(afqmc_ctx* c, const zd* Lt64)
 {
   const long M = c->M, N = c->N, K = c->K, NM = N * M;
   for (int sp = 0; sp < 2; sp++) {
-    ZGemmArgs a = gargs();
-    a.A = Lt64 + sp * K * NM;  // A_ab(l, n) = Lt(n, a, l)
+    F64Args a = f64args((int)M, (int)M, (int)K);
+    a.A = Lt64 + sp * K * NM;  // A_ab(k, n) = Lt(n, b, k)
     a.sam = 1;
     a.sak = NM;
-    a.sa1 = M;
-    a.sa2 = 0;
-    a.B = Lt64 + sp * K * NM;  // B_ab(k, n) = Lt(n, b, k)
+    a.sa2 = M;
+    a.B = Lt64 + sp * K * NM;  // B_ab(l, n) = Lt(n, a, l)
     a.sbn = 1;
     a.sbk = NM;
-    a.sb1 = 0;
-    a.sb2 = M;
+    a.sb1 = M;
     a.bdiv = (int)N;
-    a.C = (typename ztype<OT>::type*)c->Vx + sp * NM * NM;  // C_ab(l, k) -> Vx[(a,k)][(b,l)]
-    a.scm = 1;
-    a.scn = NM;
+    a.C = (typename ztype<OT>::type*)c->Vx + sp * NM * NM;  // C_ab(k, l) -> Vx[(a,k)][(b,l)]
+    a.scm = NM;
+    a.scn = 1;
     a.sc1 = M * NM;
     a.sc2 = M;
-    a.m = (int)M;
-    a.n = (int)M;
-    a.k = (int)K;
-    RET((zgemm<CP_F64, double, double, OT, false, false>(c, "build_vx", a, (int)(N * N))));
+    RET(zgemm64<typename ztype<OT>::type>(c, "build_vx", a, (int)(N * N)));
   }
   // Vx_s is symmetric (swap (a,k) <-> (b,l)): keep the doubled lower triangle
   using ZT = typename ztype<OT>::type;
@@ -1692,12 +1926,16 @@ int do_energy(afqmc_ctx* c, double* eav_out)
                            c->e_direct, c->e_exch, c->e_one, nw);
       }));
     } else {
-      dim3 grid((nw + 31) / 32, (unsigned)((NAK + 31) / 32));
-      RET(launch(c, "g_transpose", [&]() {
-        hipLaunchKernelGGL((ztranspose_kernel<zd, zd>), grid, dim3(256), 0, c->stream, (const zd*)c->G, c->Gtmp,
-                           (int)NAK, nw, (long)nw, NAK);
-      }));
-      RET((energy_cholesky<CP_F64, double, CP_F64, double, double, double, double>(c, c->Gtmp, c->Lt, c->Lt)));
+      const void* G = c->G;
+      if (!g_wfirst(c)) {
+        dim3 grid((nw + 31) / 32, (unsigned)((NAK + 31) / 32));
+        RET(launch(c, "g_transpose", [&]() {
+          hipLaunchKernelGGL((ztranspose_kernel<zd, zd>), grid, dim3(256), 0, c->stream, (const zd*)c->G, c->Gtmp,
+                             (int)NAK, nw, (long)nw, NAK);
+        }));
+        G = c->Gtmp;
+      }
+      RET((energy_cholesky<CP_F64, double, CP_F64, double, double, double, double>(c, G, c->Lt, c->Lt)));
     }
   } else if (c->mode == AFQMC_FP64_DENSE) {
     RET((energy_cholesky<CP_F64, double, CP_F64, double, double, double, double>(c, c->G, c->Lt, c->Lt)));
@@ -2242,22 +2480,25 @@ int afqmc_upload_system(afqmc_ctx* c, const double* trial_alpha, const double* t
   zd* Lt64 = nullptr;
   RET(dalloc(c, &Lt64, 2 * K * NM));
   for (int sp = 0; sp < 2; sp++) {
-    ZGemmArgs a = gargs();
-    a.A = c->trial + sp * MN;  // A(a, i) = trial[i][a]
-    a.sam = 1;
-    a.sak = N;
-    a.B = Ld64;  // B(k, i) = Ld[n][i][k], batch n
-    a.sbn = 1;
-    a.sbk = M;
-    a.sb1 = MM;
-    a.C = Lt64 + sp * K * NM;
-    a.scm = M;
-    a.scn = 1;
-    a.sc1 = NM;
-    a.m = (int)N;
-    a.n = (int)M;
-    a.k = (int)M;
-    RET((zgemm<CP_F64, double, double, double, false, false>(c, "halfrotate_gemm", a, (int)K)));
+    // columns (n, k); at most 2^30 of them in a product
+    const long nmax = std::max<long>(1, (1L << 30) / M);
+    for (long n0 = 0; n0 < K; n0 += nmax) {
+      const long cnt = std::min(nmax, K - n0);
+      F64Args a = f64args((int)N, (int)(cnt * M), (int)M);
+      a.ni = (int)M;
+      a.A = c->trial + sp * MN;  // A(a, i) = trial[i][a]
+      a.sam = 1;
+      a.sak = N;
+      a.B = Ld64 + n0 * MM;  // B((n, k), i) = Ld[n][i][k]
+      a.sbn = 1;
+      a.sbno = MM;
+      a.sbk = M;
+      a.C = Lt64 + sp * K * NM + n0 * NM;
+      a.scm = M;
+      a.scn = 1;
+      a.scno = NM;
+      RET(zgemm64<zd>(c, "halfrotate_gemm", a, 1));
+    }
   }
   if (c->mode == AFQMC_FP64_CSR) {
     c->sp_rp = rp;
@@ -2522,7 +2763,7 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
       }));
     return AFQMC_OK;
   case AFQMC_BUF_HYBRIDW: return raw(c->hybridW, sizeof(zd) * nw);
-  case AFQMC_BUF_G: return d ? wlast(c->G, NAK, c->mixed, c->tp_G) : raw(c->G, sizeof(zd) * NAK * nw);
+  case AFQMC_BUF_G: return g_wfirst(c) ? wlast(c->G, NAK, c->mixed, c->tp_G) : raw(c->G, sizeof(zd) * NAK * nw);
   case AFQMC_BUF_VBIAS: return d ? wlast(c->vbias, K, false) : raw(c->vbias, sizeof(zd) * K * nw);
   case AFQMC_BUF_X: return d ? wlast(c->X, K, c->mixed, c->tp_X) : raw(c->X, sizeof(zd) * K * nw);
   case AFQMC_BUF_VHS:
@@ -2940,28 +3181,7 @@ extern "C" int afqmc_mixed_density_matrix_noalloc(int nmo, int naea, int nwalk, 
   c->N = naea;
   c->nw = nwalk;
   // T1[w][s] = W[w][s]^T trialwfn_s; every entry is written (beta = 0)
-  ZGemmArgs a = gargs();
-  a.A = W;
-  a.sam = 1;
-  a.sak = N;
-  a.sa1 = 2 * M * N;
-  a.sa2 = M * N;
-  a.B = trialwfn;
-  a.sbn = 1;
-  a.sbk = N;
-  a.sb1 = 0;
-  a.sb2 = M * N;
-  a.C = T1;
-  a.scm = N;
-  a.scn = 1;
-  a.sc1 = 2 * N * N;
-  a.sc2 = N * N;
-  a.bdiv = 2;
-  a.m = naea;
-  a.n = naea;
-  a.k = nmo;
-  int r = zgemm_run<CP_F64, double, double, double, false, false>(c, "ovlp_gemm", a, 2 * nwalk,
-                                                                   default_cfg<CP_F64>(a));
+  int r = overlap_product(c, (const zd*)W, (const zd*)trialwfn, T1);
   // in-place inverse and determinant (no status flag: nothing is read back)
   if (r == AFQMC_OK) r = gj_inverse_into(c, T1, T1, (zd*)ovlp, 2, 1, nullptr, nullptr, nullptr, nullptr);
   if (r == AFQMC_OK) {
@@ -2986,7 +3206,7 @@ extern "C" int afqmc_mixed_density_matrix_noalloc(int nmo, int naea, int nwalk, 
     g.scn = nw;
     g.sc1 = 1;
     g.sc2 = N * M * nw;
-    r = zgemm_run<CP_F64, double, double, double, true, true>(c, "gc_gemm", g, 2 * nwalk, default_cfg<CP_F64>(g));
+    r = zgemm64<zd>(c, "gc_gemm", g, 2 * nwalk);
   }
   c->stream = nullptr;
   return r;

@@ -9,17 +9,16 @@
 // interleaved storage.  No operand is ever stored expanded.
 //
 // Compute precisions:
-//   CP_F64    v_mfma_f64_16x16x4_f64, FP64 accumulation
+//   CP_F64    zgemm_f64_kernel (gemm_f64.hpp), not this one
 //   CP_F32    v_mfma_f32_16x16x4_f32, FP32 accumulation
 //   CP_BF16X3 v_mfma_f32_16x16x32_bf16 on a hi/lo split of both operands
 //             (x = hi + lo, hi = bf16(x), lo = bf16(x - hi)); the three
 //             products hi*hi + hi*lo + lo*hi accumulate in FP32.
 //
-// Output layouts (lane l, accumulator register j, column l%16): the FP32 and
-// BF16 16x16 forms hold rows 4*(l/16)+j; the FP64 form holds rows
-// 4*j+(l/16).  Within one MFMA, A and B use the same
+// Output layout (lane l, accumulator register j, column l%16): rows
+// 4*(l/16)+j.  Within one MFMA, A and B use the same
 // lane->k assignment, so the k order inside a fragment is free; it is chosen
-// so that each lane reads whole complex numbers (FP64/FP32) or four
+// so that each lane reads whole complex numbers (FP32) or four
 // consecutive complex numbers (BF16) from LDS.
 #pragma once
 #include "common.hpp"
@@ -66,16 +65,6 @@ struct ZGemmArgs {
   void* C3;
 };
 
-template <int CP> struct LdsT;
-template <> struct LdsT<CP_F64> {
-  using T = zd;
-  static constexpr int PAD = 1;
-};
-template <> struct LdsT<CP_F32> {
-  using T = zf;
-  static constexpr int PAD = 2;
-};
-
 template <class Z> __device__ inline void zero_z(Z& z)
 {
   z.re = 0;
@@ -103,6 +92,7 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
   constexpr int EB = (BNC * BKC + NT - 1) / NT;
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be a multiple of 16");
   static_assert(CP != CP_BF16X3 || BKC % 16 == 0, "bf16 k-tile must be a multiple of 16 complex");
+  static_assert(CP == CP_F32 || CP == CP_BF16X3, "FP32 and split-BF16 products");
   static_assert(CP == CP_BF16X3 || BKC % 4 == 0, "k-tile must be a multiple of 4 complex");
   static_assert(CP == CP_BF16X3 || (!std::is_same<AT, bfs>::value && !std::is_same<BT, bfs>::value),
                 "split-BF16 operands need the BF16 path");
@@ -113,7 +103,7 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
   static_assert(!BDMA || (BNC / WN) % 16 == 0, "each wave's B rows must start at a multiple of 16");
   using AZ = typename ztype<AT>::type;
   using BZ = typename ztype<BT>::type;
-  using ACC = typename std::conditional<CP == CP_F64, doublex4, floatx4>::type;
+  using ACC = floatx4;
 
   const int tid = threadIdx.x;
   const int lane = tid & 63, wave = tid >> 6;
@@ -164,12 +154,10 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
       for (int q = 0; q < 4; q++) acc[i][j][q] = 0;
 
   if constexpr (CP != CP_BF16X3) {
-  using L = LdsT<CP>;
-  using LT = typename L::T;
-  constexpr int LDK = BKC + L::PAD;
+  constexpr int LDK = BKC + 2;
   // two LDS stages (ping-pong): the next k-tile is stored while others compute
-  __shared__ __align__(16) LT sA[2][BM * LDK];
-  __shared__ __align__(16) LT sB[2][BNC * LDK];
+  __shared__ __align__(16) zf sA[2][BM * LDK];
+  __shared__ __align__(16) zf sB[2][BNC * LDK];
   AZ ra[EA];
   BZ rb[EB];
   auto gload = [&](int k0) {
@@ -199,11 +187,7 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
       if (e >= BM * BKC) break;
       int row, kc;
       if (AK) { row = e / BKC; kc = e % BKC; } else { kc = e / BM; row = e % BM; }
-      if constexpr (CP == CP_F64) {
-        sA[st][row * LDK + kc] = zd{(double)ra[i].re, (double)ra[i].im};
-      } else {
-        sA[st][row * LDK + kc] = zf{(float)ra[i].re, (float)ra[i].im};
-      }
+      sA[st][row * LDK + kc] = zf{(float)ra[i].re, (float)ra[i].im};
     }
 #pragma unroll
     for (int i = 0; i < EB; i++) {
@@ -211,13 +195,8 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
       if (e >= BNC * BKC) break;
       int col, kc;
       if (BK) { col = e / BKC; kc = e % BKC; } else { kc = e / BNC; col = e % BNC; }
-      if constexpr (CP == CP_F64) {
-        const double bi = (double)rb[i].im;
-        sB[st][col * LDK + kc] = zd{(double)rb[i].re, p.conjb ? -bi : bi};
-      } else {
-        const float bi = (float)rb[i].im;
-        sB[st][col * LDK + kc] = zf{(float)rb[i].re, p.conjb ? -bi : bi};
-      }
+      const float bi = (float)rb[i].im;
+      sB[st][col * LDK + kc] = zf{(float)rb[i].re, p.conjb ? -bi : bi};
     }
   };
 
@@ -231,27 +210,21 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
     const int cur = kt & 1;
     if (kt + 1 < nk) gload((kt + 1) * BKC);
     {
-      using RT = typename std::conditional<CP == CP_F64, double, float>::type;
 #pragma unroll
       for (int kq = 0; kq < BKC / 4; kq++) {
-        LT a[TM], bv[TN];
+        zf a[TM], bv[TN];
 #pragma unroll
         for (int i = 0; i < TM; i++) a[i] = sA[cur][(arow0 + i * 16) * LDK + kq * 4 + g];
 #pragma unroll
         for (int j = 0; j < TN; j++) bv[j] = sB[cur][(bcol0 + j * 8) * LDK + kq * 4 + g];
 #pragma unroll
         for (int j = 0; j < TN; j++) {
-          RT b0 = s ? bv[j].im : bv[j].re;
-          RT b1 = s ? bv[j].re : -bv[j].im;
+          float b0 = s ? bv[j].im : bv[j].re;
+          float b1 = s ? bv[j].re : -bv[j].im;
 #pragma unroll
           for (int i = 0; i < TM; i++) {
-            if constexpr (CP == CP_F64) {
-              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].re, b0, acc[i][j], 0, 0, 0);
-              acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i].im, b1, acc[i][j], 0, 0, 0);
-            } else {
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].re, b0, acc[i][j], 0, 0, 0);
-              acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].im, b1, acc[i][j], 0, 0, 0);
-            }
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].re, b0, acc[i][j], 0, 0, 0);
+            acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(a[i].im, b1, acc[i][j], 0, 0, 0);
           }
         }
       }
@@ -504,10 +477,7 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
   // first: D may alias F, so loads issued between the stores could not
   // overlap them.
   const bool has_beta = (p.br != 0.0 || p.bi != 0.0);
-  // FP64 16x16x4 interleaves rows (row = 4*reg + lane/16); the FP32 and BF16
-  // 16x16 forms keep 4 consecutive rows per lane group.
-  const int rbase = m0 + wm * WTM + ((CP == CP_F64) ? g : 4 * g);
-  constexpr int RQ = (CP == CP_F64) ? 4 : 1;  // row step of the accumulator register
+  const int rbase = m0 + wm * WTM + 4 * g;
   const int cbase = n0 + (wn * WTN + r) / 2;
   // one accumulator row block at a time: its F (and C for beta) values are
   // loaded first, then the block is written
@@ -519,7 +489,7 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
     for (int j = 0; j < TN; j++)
 #pragma unroll
       for (int q = 0; q < 4; q++) {
-        const int row = rbase + i * 16 + RQ * q, col = cbase + j * 8;
+        const int row = rbase + i * 16 + q, col = cbase + j * 8;
         const bool in = row < p.m && col < p.n;
         const long off = 2 * ((long)row * p.scm + (long)col * p.scn);
         const long foff = (p.sfm || p.sfn) ? 2 * ((long)row * p.sfm + (long)col * p.sfn) : off;
@@ -530,7 +500,7 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_kernel(ZGemmArgs p)
     for (int j = 0; j < TN; j++)
 #pragma unroll
       for (int q = 0; q < 4; q++) {
-        const int row = rbase + i * 16 + RQ * q, col = cbase + j * 8;
+        const int row = rbase + i * 16 + q, col = cbase + j * 8;
         const double v = (double)acc[i][j][q];
         const double pv = __shfl_xor(v, 1);
         const double re = s ? pv : v, im = s ? v : pv;
