@@ -677,48 +677,41 @@ ZGemmArgs gargs()
 }
 
 // C = alpha * A * B + beta * C for CSR A [nrows][K] and B [K][nw] (walker
-// index last).  Rows averaging 512 entries or more: with columns known to be
-// sorted within rows, 4 to 16 rows share each LDS-staged window of B;
-// otherwise a workgroup of 4 or 16 waves shares each row.  Shorter rows take
-// one wave per (row, 64 walkers), which measured faster than staging.
+// index last).  Sorted rows against a B larger than the L2 (32 MB), with
+// enough rows for a workgroup of 16 on every CU and 8 entries a window, take
+// the windowed kernel (1.33x at 65536 columns x 256 walkers; the row kernel
+// is 1.3-2x faster on smaller B).  The others take one wave per row and
+// chunk of walkers when that alone gives four waves per SIMD or the rows are
+// short, else 16 (1024 entries per row) or 4 waves per row.
 int csrmm_n(afqmc_ctx* c, const char* name, int nrows, int K, long long nnz, const int* rp, const int* col,
             const zd* val, const zd* B, long ldb, zd* C, long ldc, zd alpha, zd beta, bool sorted = false)
 {
   const int nw = c->nw;
-  const long nchunk = (nw + 63) / 64;
   const double avg = nrows > 0 ? (double)nnz / nrows : 0.0;
-  if (sorted && avg >= 512) {
-    // rows per workgroup: the most B reuse that still gives 256 workgroups
-    if (((nrows + 15) / 16) * nchunk >= 256)
-      return launch(c, name, [&]() {
-        hipLaunchKernelGGL((csrmm_n_lds_kernel<16, 64>), dim3((unsigned)(((nrows + 15) / 16) * nchunk)), dim3(1024),
-                           0, c->stream, nrows, nw, K, rp, col, val, B, ldb, C, ldc, alpha, beta);
-      });
-    if (((nrows + 7) / 8) * nchunk >= 256)
-      return launch(c, name, [&]() {
-        hipLaunchKernelGGL((csrmm_n_lds_kernel<8, 64>), dim3((unsigned)(((nrows + 7) / 8) * nchunk)), dim3(512), 0,
-                           c->stream, nrows, nw, K, rp, col, val, B, ldb, C, ldc, alpha, beta);
-      });
+  const long n64 = (nw + 63) / 64;
+  if (sorted && nw > 32 && (long)K * ldb * (long)sizeof(zd) > (32L << 20) && ((nrows + 15) / 16) * n64 >= 256 &&
+      avg * 64 >= 8.0 * K)
     return launch(c, name, [&]() {
-      hipLaunchKernelGGL((csrmm_n_lds_kernel<4, 64>), dim3((unsigned)(((nrows + 3) / 4) * nchunk)), dim3(256), 0,
-                         c->stream, nrows, nw, K, rp, col, val, B, ldb, C, ldc, alpha, beta);
+      hipLaunchKernelGGL(csrmm_win_kernel, dim3((unsigned)(((nrows + 15) / 16) * n64)), dim3(1024), 0, c->stream,
+                         nrows, nw, K, rp, col, val, B, ldb, C, ldc, alpha, beta);
     });
-  }
-  if (avg >= 4096)
+  auto rows = [&](auto Sc, auto WLc) {
+    constexpr int S = decltype(Sc)::value, WL = decltype(WLc)::value;
+    const long items = (long)nrows * ((nw + WL - 1) / WL);
     return launch(c, name, [&]() {
-      hipLaunchKernelGGL(csrmm_n_split_kernel<16>, dim3((unsigned)(nrows * nchunk)), dim3(1024), 0, c->stream, nrows,
-                         nw, K, rp, col, val, B, ldb, C, ldc, alpha, beta);
+      hipLaunchKernelGGL((csrmm_row_kernel<S, WL>), dim3((unsigned)(S == 1 ? (items + 3) / 4 : items)),
+                         dim3(S == 1 ? 256 : 64 * S), 0, c->stream, nrows, nw, K, rp, col, val, B, ldb, C, ldc, alpha,
+                         beta);
     });
-  if (avg >= 512)
-    return launch(c, name, [&]() {
-      hipLaunchKernelGGL(csrmm_n_split_kernel<4>, dim3((unsigned)(nrows * nchunk)), dim3(256), 0, c->stream, nrows,
-                         nw, K, rp, col, val, B, ldb, C, ldc, alpha, beta);
-    });
-  const long waves = (long)nrows * nchunk;
-  return launch(c, name, [&]() {
-    hipLaunchKernelGGL(csrmm_n_kernel, dim3((unsigned)((waves + 3) / 4)), dim3(256), 0, c->stream, nrows, nw, K, rp,
-                       col, val, B, ldb, C, ldc, alpha, beta);
-  });
+  };
+  auto width = [&](auto Sc) {
+    if (nw <= 16) return rows(Sc, std::integral_constant<int, 16>());
+    if (nw <= 32) return rows(Sc, std::integral_constant<int, 32>());
+    return rows(Sc, std::integral_constant<int, 64>());
+  };
+  if (avg < 256 || (long)nrows * n64 >= 4096) return width(std::integral_constant<int, 1>());
+  if (avg < 1024) return width(std::integral_constant<int, 4>());
+  return width(std::integral_constant<int, 16>());
 }
 
 // Batched inverse + determinant of the nw*2 overlap matrices T (in place

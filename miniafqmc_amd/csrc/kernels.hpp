@@ -453,176 +453,182 @@ __global__ void wd_logs_kernel(const zd* __restrict__ Wd, zd* __restrict__ Wl, i
 // CSR x dense, mySPBLAS::csrmm 'N' semantics (src/Numerics/sparse.hpp:166-180):
 // C(r, w) = alpha * sum_{p in row r, col<K} val[p] * B(col[p], w) + beta*C(r,w)
 // B(c, w) at B[c*ldb + w]; C(r, w) at C[r*ldc + w] (row-major, walker last).
-// One wave per (row, 64-walker chunk); nonzero indices are wave-uniform.
-__global__ __launch_bounds__(256) void csrmm_n_kernel(int nrows, int nw, int K, const int* __restrict__ rowptr,
-                                                      const int* __restrict__ col, const zd* __restrict__ val,
-                                                      const zd* __restrict__ B, long ldb, zd* __restrict__ C,
-                                                      long ldc, zd alpha, zd beta)
+
+// a += v * b in four fused multiply-adds
+__device__ __forceinline__ void zfma(zd& a, zd v, zd b)
 {
-  const int wave = (blockIdx.x * blockDim.x + threadIdx.x) >> 6;
-  const int lane = threadIdx.x & 63;
-  const int nchunk = (nw + 63) / 64;
-  const int r = wave / nchunk, ch = wave % nchunk;
-  if (r >= nrows) return;
-  const int w = ch * 64 + lane;
-  const int p0 = rowptr[0];
-  const int pb = __builtin_amdgcn_readfirstlane(rowptr[r] - p0);
-  const int pe = __builtin_amdgcn_readfirstlane(rowptr[r + 1] - p0);
-  zd acc{0, 0};
-  if (w < nw) {
-    for (int p = pb; p < pe; p++) {
-      int c = col[p];
-      if (c >= K) continue;
-      zd a = val[p];
-      zd bv = B[(long)c * ldb + w];
-      acc.re += a.re * bv.re - a.im * bv.im;
-      acc.im += a.re * bv.im + a.im * bv.re;
-    }
-    zd o = zmul(alpha, acc);
-    if (beta.re != 0.0 || beta.im != 0.0) o = zadd(o, zmul(beta, C[(long)r * ldc + w]));
-    C[(long)r * ldc + w] = o;
-  }
+  a.re = fma(v.re, b.re, a.re);
+  a.im = fma(v.re, b.im, a.im);
+  a.re = fma(-v.im, b.im, a.re);
+  a.im = fma(v.im, b.re, a.im);
+}
+__device__ inline void csr_store(zd* C, zd acc, zd alpha, zd beta)
+{
+  zd o = zmul(alpha, acc);
+  if (beta.re != 0.0 || beta.im != 0.0) o = zadd(o, zmul(beta, *C));
+  *C = o;
 }
 
-// csrmm 'N' for long rows: one workgroup of S waves per (row, 64-walker
-// chunk).  Wave s sums a contiguous segment of the row's entries into two
-// accumulators (even and odd entries, so consecutive FMAs do not wait on
-// each other); the S partial sums are reduced through LDS in a fixed order.
-// Same semantics as csrmm_n_kernel (entries with col >= K skipped).
-template <int S>
-__global__ __launch_bounds__(64 * S) void csrmm_n_split_kernel(int nrows, int nw, int K, const int* __restrict__ rowptr,
-                                                              const int* __restrict__ col,
-                                                              const zd* __restrict__ val, const zd* __restrict__ B,
-                                                              long ldb, zd* __restrict__ C, long ldc, zd alpha,
-                                                              zd beta)
+// S waves per row and chunk of WL walkers (64 / WL groups of lanes take
+// entries side by side), four entries in flight per group; the partial sums
+// are joined in a fixed order (entries of a group, groups, waves).
+// Bound: latency when rows x chunks are few, then the L2 (each entry reads
+// 16 B of B per walker).  Measured (MI355X, before -> after): 2048 rows of
+// 2048 entries, 16 walkers: 285 -> 72 us (16 waves per row, 16-lane groups;
+// one 64-lane wave per row left 48 lanes idle); 384 rows of 1382, 64
+// walkers: 788 -> 44 us (16 waves; 96 workgroups of 4 rows before); 65536
+// rows of 205, 256 walkers: 2360 -> 1757 us (31 TB/s of L2 reads).
+template <int S, int WL>
+__global__ __launch_bounds__(S == 1 ? 256 : 64 * S) void csrmm_row_kernel(int nrows, int nw, int K,
+                                                                       const int* __restrict__ rowptr,
+                                                                       const int* __restrict__ col,
+                                                                       const zd* __restrict__ val,
+                                                                       const zd* __restrict__ B, long ldb,
+                                                                       zd* __restrict__ C, long ldc, zd alpha, zd beta)
 {
-  __shared__ zd part[S][64];
-  const int nchunk = (nw + 63) / 64;
-  const int r = blockIdx.x / nchunk, ch = blockIdx.x % nchunk;
-  const int sw = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int w = ch * 64 + lane;
+  constexpr int NG = 64 / WL;  // entries taken side by side by the lane groups
+  constexpr int U = 4;
+  constexpr int RW = S == 1 ? 4 : 1;  // rows per workgroup
+  __shared__ zd part[S == 1 ? 1 : S][WL];
+  const int nchunk = (nw + WL - 1) / WL;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const long item = (long)blockIdx.x * RW + (S == 1 ? wave : 0);
+  const int r = (int)(item / nchunk), ch = (int)(item % nchunk);
+  const int sw = S == 1 ? 0 : wave;
+  if (r >= nrows) return;  // S == 1 only (whole waves; no barrier follows)
+  const int grp = lane / WL;
+  const int w = ch * WL + lane % WL;
+  const int wc = min(w, nw - 1);
   const int p0 = rowptr[0];
-  const int pb = rowptr[r] - p0, pe = rowptr[r + 1] - p0;
-  const int len = pe - pb, per = (len + S - 1) / S;
+  const int pb = __builtin_amdgcn_readfirstlane(rowptr[r] - p0), pe = __builtin_amdgcn_readfirstlane(rowptr[r + 1] - p0);
+  const int len = pe - pb, per = ((len + S - 1) / S + NG - 1) / NG * NG;
   const int qb = pb + min(len, sw * per), qe = pb + min(len, (sw + 1) * per);
-  zd a0{0, 0}, a1{0, 0};
-  if (w < nw) {
-    int p = qb;
-    for (; p + 1 < qe; p += 2) {
-      const int c0 = col[p], c1 = col[p + 1];
-      const zd v0 = val[p], v1 = val[p + 1];
-      if (c0 < K) {
-        const zd b0 = B[(long)c0 * ldb + w];
-        a0.re += v0.re * b0.re - v0.im * b0.im;
-        a0.im += v0.re * b0.im + v0.im * b0.re;
-      }
-      if (c1 < K) {
-        const zd b1 = B[(long)c1 * ldb + w];
-        a1.re += v1.re * b1.re - v1.im * b1.im;
-        a1.im += v1.re * b1.im + v1.im * b1.re;
-      }
-    }
-    if (p < qe) {
-      const int c0 = col[p];
-      const zd v0 = val[p];
-      if (c0 < K) {
-        const zd b0 = B[(long)c0 * ldb + w];
-        a0.re += v0.re * b0.re - v0.im * b0.im;
-        a0.im += v0.re * b0.im + v0.im * b0.re;
-      }
-    }
-  }
-  part[sw][lane] = zadd(a0, a1);
-  __syncthreads();
-  if (sw == 0 && w < nw) {
-    zd acc = part[0][lane];
+  zd acc[U];
 #pragma unroll
-    for (int q = 1; q < S; q++) acc = zadd(acc, part[q][lane]);
-    zd o = zmul(alpha, acc);
-    if (beta.re != 0.0 || beta.im != 0.0) o = zadd(o, zmul(beta, C[(long)r * ldc + w]));
-    C[(long)r * ldc + w] = o;
+  for (int u = 0; u < U; u++) acc[u] = zd{0, 0};
+  int p = qb;
+  for (; p + U * NG <= qe; p += U * NG) {
+    int c[U];
+    zd v[U], b[U];
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      const int q = NG == 1 ? p + u : p + u * NG + grp;
+      c[u] = col[q];
+      v[u] = val[q];
+    }
+#pragma unroll
+    for (int u = 0; u < U; u++) b[u] = c[u] < K ? B[(long)c[u] * ldb + wc] : zd{0, 0};
+#pragma unroll
+    for (int u = 0; u < U; u++) {
+      if (c[u] >= K) v[u] = zd{0, 0};
+      zfma(acc[u], v[u], b[u]);
+    }
+  }
+  for (; p < qe; p += NG) {
+    const int q = NG == 1 ? p : p + grp;
+    if (q < qe) {
+      const int c = col[q];
+      if (c < K) {
+        const zd v = val[q], b = B[(long)c * ldb + wc];
+        acc[0].re += v.re * b.re - v.im * b.im;
+        acc[0].im += v.re * b.im + v.im * b.re;
+      }
+    }
+  }
+  zd a = zadd(zadd(acc[0], acc[1]), zadd(acc[2], acc[3]));
+#pragma unroll
+  for (int o = WL; o < 64; o <<= 1) {
+    a.re += __shfl_xor(a.re, o);
+    a.im += __shfl_xor(a.im, o);
+  }
+  if constexpr (S == 1) {
+    if (lane < WL && w < nw) csr_store(&C[(long)r * ldc + w], a, alpha, beta);
+  } else {
+    if (lane < WL) part[sw][lane] = a;
+    __syncthreads();
+    if (sw == 0 && lane < WL && w < nw) {
+      zd t = part[0][lane];
+#pragma unroll
+      for (int q = 1; q < S; q++) t = zadd(t, part[q][lane]);
+      csr_store(&C[(long)r * ldc + w], t, alpha, beta);
+    }
   }
 }
 
-// value of lane j (j the same in every lane) without going through LDS
-__device__ inline int rdlane(int x, int j) { return __builtin_amdgcn_readlane(x, j); }
-__device__ inline double rdlane(double x, int j)
+// Rows whose columns are sorted, against a B that exceeds the L2: a workgroup
+// of 16 waves takes 16 rows and 64 walkers and walks the columns in windows
+// of 64, each window of B staged once for the 16 rows by direct loads into
+// one of two LDS buffers while the other is read.  An entry's value and
+// column come through scalar registers (one row per wave).  Measured: 1024
+// rows of 13110 entries over 65536 columns, 256 walkers 3.90 ms (row kernel
+// 5.19 ms, single-buffered windows with entries read from lanes 4.83 ms).
+// More rows per wave are slower (the per-row overhead of a window).
+__global__ __launch_bounds__(1024) void csrmm_win_kernel(int nrows, int nw, int K, const int* __restrict__ rowptr,
+                                                         const int* __restrict__ col, const zd* __restrict__ val,
+                                                         const zd* __restrict__ B, long ldb, zd* __restrict__ C,
+                                                         long ldc, zd alpha, zd beta)
 {
-  const long long v = __double_as_longlong(x);
-  const int lo = __builtin_amdgcn_readlane((int)(v & 0xffffffffLL), j);
-  const int hi = __builtin_amdgcn_readlane((int)(v >> 32), j);
-  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
-}
-
-// csrmm 'N' for long rows whose columns are sorted within each row: a
-// workgroup of R waves takes R consecutive rows and one chunk of 64 walkers,
-// and walks the columns in windows of CB.  Each window of B (CB rows x 64
-// walkers) is staged in LDS once and read by all R rows, so B is fetched
-// once per R rows instead of once per row.  Entries with col >= K are never
-// reached (the reference's csrmm skips them too).
-template <int R, int CB>
-__global__ __launch_bounds__(64 * R) void csrmm_n_lds_kernel(int nrows, int nw, int K, const int* __restrict__ rowptr,
-                                                            const int* __restrict__ col, const zd* __restrict__ val,
-                                                            const zd* __restrict__ B, long ldb, zd* __restrict__ C,
-                                                            long ldc, zd alpha, zd beta)
-{
-  __shared__ zd Bs[CB][64];
+  __shared__ __align__(16) zd b0[64 * 64];
+  __shared__ __align__(16) zd b1[64 * 64];
   const int nchunk = (nw + 63) / 64;
   const int rb = blockIdx.x / nchunk, ch = blockIdx.x % nchunk;
-  const int sw = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int r = rb * R + sw;
-  const int w = ch * 64 + lane;
+  const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6), lane = threadIdx.x & 63;
+  const int w = ch * 64 + lane, wc = min(w, nw - 1);
   const int p0 = rowptr[0];
-  int p = 0, pe = 0;
-  if (r < nrows) {
-    p = rowptr[r] - p0;
-    pe = rowptr[r + 1] - p0;
-  }
-  p = __builtin_amdgcn_readfirstlane(p);  // one row per wave
-  pe = __builtin_amdgcn_readfirstlane(pe);
-  zd a0{0, 0}, a1{0, 0};
-  for (int c0 = 0; c0 < K; c0 += CB) {
-    for (int e = threadIdx.x; e < CB * 64; e += 64 * R) {
-      const int cc = e >> 6, l = e & 63, ww = ch * 64 + l;
-      Bs[cc][l] = (c0 + cc < K && ww < nw) ? B[(long)(c0 + cc) * ldb + ww] : zd{0, 0};
+  const int r = rb * 16 + wave;
+  int p = __builtin_amdgcn_readfirstlane(r < nrows ? rowptr[r] - p0 : 0);
+  const int pe = __builtin_amdgcn_readfirstlane(r < nrows ? rowptr[r + 1] - p0 : 0);
+  // lane i holds the column of the row's i-th entry that is still to come
+  int cl = p + lane < pe ? col[p + lane] : 0x7fffffff;
+  zd acc{0, 0};
+  auto issue = [&](zd* dst, int c0) __attribute__((always_inline)) {
+#pragma unroll
+    for (int i = 0; i < 4; i++) {
+      const int cc = i * 16 + wave;
+      __builtin_amdgcn_global_load_lds((const void*)(B + (long)min(c0 + cc, K - 1) * ldb + wc),
+                                       (__attribute__((address_space(3))) void*)&dst[cc * 64], 16, 0, 0);
     }
-    __syncthreads();
-    const int cend = c0 + CB;
-    // the row's entries in this window, 64 at a time: lane i loads entry
-    // p + i, the window's entries form a prefix (columns sorted), and each
-    // is read from its lane into scalar registers
+  };
+  auto window = [&](const zd* bs, int c0) __attribute__((always_inline)) {
+    const int cend = min(c0 + 64, K);
     for (;;) {
-      const int q = p + lane;
-      const bool inw = q < pe && col[q] < cend;
-      const int cq = inw ? col[q] - c0 : 0;
-      const zd vq = inw ? val[q] : zd{0, 0};
-      const int n = __popcll(__ballot(inw));
-      for (int j = 0; j + 1 < n; j += 2) {
-        const int c_0 = rdlane(cq, j), c_1 = rdlane(cq, j + 1);
-        const zd v0{rdlane(vq.re, j), rdlane(vq.im, j)}, v1{rdlane(vq.re, j + 1), rdlane(vq.im, j + 1)};
-        const zd b0 = Bs[c_0][lane], b1 = Bs[c_1][lane];
-        a0.re += v0.re * b0.re - v0.im * b0.im;
-        a0.im += v0.re * b0.im + v0.im * b0.re;
-        a1.re += v1.re * b1.re - v1.im * b1.im;
-        a1.im += v1.re * b1.im + v1.im * b1.re;
+      // the window's entries are a prefix of those to come; the next lane
+      // load is issued before they are summed
+      const int m = __popcll(__ballot(cl < cend));
+      const int q = p + m + lane;
+      cl = q < pe ? col[q] : 0x7fffffff;
+      int j = 0;
+      for (; j + 4 <= m; j += 4) {
+        int c[4];
+        zd v[4];
+#pragma unroll
+        for (int u = 0; u < 4; u++) {
+          c[u] = col[p + j + u] - c0;
+          v[u] = val[p + j + u];
+        }
+#pragma unroll
+        for (int u = 0; u < 4; u++) zfma(acc, v[u], bs[c[u] * 64 + lane]);
       }
-      if (n & 1) {
-        const int c_0 = rdlane(cq, n - 1);
-        const zd v0{rdlane(vq.re, n - 1), rdlane(vq.im, n - 1)};
-        const zd b0 = Bs[c_0][lane];
-        a0.re += v0.re * b0.re - v0.im * b0.im;
-        a0.im += v0.re * b0.im + v0.im * b0.re;
-      }
-      p += n;
-      if (n < 64) break;
+      for (; j < m; j++) zfma(acc, val[p + j], bs[(col[p + j] - c0) * 64 + lane]);
+      p += m;
+      if (m < 64) break;  // 64: more may follow (repeated columns)
     }
-    __syncthreads();
+  };
+  const int nwin = (K + 63) / 64;
+  issue(b0, 0);
+  for (int t = 0; t < nwin; t += 2) {
+    __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+    __builtin_amdgcn_s_barrier();
+    if (t + 1 < nwin) issue(b1, (t + 1) * 64);
+    window(b0, t * 64);
+    if (t + 1 < nwin) {
+      __builtin_amdgcn_s_waitcnt(0 | (7 << 4) | (15 << 8));
+      __builtin_amdgcn_s_barrier();
+      if (t + 2 < nwin) issue(b0, (t + 2) * 64);
+      window(b1, (t + 1) * 64);
+    }
   }
-  if (r < nrows && w < nw) {
-    zd o = zmul(alpha, zadd(a0, a1));
-    if (beta.re != 0.0 || beta.im != 0.0) o = zadd(o, zmul(beta, C[(long)r * ldc + w]));
-    C[(long)r * ldc + w] = o;
-  }
+  if (r < nrows && w < nw) csr_store(&C[(long)r * ldc + w], acc, alpha, beta);
 }
 
 // ---------------------------------------------------------------------------
