@@ -12,9 +12,7 @@
 //     Lt [2][K][N*M] (spin-major).
 #include "afqmc_hip.h"
 #include "common.hpp"
-#include "gemm.hpp"
-#include "gemm_b16.hpp"
-#include "gemm_f64.hpp"
+#include "gemm_launch.hpp"
 #include "kernels.hpp"
 #include "propagate.hpp"
 
@@ -342,16 +340,6 @@ inline int nblk(long n, int t) { return (int)std::min<long>((n + t - 1) / t, 655
 // GEMM dispatch.  Each call site (name and shape) runs one of a few tile
 // shapes; afqmc_tune() times all candidates once per call site and keeps the
 // fastest, otherwise a size heuristic picks.
-struct TileCfg {
-  int BM, BNC, WM, WN;
-};
-// candidates per precision (BKC is 8 complex for FP32, 16 for BF16)
-constexpr TileCfg kCfgF32[] = {{32, 16, 1, 1}, {128, 64, 2, 2}, {128, 128, 2, 2}};
-constexpr TileCfg kCfgB16[] = {{32, 16, 1, 1}, {128, 64, 2, 2}, {128, 128, 2, 2}, {256, 64, 4, 2}, {64, 64, 2, 2}};
-
-template <int CP> constexpr int ncfg() { return CP == CP_F32 ? 3 : 5; }
-template <int CP> constexpr TileCfg cfg_at(int i) { return CP == CP_F32 ? kCfgF32[i] : kCfgB16[i]; }
-
 // Time each of n candidates (results are discarded), in two rounds keeping
 // each one's faster round; `best` starts as the default.
 template <class F> int tune_tiles(afqmc_ctx* c, int n, int& best, F&& run)
@@ -379,56 +367,32 @@ template <class F> int tune_tiles(afqmc_ctx* c, int n, int& best, F&& run)
   return AFQMC_OK;
 }
 
-template <int CP, class AT, class BT, class OT, bool AK, bool BK, int CI>
-int zgemm_cfg(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch)
+template <int CP, class AT, class BT, class OT, bool AK, bool BK>
+int zgemm_run(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch, int ci)
 {
-  constexpr TileCfg t = cfg_at<CP>(CI);
-  constexpr int BKC = (CP == CP_BF16X3) ? 16 : (t.WM * t.WN == 1 ? 16 : 8);
+  const TileCfg t = CP == CP_F32 ? kCfgF32[ci] : kCfgB16[ci];
   a.MT = (a.m + t.BM - 1) / t.BM;
   a.NT = (a.n + t.BNC - 1) / t.BNC;
   const long tiles = (long)a.MT * a.NT * batch;
   if (tiles > 2147483647L) return fail(c, AFQMC_ERR_SHAPE, "GEMM grid too large");
+  int dma = 0;
   if constexpr (CP == CP_BF16X3 && std::is_same<AT, bfs>::value && AK) {
     // direct global -> LDS staging of A: 16-byte loads of two complex at a
     // time, so every row (and batch item) must start 16-byte aligned, and
     // whole k-tiles (the triangular mode stops at column-block ends, which
     // are multiples of 16 too)
-    if (c->gemm_adma && a.sak == 1 && a.k % BKC == 0 && a.sam % 2 == 0 && a.sa1 % 2 == 0 && a.sa2 % 2 == 0 &&
-        ((uintptr_t)a.A & 15) == 0 && (!a.ktri || t.BNC % BKC == 0)) {
+    if (c->gemm_adma && a.sak == 1 && a.k % 16 == 0 && a.sam % 2 == 0 && a.sa1 % 2 == 0 && a.sa2 % 2 == 0 &&
+        ((uintptr_t)a.A & 15) == 0 && (!a.ktri || t.BNC % 16 == 0)) {
+      dma = 1;
+      // B too, on the same conditions (conj(B) only through registers)
       if constexpr (std::is_same<BT, bfs>::value && BK) {
-        // B too, on the same conditions (conj(B) only through registers)
         if (a.sbk == 1 && a.sbn % 2 == 0 && a.sb1 % 2 == 0 && a.sb2 % 2 == 0 && ((uintptr_t)a.B & 15) == 0 &&
             !a.conjb)
-          return launch(c, name, [&]() {
-            hipLaunchKernelGGL((zgemm_kernel<CP, AT, BT, OT, AK, BK, t.BM, t.BNC, BKC, t.WM, t.WN, true, true>),
-                               dim3((unsigned)tiles), dim3(64 * t.WM * t.WN), 0, c->stream, a);
-          });
+          dma = 2;
       }
-      return launch(c, name, [&]() {
-        hipLaunchKernelGGL((zgemm_kernel<CP, AT, BT, OT, AK, BK, t.BM, t.BNC, BKC, t.WM, t.WN, true>),
-                           dim3((unsigned)tiles), dim3(64 * t.WM * t.WN), 0, c->stream, a);
-      });
     }
   }
-  return launch(c, name, [&]() {
-    hipLaunchKernelGGL((zgemm_kernel<CP, AT, BT, OT, AK, BK, t.BM, t.BNC, BKC, t.WM, t.WN>), dim3((unsigned)tiles),
-                       dim3(64 * t.WM * t.WN), 0, c->stream, a);
-  });
-}
-
-template <int CP, class AT, class BT, class OT, bool AK, bool BK>
-int zgemm_run(afqmc_ctx* c, const char* name, const ZGemmArgs& a, int batch, int ci)
-{
-  switch (ci) {
-  case 0: return zgemm_cfg<CP, AT, BT, OT, AK, BK, 0>(c, name, a, batch);
-  case 1: return zgemm_cfg<CP, AT, BT, OT, AK, BK, 1>(c, name, a, batch);
-  case 2: return zgemm_cfg<CP, AT, BT, OT, AK, BK, 2>(c, name, a, batch);
-  case 3: if constexpr (ncfg<CP>() > 3) return zgemm_cfg<CP, AT, BT, OT, AK, BK, (ncfg<CP>() > 3 ? 3 : 0)>(c, name, a, batch);
-          break;
-  case 4: if constexpr (ncfg<CP>() > 4) return zgemm_cfg<CP, AT, BT, OT, AK, BK, (ncfg<CP>() > 4 ? 4 : 0)>(c, name, a, batch);
-          break;
-  }
-  return zgemm_cfg<CP, AT, BT, OT, AK, BK, 0>(c, name, a, batch);
+  return launch(c, name, [&]() { zgemm_launch<CP, AT, BT, OT, AK, BK>(c->stream, a, (unsigned)tiles, ci, dma); });
 }
 
 template <int CP> int default_cfg(const ZGemmArgs& a)
@@ -437,18 +401,6 @@ template <int CP> int default_cfg(const ZGemmArgs& a)
   return 0;                              // one-wave 32 x 16 tiles
 }
 
-// Split-BF16 products whose operands are both split-BF16 with k contiguous
-// run zgemm_b16dma_kernel (both operands staged by direct loads through a
-// ring of LDS stages); candidates (rows, complex columns, waves, stages):
-struct RingCfg {
-  int BM, BN, WM, WN, S;
-};
-constexpr RingCfg kRing[] = {{128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {256, 128, 4, 2, 3}};
-// three-piece operands take half as much LDS again per stage
-constexpr RingCfg kRing3[] = {{128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {128, 128, 2, 2, 3}};
-constexpr int kNRing = 4;
-template <int NP> constexpr RingCfg ring_at(int i) { return NP == 3 ? kRing3[i] : kRing[i]; }
-
 bool ring_ok(const afqmc_ctx* c, const ZGemmArgs& a)
 {
   return c->gemm_adma && c->gemm_ring && a.sak == 1 && a.sbk == 1 && a.k % 16 == 0 && a.sam % 2 == 0 &&
@@ -456,27 +408,14 @@ bool ring_ok(const afqmc_ctx* c, const ZGemmArgs& a)
          ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.B & 15) == 0 && !a.conjb;
 }
 
-template <class OT, int RI, int NP> int ring_cfg(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch)
+template <class OT, int NP> int ring_run(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch, int ri)
 {
-  constexpr RingCfg t = ring_at<NP>(RI);
+  const RingCfg t = NP == 3 ? kRing3[ri] : kRing[ri];
   a.MT = (a.m + t.BM - 1) / t.BM;
   a.NT = (a.n + t.BN - 1) / t.BN;
   const long tiles = (long)a.MT * a.NT * batch;
   if (tiles > 2147483647L) return fail(c, AFQMC_ERR_SHAPE, "GEMM grid too large");
-  return launch(c, name, [&]() {
-    hipLaunchKernelGGL((zgemm_b16dma_kernel<OT, t.BM, t.BN, t.WM, t.WN, t.S, NP>), dim3((unsigned)tiles),
-                       dim3(64 * t.WM * t.WN), 0, c->stream, a);
-  });
-}
-
-template <class OT, int NP> int ring_run(afqmc_ctx* c, const char* name, const ZGemmArgs& a, int batch, int ri)
-{
-  switch (ri) {
-  case 1: return ring_cfg<OT, 1, NP>(c, name, a, batch);
-  case 2: return ring_cfg<OT, 2, NP>(c, name, a, batch);
-  case 3: return ring_cfg<OT, 3, NP>(c, name, a, batch);
-  default: return ring_cfg<OT, 0, NP>(c, name, a, batch);
-  }
+  return launch(c, name, [&]() { ring_launch<OT, NP>(c->stream, a, (unsigned)tiles, ri); });
 }
 
 int ring_default(const ZGemmArgs& a)
@@ -518,14 +457,6 @@ bool ring3_ok(const ZGemmArgs& a)
          ((uintptr_t)a.B & 15) == 0 && ((uintptr_t)a.A3 & 15) == 0 && ((uintptr_t)a.B3 & 15) == 0 && !a.conjb;
 }
 
-// FP64 products (zgemm_f64_kernel): every operand order, tile candidates
-// (rows, complex columns, waves, LDS stages).
-struct F64Cfg {
-  int BM, BN, WM, WN, S;
-};
-constexpr F64Cfg kF64[] = {{32, 32, 2, 2, 3}, {64, 64, 2, 2, 2}, {128, 64, 4, 2, 2}};
-constexpr int kNF64 = 3;
-
 F64Args f64args(int m, int n, int k)
 {
   F64Args a;
@@ -559,29 +490,18 @@ int f64_default(const F64Args& a, int batch)
   return best;
 }
 
-template <class OZ, int CI, bool DMA> int f64_cfg(afqmc_ctx* c, const char* name, F64Args a, int batch)
-{
-  constexpr F64Cfg t = kF64[CI];
-  a.MT = (a.m + t.BM - 1) / t.BM;
-  a.NT = (a.n + t.BN - 1) / t.BN;
-  const long tiles = (long)a.MT * a.NT * batch;
-  if (tiles > 2147483647L) return fail(c, AFQMC_ERR_SHAPE, "GEMM grid too large");
-  return launch(c, name, [&]() {
-    hipLaunchKernelGGL((zgemm_f64_kernel<OZ, t.BM, t.BN, t.WM, t.WN, t.S, DMA>), dim3((unsigned)tiles),
-                       dim3(64 * t.WM * t.WN), 0, c->stream, a);
-  });
-}
-
-template <class OZ> int f64_run(afqmc_ctx* c, const char* name, const F64Args& a, int batch, int ci)
+template <class OZ> int f64_run(afqmc_ctx* c, const char* name, F64Args a, int batch, int ci)
 {
   // the direct loads move 16 aligned bytes; a caller's own device pointers
-  // (the allocation-free entry point) may hold less
-  if ((((uintptr_t)a.A | (uintptr_t)a.B) & 15) != 0) return f64_cfg<OZ, 0, false>(c, name, a, batch);
-  switch (ci) {
-  case 1: return f64_cfg<OZ, 1, true>(c, name, a, batch);
-  case 2: return f64_cfg<OZ, 2, true>(c, name, a, batch);
-  default: return f64_cfg<OZ, 0, true>(c, name, a, batch);
-  }
+  // (the allocation-free entry point) may hold less: the first tile through
+  // registers
+  const bool dma = (((uintptr_t)a.A | (uintptr_t)a.B) & 15) == 0;
+  if (!dma) ci = 0;
+  a.MT = (a.m + kF64[ci].BM - 1) / kF64[ci].BM;
+  a.NT = (a.n + kF64[ci].BN - 1) / kF64[ci].BN;
+  const long tiles = (long)a.MT * a.NT * batch;
+  if (tiles > 2147483647L) return fail(c, AFQMC_ERR_SHAPE, "GEMM grid too large");
+  return launch(c, name, [&]() { f64_launch<OZ>(c->stream, a, (unsigned)tiles, ci, dma); });
 }
 
 template <class OZ> int zgemm64(afqmc_ctx* c, const char* name, const F64Args& a, int batch)
@@ -655,13 +575,13 @@ int zgemm(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch)
   char keyb[160];
   std::snprintf(keyb, sizeof(keyb), "%s/%d/%d/%d/%d/%d/%d%d", name, CP, a.m, a.n, a.k, batch, (int)AK, (int)BK);
   const std::string key(keyb);
-  if (c->force_cfg > 0 && c->force_cfg <= ncfg<CP>())
+  if (c->force_cfg > 0 && c->force_cfg <= (CP == CP_F32 ? kNF32 : kNB16))
     return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, c->force_cfg - 1);
   auto it = c->tune.find(key);
   if (it != c->tune.end() && !c->tuning) return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, it->second);
   if (!c->tuning) return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, default_cfg<CP>(a));
   int best = default_cfg<CP>(a);
-  RET(tune_tiles(c, ncfg<CP>(), best, [&](int ci) { return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, ci); }));
+  RET(tune_tiles(c, (CP == CP_F32 ? kNF32 : kNB16), best, [&](int ci) { return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, ci); }));
   c->tune[key] = best;
   return zgemm_run<CP, AT, BT, OT, AK, BK>(c, name, a, batch, best);
   }

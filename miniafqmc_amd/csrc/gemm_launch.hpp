@@ -1,0 +1,40 @@
+// The matrix-product kernels' tile candidates and launchers.  The launchers
+// are instantiated in gemm_f32.hip, gemm_b16.hip, gemm_b16b.hip, gemm_ring.hip
+// and gemm_f64.hip, so that the kernels compile side by side.
+#pragma once
+#include "gemm.hpp"
+#include "gemm_f64.hpp"
+
+// zgemm_kernel: FP32 (BKC 16 or 8 complex) and split-BF16 (BKC 16)
+struct TileCfg {
+  int BM, BNC, WM, WN;
+};
+constexpr TileCfg kCfgF32[] = {{32, 16, 1, 1}, {128, 64, 2, 2}, {128, 128, 2, 2}};
+constexpr TileCfg kCfgB16[] = {{32, 16, 1, 1}, {128, 64, 2, 2}, {128, 128, 2, 2}, {256, 64, 4, 2}, {64, 64, 2, 2}};
+constexpr int kNF32 = 3, kNB16 = 5;
+
+// Split-BF16 products whose operands are both split-BF16 with k contiguous
+// run zgemm_b16dma_kernel (both operands staged by direct loads through a
+// ring of LDS stages); candidates (rows, complex columns, waves, stages):
+struct RingCfg {
+  int BM, BN, WM, WN, S;
+};
+constexpr RingCfg kRing[] = {{128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {256, 128, 4, 2, 3}};
+// three-piece operands take half as much LDS again per stage
+constexpr RingCfg kRing3[] = {{128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {128, 128, 2, 2, 3}};
+constexpr int kNRing = 4;
+
+// FP64 products (zgemm_f64_kernel): every operand order, tile candidates
+// (rows, complex columns, waves, LDS stages).
+struct F64Cfg {
+  int BM, BN, WM, WN, S;
+};
+constexpr F64Cfg kF64[] = {{32, 32, 2, 2, 3}, {64, 64, 2, 2, 2}, {128, 64, 4, 2, 2}};
+constexpr int kNF64 = 3;
+
+// tiles: the grid; ci: the candidate; dma: split-BF16 operands staged by
+// direct loads (0 none, 1 A, 2 both)
+template <int CP, class AT, class BT, class OT, bool AK, bool BK>
+void zgemm_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ci, int dma);
+template <class OT, int NP> void ring_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ri);
+template <class OZ> void f64_launch(hipStream_t st, const F64Args& a, unsigned tiles, int ci, bool dma);

@@ -1,0 +1,28 @@
+// Split-BF16 products through the staged-ring kernel.
+#include "gemm_b16.hpp"
+#include "gemm_launch.hpp"
+
+template <class OT, int NP> void ring_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ri)
+{
+  auto go = [&](auto ric) {
+    constexpr int RI = decltype(ric)::value;
+    constexpr RingCfg t = NP == 3 ? kRing3[RI] : kRing[RI];
+    hipLaunchKernelGGL((zgemm_b16dma_kernel<OT, t.BM, t.BN, t.WM, t.WN, t.S, NP>), dim3(tiles), dim3(64 * t.WM * t.WN),
+                       0, st, a);
+  };
+  switch (ri) {
+  case 1: return go(std::integral_constant<int, 1>());
+  case 2: return go(std::integral_constant<int, 2>());
+  case 3: return go(std::integral_constant<int, 3>());
+  default: return go(std::integral_constant<int, 0>());
+  }
+}
+
+#define RING_LAUNCH(OT, NP) template void ring_launch<OT, NP>(hipStream_t, const ZGemmArgs&, unsigned, int);
+RING_LAUNCH(bfs, 1)
+RING_LAUNCH(bfs, 2)
+RING_LAUNCH(float, 2)
+RING_LAUNCH(double, 2)
+RING_LAUNCH(bfs, 3)
+RING_LAUNCH(float, 3)
+RING_LAUNCH(double, 3)
