@@ -108,3 +108,51 @@ __device__ inline zd load_z(const zf* p)
   zf v = *p;
   return {(double)v.re, (double)v.im};
 }
+
+// The exchange energy as one launch (XD mode of the GEMM kernels).  The
+// lower-triangular block of each spin is cut into chunks of xch columns
+// (AFQMC_OPT_EXCHANGE_CHUNK), chunk c holding the rows p >= c * xch; a work
+// item is a chunk's tile of BN rows for one spin.  Item t of a spin's xt:
+// chunk c has NT0 - c * xch / BN of them.  Consecutive workgroup ids are dealt
+// round-robin to the 8 XCDs, so the MT walker tiles of an item, which read the
+// same part of the block, stay on one XCD.
+struct ExchArgs {
+  const zd* G;   // FP64 density matrix [nw][2 NM] for the dot (null: plain product)
+  zd* part;      // [2][xt][nw] partial energies
+  long NM, xch;  // block size, columns per chunk
+  int xt;        // items per spin
+};
+struct ExchTile {
+  int mt, sp, t, n0;  // walker tile, spin, item, first row of the tile within its chunk
+  long q0;            // first column (and row) of the chunk
+};
+// false when the workgroup has no item (the grid is padded to 8 XCDs)
+__device__ __forceinline__ bool exch_tile(const ExchArgs& x, int MT, int BN, ExchTile& o)
+{
+  const int xtp = (x.xt + 7) & ~7;
+  const int q = blockIdx.x >> 3;
+  int t = (int)(blockIdx.x & 7) + 8 * (q / MT);
+  o.mt = q % MT;
+  o.sp = t / xtp;
+  t -= o.sp * xtp;
+  if (t >= x.xt) return false;
+  o.t = t;
+  int ntc = (int)((x.NM + BN - 1) / BN), c = 0;
+  const int d = (int)(x.xch / BN);
+  while (t >= ntc) {
+    t -= ntc;
+    ntc -= d;
+    c++;
+  }
+  o.n0 = t * BN;
+  o.q0 = (long)c * x.xch;
+  return true;
+}
+// items per spin and the padded grid
+inline int exch_items(long NM, long xch, int BN)
+{
+  long t = 0;
+  for (long q0 = 0; q0 < NM; q0 += xch) t += (NM - q0 + BN - 1) / BN;
+  return (int)t;
+}
+inline unsigned exch_grid(int xt, int MT) { return (unsigned)(2 * ((xt + 7) & ~7) * MT); }

@@ -1579,6 +1579,111 @@ int do_ortho(afqmc_ctx* c)
   });
 }
 
+// The exchange energy from the dense block in one launch: every chunk and row
+// tile of both spins is a work item whose product is dotted with G as it ends
+// (ExchArgs), and the items' partials are summed per walker.  As one product
+// and one dot per chunk and spin, 256 walkers gave each launch at most 128
+// tiles of 256 x 128 on 256 CUs (256 orbitals, three pieces: 7.1 ms per
+// energy in 32 launches).  FP64 takes chunks too: unsplit, the last tiles of
+// the triangle run alone.  Split-BF16 products keep AFQMC_OPT_EXCHANGE_CHUNK,
+// which bounds their FP32 accumulation.
+// Measured per energy: 256 orbitals, 256 walkers, three pieces 7.1 -> 2.56 ms
+// (1290 TFLOP/s of MFMA), in FP64 12.4 -> 9.0 ms (61 TFLOP/s); 384 orbitals,
+// 256 walkers, two pieces 15.2 + 1.4 -> 6.6 ms.
+constexpr long kF64ExchChunk = 2048;
+
+template <int CP> bool exch_one_ok(const afqmc_ctx* c)
+{
+  if (CP == CP_F64) return true;
+  const long NM = (long)c->N * c->M;
+  if (NM % 16) return false;
+  return CP == CP_BF16X6 || (CP == CP_BF16X3 && c->gemm_adma && c->gemm_ring);
+}
+
+// G: FP64 [nw][2NM]; Gs (and Gs3): its split forms
+template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const zb* Gs, const uint32_t* Gs3)
+{
+  const long NM = (long)c->N * c->M, nw = c->nw;
+  ExchArgs x;
+  x.G = G;
+  x.NM = NM;
+  x.xch = CP == CP_F64 ? kF64ExchChunk : c->exch_chunk > 0 ? c->exch_chunk : NM;
+  if (x.xch > NM) x.xch = NM;
+  // tile: least padded walkers over the tile's rate, with at least two
+  // workgroups per CU where the smaller tiles give them
+  int best = 0;
+  double tb = 1e300;
+  constexpr int n = CP == CP_F64 ? kNF64 : kNRing;
+  constexpr double rate64[] = {57.4, 62.7, 63.9};
+  constexpr double rateb[] = {0.86, 1.0, 1.0, 0.9, 0.55};
+  auto dims = [&](int i, int& BM, int& BN) {
+    BM = CP == CP_F64 ? kF64[i % kNF64].BM : CP == CP_BF16X6 ? kRing3[i].BM : kRing[i].BM;
+    BN = CP == CP_F64 ? kF64[i % kNF64].BN : CP == CP_BF16X6 ? kRing3[i].BN : kRing[i].BN;
+  };
+  for (int i = 0; i < n; i++) {
+    int BM, BN;
+    dims(i, BM, BN);
+    const double tiles = 2.0 * ((nw + BM - 1) / BM) * exch_items(NM, x.xch, BN);
+    const double percu = std::ceil(tiles / 256.0);
+    const double t = percu * BM * BN / ((CP == CP_F64 ? rate64[i % kNF64] : rateb[i]) * (percu < 2.0 ? 0.7 : 1.0));
+    if (t < tb) {
+      tb = t;
+      best = i;
+    }
+  }
+  if (c->force_cfg > 0 && c->force_cfg <= n) best = c->force_cfg - 1;
+  int BM, BN;
+  dims(best, BM, BN);
+  const int MT = (int)((nw + BM - 1) / BM);
+  x.xt = exch_items(NM, x.xch, BN);
+  const size_t need = sizeof(zd) * 2 * (size_t)x.xt * nw;
+  if (c->ybuf_bytes < need) {
+    dfree(c, c->Ybuf);
+    c->Ybuf = nullptr;
+    c->ybuf_bytes = 0;
+    RET(dalloc_bytes(c, &c->Ybuf, need));
+    c->ybuf_bytes = need;
+  }
+  x.part = (zd*)c->Ybuf;
+  const double inv_dt = 1.0 / c->dt_sys;
+  const unsigned grid = exch_grid(x.xt, MT);
+  if constexpr (CP == CP_F64) {
+    F64Args a = f64args((int)nw, 0, 0);
+    a.A = G;
+    a.sam = 2 * NM;
+    a.sak = 1;
+    a.B = c->Vx;
+    a.sbn = NM;
+    a.sbk = 1;
+    a.ar = inv_dt;
+    a.MT = MT;
+    a.NT = 1;
+    a.x = x;
+    RET(launch(c, "energy_vx_gemm", [&]() { f64_exch_launch(c->stream, a, grid, best); }));
+  } else {
+    ZGemmArgs a = gargs();
+    a.A = Gs;
+    a.A3 = Gs3;
+    a.sam = 2 * NM;
+    a.sak = 1;
+    a.B = c->Vx;
+    a.B3 = c->Vx3;
+    a.sbn = NM;
+    a.sbk = 1;
+    a.m = (int)nw;
+    a.ar = inv_dt;
+    a.MT = MT;
+    a.NT = 1;
+    a.x = x;
+    RET(launch(c, "energy_vx_gemm",
+               [&]() { ring_exch_launch<CP == CP_BF16X6 ? 3 : 2>(c->stream, a, grid, best); }));
+  }
+  return launch(c, "energy_exch_dot", [&]() {
+    hipLaunchKernelGGL(exch_sum_kernel, dim3((unsigned)((nw + 15) / 16), 2), dim3(256), 0, c->stream, x.part, x.xt,
+                       (int)nw, c->e_exch_part);
+  });
+}
+
 // Local energy from G in [nw][2][N][M] layout (type GT): one-body haj.G,
 // Coulomb term from v = Lv.G (Lv [2][K][NM] of type LVT, scaled by sqrt(dt),
 // contracted in precision CPV) and exchange in precision CP, from the dense
@@ -1606,7 +1711,23 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     hipLaunchKernelGGL((sumsq_kernel<zd>), dim3(nw), dim3(256), 0, c->stream, K, c->e_v, 1L, (long)K, c->e_direct,
                        inv_dt);
   }));
-  if (c->Vx) {
+  bool one = false;
+  if constexpr (std::is_same<GT, double>::value && (CP == CP_F64 || CP == CP_BF16X3 || CP == CP_BF16X6)) {
+    one = c->Vx && exch_one_ok<CP>(c);
+    if (one) {
+      if (CP == CP_BF16X3) {
+        // split-BF16 G in two pieces, as the product's loader would split it
+        if (!c->G3) RET(dalloc(c, &c->G3, 2 * (size_t)NM * nw));
+        RET(launch(c, "g_split", [&]() {
+          hipLaunchKernelGGL((zconvert_kernel<zd, zb>), dim3(nblk(2 * NM * nw, 256)), dim3(256), 0, c->stream,
+                             (const zd*)Gp, c->G3, 2 * NM * nw);
+        }));
+      }
+      RET(exch_one<CP>(c, (const zd*)Gp, c->G3, c->G3l));
+    }
+  }
+  if (one) {
+  } else if (c->Vx) {
     // exchange from the dense same-spin block of Vakbl held in HBM as its
     // lower triangle with the strictly lower part doubled:
     // Z(w, p) = sum_{q <= p} G_s(w, q) Vx'_s(p, q);  e_x(w, s) = sum_p G_s(w, p) Z(w, p)
@@ -1615,7 +1736,7 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     // the triangle) and its dot with G is added in FP64, which bounds the
     // accumulation error of reduced-precision contractions.
     using ZT = typename ztype<YT>::type;
-    const long ch = (CP != CP_F64 && c->exch_chunk > 0 && c->exch_chunk < NM) ? c->exch_chunk : NM;
+    const long ch = (c->exch_chunk > 0 && c->exch_chunk < NM) ? c->exch_chunk : NM;
     for (int sp = 0; sp < 2; sp++) {
       for (long q0 = 0; q0 < NM; q0 += ch) {
         const long kc = std::min(ch, NM - q0);

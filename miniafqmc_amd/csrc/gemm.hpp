@@ -63,6 +63,8 @@ struct ZGemmArgs {
   // and of a split-BF16 output C (when not null): its third pieces, with C's
   // element strides and batch offsets
   void* C3;
+  // XD mode of zgemm_b16dma_kernel: A, B at the spin and chunk (0, 0), m walkers
+  ExchArgs x;
 };
 
 template <class Z> __device__ inline void zero_z(Z& z)

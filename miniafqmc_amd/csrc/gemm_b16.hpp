@@ -59,9 +59,12 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 // output).  Launch conditions (checked by the host): A and B split-BF16, unit
 // k stride, rows and batch offsets 16-byte aligned, k % 16 == 0, no conj(B);
 // NP = 3 also third-piece rows 16-byte aligned.
+// XD: the exchange energy (ExchArgs): the tile's product, rounded to FP32 as
+// the stored form was, is dotted with the FP64 G of the same walkers and rows
+// and leaves one FP64 partial per walker, so the product is never stored.
 // WPE: waves per SIMD the register allocation must allow (0: no bound
 // beyond the workgroup size).
-template <class OT, int BM, int BN, int WM, int WN, int STAGES, int NP = 2, int WPE = 0>
+template <class OT, int BM, int BN, int WM, int WN, int STAGES, int NP = 2, bool XD = false, int WPE = 0>
 __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmArgs p)
 {
   constexpr int NT = 64 * WM * WN;
@@ -90,7 +93,10 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
 
   // XCD-aware tile order, as zgemm_kernel
   long lin = blockIdx.x;
-  {
+  ExchTile xt{};
+  if constexpr (XD) {
+    if (!exch_tile(p.x, p.MT, BN, xt)) return;
+  } else {
     const long T = gridDim.x, per = T / 8;
     if (p.ktri) {
       if ((p.NT & 7) == 0 && T == (long)p.MT * p.NT) {
@@ -101,17 +107,20 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
       lin = (lin % 8) * per + lin / 8;
     }
   }
-  const int mt = (int)(lin % p.MT);
+  const int mt = XD ? xt.mt : (int)(lin % p.MT);
   const long rest = lin / p.MT;
   const int ntl = (int)(rest % p.NT);
-  const int m0 = mt * BM, n0 = (p.ktri ? p.NT - 1 - ntl : ntl) * BN;
-  const int kend = p.ktri ? min(p.k, n0 + BN) : p.k;
-  const int b = (int)(rest / p.NT);
-  const long bq = b / p.bdiv, br_ = b % p.bdiv;
-  const zb* __restrict__ A = (const zb*)p.A + bq * p.sa1 + br_ * p.sa2;
-  const zb* __restrict__ B = (const zb*)p.B + bq * p.sb1 + br_ * p.sb2;
-  const uint32_t* __restrict__ A3 = NP == 3 ? (const uint32_t*)p.A3 + bq * p.sa1 + br_ * p.sa2 : nullptr;
-  const uint32_t* __restrict__ B3 = NP == 3 ? (const uint32_t*)p.B3 + bq * p.sb1 + br_ * p.sb2 : nullptr;
+  const int m0 = mt * BM, n0 = XD ? xt.n0 : (p.ktri ? p.NT - 1 - ntl : ntl) * BN;
+  const int pn = XD ? (int)(p.x.NM - xt.q0) : p.n;  // rows of B
+  const int kend = XD ? (int)min(min(p.x.xch, p.x.NM - xt.q0), (long)(n0 + BN)) : p.ktri ? min(p.k, n0 + BN) : p.k;
+  const int b = XD ? 0 : (int)(rest / p.NT);
+  const long bq = XD ? 0 : b / p.bdiv, br_ = XD ? 0 : b % p.bdiv;
+  const long oa = XD ? xt.sp * p.x.NM + xt.q0 : bq * p.sa1 + br_ * p.sa2;
+  const long ob = XD ? (xt.sp * p.x.NM + xt.q0) * p.x.NM + xt.q0 : bq * p.sb1 + br_ * p.sb2;
+  const zb* __restrict__ A = (const zb*)p.A + oa;
+  const zb* __restrict__ B = (const zb*)p.B + ob;
+  const uint32_t* __restrict__ A3 = NP == 3 ? (const uint32_t*)p.A3 + oa : nullptr;
+  const uint32_t* __restrict__ B3 = NP == 3 ? (const uint32_t*)p.B3 + ob : nullptr;
 
   __shared__ __align__(16) uint2 s0[STG];
   __shared__ __align__(16) uint2 s1[STG];
@@ -131,7 +140,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
 #pragma unroll
   for (int i = 0; i < BL; i++) {
     const int u = i * NT + tid, row = u / CH, pc = u % CH;
-    pb[i] = B + (long)min(n0 + row, p.n - 1) * p.sbn + 2 * (pc ^ b16::swz(row));
+    pb[i] = B + (long)min(n0 + row, pn - 1) * p.sbn + 2 * (pc ^ b16::swz(row));
   }
   // third pieces: unit u is slot u % 8 of LDS row u / 8 = 16q + r, which
   // holds chunk x / 2 (four complex) of tile row 32q + 16 (x & 1) + r, where
@@ -151,7 +160,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
 #pragma unroll
   for (int i = 0; i < BL3; i++) {
     const int u = i * NT + tid;
-    pb3[i] = B3 + (long)min(n0 + row3(u), p.n - 1) * p.sbn + 4 * chunk3(u);
+    pb3[i] = B3 + (long)min(n0 + row3(u), pn - 1) * p.sbn + 4 * chunk3(u);
   }
   const int w0 = __builtin_amdgcn_readfirstlane(wave);
   auto issue = [&](uint2* st, int k0) __attribute__((always_inline)) {
@@ -328,6 +337,44 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
       if (j + 3 < nk + STAGES - 1) step(std::integral_constant<int, 3>(), j + 3);
   }
 
+  if constexpr (XD) {
+    // lane: element (walker 4g + q, row r) of each block; the tile's dot per
+    // walker over the lane's rows, the 16 lanes of a group, then the WN waves
+    __shared__ zd red[WN][BM];
+    const zd* G = p.x.G + xt.sp * p.x.NM + xt.q0 + n0 + wn * WTN + r;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int lw = wm * WTM + 16 * i + 4 * g + q;
+        const zd* Gw = G + (long)min(m0 + lw, p.m - 1) * 2 * p.x.NM;
+        zd a{0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          if (n0 + wn * WTN + 16 * j + r >= pn) continue;
+          const double y_r = (double)(float)(p.ar * (double)cr[i][j][q]);
+          const double y_i = (double)(float)(p.ar * (double)ci[i][j][q]);
+          const zd gv = Gw[16 * j];
+          a.re += gv.re * y_r - gv.im * y_i;
+          a.im += gv.re * y_i + gv.im * y_r;
+        }
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+          a.re += __shfl_xor(a.re, o);
+          a.im += __shfl_xor(a.im, o);
+        }
+        if (r == 0) red[wn][lw] = a;
+      }
+    __syncthreads();
+    for (int lw = tid; lw < BM; lw += NT) {
+      if (m0 + lw >= p.m) continue;
+      zd a = red[0][lw];
+#pragma unroll
+      for (int v = 1; v < WN; v++) a = zadd(a, red[v][lw]);
+      p.x.part[((long)xt.sp * p.x.xt + xt.t) * p.m + m0 + lw] = a;
+    }
+    return;
+  }
   // epilogue: the lane holds (re, im) of complex element (row 4g + q, column
   // r) of each 16 x 16 block; arithmetic in FP64 as zgemm_kernel's epilogue
   constexpr bool OSPLIT = std::is_same<OT, bfs>::value;

@@ -62,6 +62,8 @@ struct F64Args {
   // (0: every item covers k)
   long ktot;
   int MT, NT;                 // tile grid (filled by the launcher)
+  // XD mode: A, B at the spin and chunk (0, 0), m walkers
+  ExchArgs x;
 };
 
 namespace f64g {
@@ -80,8 +82,10 @@ __device__ __forceinline__ void put(zb* p, long o, double re, double im) { p[o] 
 } // namespace f64g
 
 // OZ: element of C and F (zd, zf; zb without F and beta).  DMA = false: the
-// operands pass through registers (operands not aligned to 16 bytes).
-template <class OZ, int BM, int BN, int WM, int WN, int STAGES, bool DMA = true>
+// operands pass through registers (operands not aligned to 16 bytes).  XD:
+// the exchange energy (ExchArgs), the tile's product dotted with G into one
+// partial per walker instead of being stored.
+template <class OZ, int BM, int BN, int WM, int WN, int STAGES, bool DMA = true, bool XD = false>
 __global__ __launch_bounds__(64 * WM * WN) void zgemm_f64_kernel(F64Args p)
 {
   constexpr int NT = 64 * WM * WN;
@@ -109,7 +113,10 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_f64_kernel(F64Args p)
   // XCDs, so each gets a contiguous run of tiles; triangular products deal
   // their column tiles round-robin instead, heaviest first
   long lin = blockIdx.x;
-  {
+  ExchTile xt{};
+  if constexpr (XD) {
+    if (!exch_tile(p.x, p.MT, BN, xt)) return;
+  } else {
     const long T = gridDim.x, per = T / 8;
     if (p.ktri) {
       if ((p.NT & 7) == 0 && T == (long)p.MT * p.NT) {
@@ -120,17 +127,22 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_f64_kernel(F64Args p)
       lin = (lin % 8) * per + lin / 8;
     }
   }
-  const int mt = (int)(lin % p.MT);
+  const int mt = XD ? xt.mt : (int)(lin % p.MT);
   const long rest = lin / p.MT;
   const int ntl = (int)(rest % p.NT);
-  const int m0 = mt * BM, n0 = (p.ktri ? p.NT - 1 - ntl : ntl) * BN;
-  const int b = (int)(rest / p.NT);
-  const long bq = b / p.bdiv, br_ = b % p.bdiv;
+  const int m0 = mt * BM, n0 = XD ? xt.n0 : (p.ktri ? p.NT - 1 - ntl : ntl) * BN;
+  const int b = XD ? 0 : (int)(rest / p.NT);
+  const long bq = XD ? 0 : b / p.bdiv, br_ = XD ? 0 : b % p.bdiv;
+  const int pn = XD ? (int)(p.x.NM - xt.q0) : p.n;
   int kend = p.k;
-  if (p.ktot) kend = (int)min((long)p.k, p.ktot - br_ * p.k);
-  if (p.ktri) kend = min(kend, n0 + BN);
-  const zd* A = (const zd*)p.A + bq * p.sa1 + br_ * p.sa2;
-  const zd* B = (const zd*)p.B + bq * p.sb1 + br_ * p.sb2;
+  if constexpr (XD) {
+    kend = (int)min(min(p.x.xch, p.x.NM - xt.q0), (long)(n0 + BN));
+  } else {
+    if (p.ktot) kend = (int)min((long)p.k, p.ktot - br_ * p.k);
+    if (p.ktri) kend = min(kend, n0 + BN);
+  }
+  const zd* A = (const zd*)p.A + (XD ? xt.sp * p.x.NM + xt.q0 : bq * p.sa1 + br_ * p.sa2);
+  const zd* B = (const zd*)p.B + (XD ? (xt.sp * p.x.NM + xt.q0) * p.x.NM + xt.q0 : bq * p.sb1 + br_ * p.sb2);
 
   // unit u = i * NT + tid of a tile is (row u / 8, slot u % 8) and holds the
   // row's k = slot ^ swz(row), which is the same for all of a thread's units
@@ -140,12 +152,12 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_f64_kernel(F64Args p)
 #pragma unroll
   for (int i = 0; i < AL; i++) {
     const int row = min(m0 + (i * NT + tid) / KT, p.m - 1);
-    pa[i] = A + (long)(row / p.mi) * p.samo + (long)(row % p.mi) * p.sam + (long)kc * p.sak;
+    pa[i] = A + (XD ? (long)row * p.sam : (long)(row / p.mi) * p.samo + (long)(row % p.mi) * p.sam) + (long)kc * p.sak;
   }
 #pragma unroll
   for (int i = 0; i < BL; i++) {
-    const int col = min(n0 + (i * NT + tid) / KT, p.n - 1);
-    pb[i] = B + (long)(col / p.ni) * p.sbno + (long)(col % p.ni) * p.sbn + (long)kc * p.sbk;
+    const int col = min(n0 + (i * NT + tid) / KT, pn - 1);
+    pb[i] = B + (XD ? (long)col * p.sbn : (long)(col / p.ni) * p.sbno + (long)(col % p.ni) * p.sbn) + (long)kc * p.sbk;
   }
   const int w0 = __builtin_amdgcn_readfirstlane(wave);
   const int klast = kend - 1 - kc;  // largest k0 whose chunk lies inside (may be negative)
@@ -263,6 +275,43 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_f64_kernel(F64Args p)
       if (j + 3 < nk + STAGES - 1) step(std::integral_constant<int, 3>(), j + 3);
   }
 
+  if constexpr (XD) {
+    // lane: element (walker 4q + g, row r) of each block; the tile's dot per
+    // walker over the lane's rows, the 16 lanes of a group, then the WN waves
+    __shared__ zd red[WN][BM];
+    const zd* G = p.x.G + xt.sp * p.x.NM + xt.q0 + n0 + wn * WTN + r;
+#pragma unroll
+    for (int i = 0; i < TM; i++)
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int lw = wm * WTM + 16 * i + 4 * q + g;
+        const zd* Gw = G + (long)min(m0 + lw, p.m - 1) * 2 * p.x.NM;
+        zd a{0.0, 0.0};
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          if (n0 + wn * WTN + 16 * j + r >= pn) continue;
+          const double y_r = p.ar * cr[i][j][q], y_i = p.ar * ci[i][j][q];
+          const zd gv = Gw[16 * j];
+          a.re += gv.re * y_r - gv.im * y_i;
+          a.im += gv.re * y_i + gv.im * y_r;
+        }
+#pragma unroll
+        for (int o = 1; o < 16; o <<= 1) {
+          a.re += __shfl_xor(a.re, o);
+          a.im += __shfl_xor(a.im, o);
+        }
+        if (r == 0) red[wn][lw] = a;
+      }
+    __syncthreads();
+    for (int lw = tid; lw < BM; lw += NT) {
+      if (m0 + lw >= p.m) continue;
+      zd a = red[0][lw];
+#pragma unroll
+      for (int v = 1; v < WN; v++) a = zadd(a, red[v][lw]);
+      p.x.part[((long)xt.sp * p.x.xt + xt.t) * p.m + m0 + lw] = a;
+    }
+    return;
+  }
   // epilogue: the lane holds complex element (row 4q + g, column r) of each
   // 16 x 16 block
   const long coff = bq * p.sc1 + br_ * p.sc2;

@@ -19,10 +19,12 @@ constexpr int kNF32 = 3, kNB16 = 5;
 struct RingCfg {
   int BM, BN, WM, WN, S;
 };
-constexpr RingCfg kRing[] = {{128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {256, 128, 4, 2, 3}};
+constexpr RingCfg kRing[] = {
+    {128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {256, 128, 4, 2, 3}, {64, 64, 2, 2, 2}};
 // three-piece operands take half as much LDS again per stage
-constexpr RingCfg kRing3[] = {{128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {128, 128, 2, 2, 3}};
-constexpr int kNRing = 4;
+constexpr RingCfg kRing3[] = {
+    {128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {128, 128, 2, 2, 3}, {64, 64, 2, 2, 2}};
+constexpr int kNRing = 5;
 
 // FP64 products (zgemm_f64_kernel): every operand order, tile candidates
 // (rows, complex columns, waves, LDS stages).
@@ -38,3 +40,6 @@ template <int CP, class AT, class BT, class OT, bool AK, bool BK>
 void zgemm_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ci, int dma);
 template <class OT, int NP> void ring_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ri);
 template <class OZ> void f64_launch(hipStream_t st, const F64Args& a, unsigned tiles, int ci, bool dma);
+// the exchange energy (a.x, grid from exch_grid)
+template <int NP> void ring_exch_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ri);
+void f64_exch_launch(hipStream_t st, const F64Args& a, unsigned tiles, int ci);

@@ -2,21 +2,35 @@
 #include "gemm_b16.hpp"
 #include "gemm_launch.hpp"
 
-template <class OT, int NP> void ring_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ri)
+namespace {
+template <class OT, int NP, bool XD> void ring_go(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ri)
 {
   auto go = [&](auto ric) {
     constexpr int RI = decltype(ric)::value;
     constexpr RingCfg t = NP == 3 ? kRing3[RI] : kRing[RI];
-    hipLaunchKernelGGL((zgemm_b16dma_kernel<OT, t.BM, t.BN, t.WM, t.WN, t.S, NP>), dim3(tiles), dim3(64 * t.WM * t.WN),
-                       0, st, a);
+    hipLaunchKernelGGL((zgemm_b16dma_kernel<OT, t.BM, t.BN, t.WM, t.WN, t.S, NP, XD>), dim3(tiles),
+                       dim3(64 * t.WM * t.WN), 0, st, a);
   };
   switch (ri) {
   case 1: return go(std::integral_constant<int, 1>());
   case 2: return go(std::integral_constant<int, 2>());
   case 3: return go(std::integral_constant<int, 3>());
+  case 4: return go(std::integral_constant<int, 4>());
   default: return go(std::integral_constant<int, 0>());
   }
 }
+} // namespace
+
+template <class OT, int NP> void ring_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ri)
+{
+  ring_go<OT, NP, false>(st, a, tiles, ri);
+}
+template <int NP> void ring_exch_launch(hipStream_t st, const ZGemmArgs& a, unsigned tiles, int ri)
+{
+  ring_go<float, NP, true>(st, a, tiles, ri);
+}
+template void ring_exch_launch<2>(hipStream_t, const ZGemmArgs&, unsigned, int);
+template void ring_exch_launch<3>(hipStream_t, const ZGemmArgs&, unsigned, int);
 
 #define RING_LAUNCH(OT, NP) template void ring_launch<OT, NP>(hipStream_t, const ZGemmArgs&, unsigned, int);
 RING_LAUNCH(bfs, 1)

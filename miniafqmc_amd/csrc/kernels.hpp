@@ -1531,6 +1531,25 @@ __global__ __launch_bounds__(256) void coldot_kernel(int n, const AT* __restrict
   }
 }
 
+// out[2 w + sp] = sum_t part[sp][t][w] (the exchange energy's partials), 16
+// walkers and 16 groups of items per workgroup, summed in a fixed order.
+__global__ __launch_bounds__(256) void exch_sum_kernel(const zd* __restrict__ part, int xt, int nw,
+                                                       zd* __restrict__ out)
+{
+  __shared__ zd sh[16][16];
+  const int wl = threadIdx.x & 15, grp = threadIdx.x >> 4, sp = blockIdx.y;
+  const int w = blockIdx.x * 16 + wl;
+  zd a{0, 0};
+  if (w < nw)
+    for (int t = grp; t < xt; t += 16) a = zadd(a, part[((long)sp * xt + t) * nw + w]);
+  sh[grp][wl] = a;
+  __syncthreads();
+  if (grp == 0 && w < nw) {
+    for (int q = 1; q < 16; q++) a = zadd(a, sh[q][wl]);
+    out[2 * w + sp] = a;
+  }
+}
+
 // Exchange reduction: for each batch item q (a walker-spin and a chunk of
 // Cholesky vectors), sum over n in the chunk of sum_ab Y_n(a,b) Y_n(b,a),
 // with Y stored [nq][N][N] per n.  out[q] += result (FP64 accumulation).

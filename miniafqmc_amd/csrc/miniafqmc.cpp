@@ -30,7 +30,7 @@ namespace {
 // upload fall under none.
 struct TimerSites {
   const char* timer;
-  const char* sites[17];
+  const char* sites[18];
 };
 const TimerSites kTimers[] = {
     {"compact Mixed Density Matrix", {"gc_gemm", "det_restore"}},
@@ -46,7 +46,7 @@ const TimerSites kTimers[] = {
     {"Local Energy",
      {"energy_one", "energy_two", "energy_direct", "energy_exch_dot", "energy_pairsum", "energy_assemble",
       "energy_zero", "energy_trace", "energy_v_gemm", "energy_v_reduce", "energy_vx_gemm", "energy_y_gemm", "csrmm_vakbl", "g_transpose",
-      "gc64_gemm", "convert", "g_split3"}},
+      "gc64_gemm", "convert", "g_split", "g_split3"}},
 };
 
 void print_help()

@@ -67,3 +67,34 @@ def test_noalloc_pointers_aligned_to_eight_bytes(require_gpu, M, N, nw):
         assert np.array_equal(got[0][0], got[1][0]) and np.array_equal(got[0][1], got[1][1])
     finally:
         hip.free_all()
+
+
+@pytest.mark.parametrize("mode,level,tol", [("fp64_dense", 1, 1e-11), ("mixed_bf16", 1, 5e-5), ("mixed_bf16", 2, 2e-6)])
+@pytest.mark.parametrize("M,N,nw", [(16, 4, 3), (40, 8, 129), (64, 36, 65), (48, 45, 20)])
+def test_exchange_in_one_launch_vs_cholesky_form(require_gpu, mode, level, tol, M, N, nw):
+    """The exchange energy's work items (chunk, row tile, walker tile, spin)
+    against the Cholesky form in FP64, per walker and relative to the largest
+    exchange energy: N*M below one tile, one chunk, and a second chunk that
+    is partial (2304, 2160 with chunks of 2048), at tile remainders of
+    walkers.  Tolerances: FP64 sums; two-piece (16-bit) and three-piece
+    (24-bit) operands of terms of one sign or another, a few times their
+    rounding."""
+    say("exchange", mode, level, M, N, nw)
+    s = m.make_system(M, N, 32, density=0.7, sigma_L=0.05, sigma_h=1.0, dt=0.005, seed=M * N)
+    W = walkers(s, nw, seed=nw)
+    Wd = np.zeros((nw, 8), complex)
+    Wd[:, 1] = 1.0
+    ex = []
+    for md, lv, dense in ((mode, level, True), ("fp64_dense", 1, False)):
+        g = m.AfqmcSys(s, nw, md, energy_precision=lv, dense_exchange=dense, cutoff=-1.0)
+        for tile in (0, 1, 2, 3, 5) if dense else (0,):
+            g.set_tile(tile)
+            g.set(nat.BUF_W, W)
+            g.set(nat.BUF_WDATA, Wd)
+            g.calculate_mixed_density_matrix()
+            g.calculate_energy()
+            ex.append(g.energy_terms()[:, 2])
+        g.close()
+    ref = ex.pop()
+    for e in ex:
+        assert np.abs(e - ref).max() <= tol * np.abs(ref).max()
