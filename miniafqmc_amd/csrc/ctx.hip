@@ -14,6 +14,7 @@
 #include "common.hpp"
 #include "gemm_launch.hpp"
 #include "kernels.hpp"
+#include "prop_small.hpp"
 #include "propagate.hpp"
 
 #include <dlfcn.h>
@@ -1398,6 +1399,19 @@ int do_propagate(afqmc_ctx* c)
   c->t1inv_valid = false;
   c->g_fresh = false;
   if (c->three & 4) return propagate_three(c);
+  // small systems in one kernel (a forced GEMM tile keeps the GEMM chain)
+  const int fmt = c->mode == AFQMC_MIXED_FP32 ? 1 : c->mode == AFQMC_MIXED_BF16 ? 2 : 0;
+  if (c->force_cfg == 0 && prop_small_ok(fmt, c->M)) {
+    PropSmallArgs a;
+    a.W = c->W;
+    a.P = fmt ? c->propg32 : c->propg;
+    a.V = c->mode == AFQMC_FP64_CSR ? c->vHSw : c->vHS;
+    a.M = c->M;
+    a.N = c->N;
+    a.nw = c->nw;
+    a.ncb = 0;
+    return launch(c, "prop_fused", [&]() { prop_small_launch(c->stream, a, fmt); });
+  }
   if (fused_prop_ok(c)) return propagate_fused(c);
   if (c->mode == AFQMC_FP64_CSR) return propagate_f64(c, c->vHSw);
   if (c->mode == AFQMC_FP64_DENSE) return propagate_f64(c, (const zd*)c->vHS);
