@@ -116,7 +116,10 @@ typedef enum {
    * over all columns.  May be changed at any time.  No counterpart in the
    * reference (its energy is FP64 throughout). */
   AFQMC_OPT_EXCHANGE_CHUNK = 4,
-  /* AFQMC_MIXED_BF16 with M a multiple of 64 up to 512 and N a multiple of
+  /* (Up to 192 orbitals, 128 in FP64, the propagator runs as one kernel of
+   * its own whatever this option says, unless a GEMM tile is forced or
+   * products take three pieces.)
+   * AFQMC_MIXED_BF16 with M a multiple of 64 up to 512 and N a multiple of
    * 16: 1 runs the whole propagator (P W, the six Taylor terms, P U) as one
    * kernel per walker and 32 columns, U kept in LDS; 0 (default) runs it as
    * eight GEMM launches, which measured 2 % faster at 512 orbitals.  Both
