@@ -398,6 +398,7 @@ int zgemm_run(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch, int ci)
 
 template <int CP> int default_cfg(const ZGemmArgs& a)
 {
+  if (CP == CP_BF16X3 && a.m >= 48 && a.n >= 128) return 4;  // 64 x 64 tiles
   if (a.m >= 96 && a.n >= 48) return 1;  // 128 x 64 tiles
   return 0;                              // one-wave 32 x 16 tiles
 }
@@ -419,11 +420,24 @@ template <class OT, int NP> int ring_run(afqmc_ctx* c, const char* name, ZGemmAr
   return launch(c, name, [&]() { ring_launch<OT, NP>(c->stream, a, (unsigned)tiles, ri); });
 }
 
-int ring_default(const ZGemmArgs& a)
+// The ring tile with the least estimated time, as f64_default.
+template <int NP> int ring_default(const ZGemmArgs& a, int batch)
 {
-  if (a.m >= 256 && a.n >= 128) return 1;
-  if (a.m >= 128 && a.n >= 256) return 2;
-  return 0;
+  int best = 0;
+  double tb = 1e300;
+  for (int i = 0; i < kNRing; i++) {
+    const RingCfg t = NP == 3 ? kRing3[i] : kRing[i];
+    const double rate = NP == 3 ? kRingRate3[i] : kRingRate[i];
+    const double tiles = (double)((a.m + t.BM - 1) / t.BM) * ((a.n + t.BN - 1) / t.BN) * batch;
+    const double percu = std::ceil(tiles / 256.0);
+    // four waves alone on a CU leave gaps (eight are two per SIMD)
+    const double e = percu * t.BM * t.BN / (rate * (percu < 2.0 && t.WM * t.WN < 8 ? 0.7 : 1.0));
+    if (e < tb) {
+      tb = e;
+      best = i;
+    }
+  }
+  return best;
 }
 
 template <class OT, int NP = 2> int zgemm_ring(afqmc_ctx* c, const char* name, const ZGemmArgs& a, int batch)
@@ -434,8 +448,8 @@ template <class OT, int NP = 2> int zgemm_ring(afqmc_ctx* c, const char* name, c
   if (c->force_cfg > 0 && c->force_cfg <= kNRing) return ring_run<OT, NP>(c, name, a, batch, c->force_cfg - 1);
   auto it = c->tune.find(key);
   if (it != c->tune.end() && !c->tuning) return ring_run<OT, NP>(c, name, a, batch, it->second);
-  if (!c->tuning) return ring_run<OT, NP>(c, name, a, batch, ring_default(a));
-  int best = ring_default(a);
+  if (!c->tuning) return ring_run<OT, NP>(c, name, a, batch, ring_default<NP>(a, batch));
+  int best = ring_default<NP>(a, batch);
   RET(tune_tiles(c, kNRing, best, [&](int ri) { return ring_run<OT, NP>(c, name, a, batch, ri); }));
   c->tune[key] = best;
   return ring_run<OT, NP>(c, name, a, batch, best);
@@ -1275,28 +1289,40 @@ int propagate_chain(afqmc_ctx* c, const void* P, const void* V)
   return AFQMC_OK;
 }
 
-// The propagator in three-piece split-BF16: W is transposed into three-piece
-// terms ([N][M] per walker and spin) and P W is written in that layout as
-// well (split, plus FP32 for the epilogues' F), so that every product reads
-// both operands k-contiguous through the staged-ring kernel.  Each product
-// runs in three, two or one pieces as `three_steps` / `one_steps` say (the
-// (h, m) words of a three-piece operand are its two-piece split, h alone its
-// one-piece form); a term is written with its third pieces only when the
-// product that reads it takes three.
-int propagate_three(afqmc_ctx* c)
+// The split-BF16 propagator through the staged-ring kernel: W is transposed
+// into split terms ([N][M] per walker and spin) and P W is written in that
+// layout as well (split, plus FP32 for the epilogues' F), so that every
+// product reads both operands k-contiguous and the spins (and, against P,
+// the walkers) are columns of one product: a Horner step is one M x 2N
+// product per walker, P W and P U one product over all walkers.  (As M x N
+// products per walker and spin, 64 electrons filled half a tile.)
+//
+// With the three-piece option each product runs in three, two or one pieces
+// as `three_steps` / `one_steps` say (the (h, m) words of a three-piece
+// operand are its two-piece split, h alone its one-piece form); a term is
+// written with its third pieces only when the product that reads it takes
+// three.  Without it every product takes two pieces.
+int propagate_split(afqmc_ctx* c)
 {
   const int M = c->M, N = c->N, nw = c->nw;
   const long MN = (long)M * N, MM = (long)M * M;
   const dim3 tgrid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)(2 * nw));
+  const bool opt3 = (c->three & 4) != 0;
   // product j in launch order: 0 P W, 7-k the Horner step k, 7 P U
-  auto three = [&](int j) { return ((c->three_steps >> j) & 1) != 0; };
-  auto one = [&](int j) { return !three(j) && ((c->one_steps >> j) & 1) != 0; };
+  auto three = [&](int j) { return opt3 && ((c->three_steps >> j) & 1) != 0; };
+  auto one = [&](int j) { return opt3 && !three(j) && ((c->one_steps >> j) & 1) != 0; };
   zb* Ta = (zb*)c->Ta;
   zb* Tb = (zb*)c->Tb;
   RET(launch(c, "prop_split_w", [&]() {
-    hipLaunchKernelGGL(transpose_split3_kernel<zd>, tgrid, dim3(256), 0, c->stream, (const zd*)c->W, Tb, c->tp_Tb, M, N);
+    if (opt3)
+      hipLaunchKernelGGL((transpose_split_kernel<zd, true>), tgrid, dim3(256), 0, c->stream, (const zd*)c->W, Tb,
+                         c->tp_Tb, M, N);
+    else
+      hipLaunchKernelGGL((transpose_split_kernel<zd, false>), tgrid, dim3(256), 0, c->stream, (const zd*)c->W, Tb,
+                         (uint32_t*)nullptr, M, N);
   }));
-  auto base = [&]() {
+  // m = M rows against n columns of M (terms [column][M])
+  auto base = [&](int n) {
     ZGemmArgs a = gargs();
     a.A = c->propg32;
     a.A3 = c->tp_P;
@@ -1304,28 +1330,23 @@ int propagate_three(afqmc_ctx* c)
     a.sak = 1;
     a.sbn = M;
     a.sbk = 1;
-    a.sb1 = 2 * MN;
-    a.sb2 = MN;
-    a.bdiv = 2;
     a.m = M;
-    a.n = N;
+    a.n = n;
     a.k = M;
-    a.scm = 1;  // terms transposed per walker and spin, [N][M]
+    a.scm = 1;
     a.scn = M;
-    a.sc1 = 2 * MN;
-    a.sc2 = MN;
     return a;
   };
   {  // S = P W: U_7 = S split (third pieces when U_6's product takes three)
      // into Ta, and S in FP32 in the same layout (D) for the Horner epilogues
-    ZGemmArgs a = base();
+    ZGemmArgs a = base(2 * nw * N);
     a.B = Tb;
     a.B3 = c->tp_Tb;
     a.C = Ta;
     a.C3 = three(1) ? c->tp_Ta : nullptr;
     a.D = c->S;
-    if (three(0)) RET((zgemm<CP_BF16X6, bfs, bfs, bfs, true, true>(c, "prop_pw", a, 2 * nw)));
-    else RET((zgemm<CP_BF16X3, bfs, bfs, bfs, true, true>(c, "prop_pw", a, 2 * nw)));
+    if (three(0)) RET((zgemm<CP_BF16X6, bfs, bfs, bfs, true, true>(c, "prop_pw", a, 1)));
+    else RET((zgemm<CP_BF16X3, bfs, bfs, bfs, true, true>(c, "prop_pw", a, 1)));
   }
   // Horner's rule as propagate_chain: U_7 = S, U_k = S + (i/k) V U_{k+1}
   zb* prev = Ta;
@@ -1333,11 +1354,12 @@ int propagate_three(afqmc_ctx* c)
   zb* bufs[2] = {Tb, Ta};
   uint32_t* bufs3[2] = {c->tp_Tb, c->tp_Ta};
   for (int k = 6; k >= 1; k--) {
-    ZGemmArgs a = base();
+    ZGemmArgs a = base(2 * N);
     a.A = c->vHS;
     a.A3 = c->tp_vHS;
     a.sa1 = MM;
-    a.sa2 = 0;
+    a.sb1 = 2 * MN;
+    a.sc1 = 2 * MN;
     a.B = prev;
     a.B3 = prev3;
     a.C = bufs[k & 1];
@@ -1346,23 +1368,33 @@ int propagate_three(afqmc_ctx* c)
     a.ai = 1.0 / (double)k;
     a.F = c->S;  // same layout as C
     a.cf = 1;
-    if (three(7 - k)) RET((zgemm<CP_BF16X6, bfs, bfs, bfs, true, true>(c, "prop_taylor", a, 2 * nw)));
-    else if (one(7 - k)) RET((zgemm<CP_BF16X1, bfs, bfs, bfs, true, true>(c, "prop_taylor", a, 2 * nw)));
-    else RET((zgemm<CP_BF16X3, bfs, bfs, bfs, true, true>(c, "prop_taylor", a, 2 * nw)));
+    if (three(7 - k)) RET((zgemm<CP_BF16X6, bfs, bfs, bfs, true, true>(c, "prop_taylor", a, nw)));
+    else if (one(7 - k)) RET((zgemm<CP_BF16X1, bfs, bfs, bfs, true, true>(c, "prop_taylor", a, nw)));
+    else RET((zgemm<CP_BF16X3, bfs, bfs, bfs, true, true>(c, "prop_taylor", a, nw)));
     prev = bufs[k & 1];
     prev3 = bufs3[k & 1];
   }
-  {  // W = P U_1
-    ZGemmArgs a = base();
-    a.B = prev;
-    a.B3 = prev3;
-    a.C = c->W;
-    a.scm = N;
-    a.scn = 1;
-    if (three(7)) RET((zgemm<CP_BF16X6, bfs, bfs, double, true, true>(c, "prop_ps", a, 2 * nw)));
-    else RET((zgemm<CP_BF16X3, bfs, bfs, double, true, true>(c, "prop_ps", a, 2 * nw)));
+  // W = P U_1, column (w, s, a) to W[w][s][.][a]
+  ZGemmArgs a = base(2 * nw * N);
+  a.B = prev;
+  a.B3 = prev3;
+  a.C = c->W;
+  a.scm = N;
+  a.scn = 1;
+  if (three(7) || (c->gemm_adma && c->gemm_ring)) {
+    a.cni = N;
+    a.scno = MN;
+    if (three(7)) return zgemm<CP_BF16X6, bfs, bfs, double, true, true>(c, "prop_ps", a, 1);
+    return zgemm<CP_BF16X3, bfs, bfs, double, true, true>(c, "prop_ps", a, 1);
   }
-  return AFQMC_OK;
+  // the register-staged kernel (AFQMC_OPT_DIRECT_LDS below 2) takes a batch
+  a.n = N;
+  a.sb1 = 2 * MN;
+  a.sb2 = MN;
+  a.sc1 = 2 * MN;
+  a.sc2 = MN;
+  a.bdiv = 2;
+  return zgemm<CP_BF16X3, bfs, bfs, double, true, true>(c, "prop_ps", a, 2 * nw);
 }
 
 // W <- P E6(V) P W in one kernel per (walker, 32 columns) (propagate.hpp):
@@ -1398,7 +1430,7 @@ int do_propagate(afqmc_ctx* c)
 {
   c->t1inv_valid = false;
   c->g_fresh = false;
-  if (c->three & 4) return propagate_three(c);
+  if (c->three & 4) return propagate_split(c);
   // small systems in one kernel (a forced GEMM tile keeps the GEMM chain)
   const int fmt = c->mode == AFQMC_MIXED_FP32 ? 1 : c->mode == AFQMC_MIXED_BF16 ? 2 : 0;
   if (c->force_cfg == 0 && prop_small_ok(fmt, c->M)) {
@@ -1417,6 +1449,7 @@ int do_propagate(afqmc_ctx* c)
   if (c->mode == AFQMC_FP64_DENSE) return propagate_f64(c, (const zd*)c->vHS);
   if (c->mode == AFQMC_MIXED_FP32)
     return propagate_chain<CP_F32, float, float, float, float>(c, c->propg32, c->vHS);
+  if (c->gemm_adma && c->gemm_ring && c->M % 16 == 0) return propagate_split(c);
   return propagate_chain<CP_BF16X3, float, bfs, bfs, bfs>(c, c->propg32, c->vHS);
 }
 

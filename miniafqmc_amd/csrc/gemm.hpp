@@ -63,6 +63,10 @@ struct ZGemmArgs {
   // and of a split-BF16 output C (when not null): its third pieces, with C's
   // element strides and batch offsets
   void* C3;
+  // zgemm_b16dma_kernel: output column n at (n / cni) * scno + (n % cni) * scn
+  // when cni is nonzero (columns of several batch items side by side)
+  int cni;
+  long scno;
   // XD mode of zgemm_b16dma_kernel: A, B at the spin and chunk (0, 0), m walkers
   ExchArgs x;
 };

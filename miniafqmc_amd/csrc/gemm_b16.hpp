@@ -35,6 +35,14 @@
 // swizzled half-rows do not).  The six products h*h, h*m, m*h, h*l, l*h,
 // m*m accumulate in that order.
 //
+// The epilogue moves whole complex numbers, 16 bytes at a time where a lane's
+// rows are contiguous, and holds one block's F and C at a time: with all of a
+// row block's in registers the FP32 and FP64 output forms spilled 70 to 105
+// registers per lane (512 orbitals, 1024 walkers, 256 x 128 tiles: P U
+// 3.9 -> 2.47 ms, Horner steps 1.74 -> 1.48 ms, of which 1.06 is their HBM
+// traffic at the rate of a large copy; 256 orbitals, 256 walkers: Horner steps
+// 178 -> 76 us with both spins in one product, bias 204 -> 154 us).
+//
 // NP = 1 (one piece, 8 significant bits): the same two-piece tiles are staged
 // and only the hi words enter the MFMAs, h*h alone.
 #pragma once
@@ -389,74 +397,119 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
   const bool has_beta = (p.br != 0.0 || p.bi != 0.0);
   const int rbase = m0 + wm * WTM + 4 * g;
   const int cbase = n0 + wn * WTN + r;
+  long ccol[TN];  // output column offsets
 #pragma unroll
-  for (int i = 0; i < TM; i++) {
-    DT fr[TN][4], fi[TN][4], vr[TN][4], vi[TN][4];
-#pragma unroll
-    for (int j = 0; j < TN; j++)
-#pragma unroll
-      for (int q = 0; q < 4; q++) {
-        const int row = rbase + i * 16 + q, col = cbase + j * 16;
-        const bool in = row < p.m && col < p.n;
-        const long off = 2 * ((long)row * p.scm + (long)col * p.scn);
-        const long foff = (p.sfm || p.sfn) ? 2 * ((long)row * p.sfm + (long)col * p.sfn) : off;
-        const bool lf = (D || p.cf) && F && in;
-        fr[j][q] = lf ? F[foff] : (DT)0;
-        fi[j][q] = lf ? F[foff + 1] : (DT)0;
-        const bool lc = !OSPLIT && C && has_beta && in;
-        vr[j][q] = lc ? C[off] : (DT)0;
-        vi[j][q] = lc ? C[off + 1] : (DT)0;
-      }
-    // column-major split output (the Taylor steps' transposed terms): the
-    // lane's four rows are 32 contiguous bytes, stored as two 16-byte words
-    bool vec = false;
-    if constexpr (OSPLIT) vec = CS && !CS3 && !D && p.scm == 1 && rbase + i * 16 + 3 < p.m;
+  for (int j = 0; j < TN; j++) {
+    const int col = cbase + j * 16;
+    ccol[j] = p.cni ? (long)(col / p.cni) * p.scno + (long)(col % p.cni) * p.scn : (long)col * p.scn;
+  }
+  using CZ = typename ztype<DT>::type;  // element of C (not split), D and F
+  if constexpr (OSPLIT) {
+    // column-major split output (the propagator's transposed terms): a lane's
+    // four rows are contiguous, so F, D and C move as 16-byte words (two
+    // each, C3 one) where the columns keep them aligned
+    bool vec = CS && p.scm == 1 && !p.sfm && !p.sfn && (p.m & 3) == 0 && ((uintptr_t)CS & 15) == 0 &&
+               (!D || ((uintptr_t)D & 15) == 0) && (!F || ((uintptr_t)F & 15) == 0) &&
+               (!CS3 || ((uintptr_t)CS3 & 15) == 0) && ((p.cni ? (p.scno | p.scn) : p.scn) & 3) == 0;
     if (vec) {
 #pragma unroll
+      for (int i = 0; i < TM; i++) {
+        const int row = rbase + i * 16;
+        if (row >= p.m) continue;
+        const bool lf = (D || p.cf) && F;
+        float4 f0[TN], f1[TN];
+#pragma unroll
         for (int j = 0; j < TN; j++) {
-          const int col = cbase + j * 16;
-          if (col >= p.n) continue;
-          auto piece = [&](int q) __attribute__((always_inline)) -> zb {
-            const double re = (double)cr[i][j][q], im = (double)ci[i][j][q];
-            const double ore = p.ar * re - p.ai * im, oim = p.ar * im + p.ai * re;
-            const double f_r = (double)fr[j][q], f_i = (double)fi[j][q];
-            const double sr = p.cf ? f_r + ore : ore, si = p.cf ? f_i + oim : oim;
-            return split_z((float)sr, (float)si);
-          };
-          const zb v0 = piece(0), v1 = piece(1), v2 = piece(2), v3 = piece(3);
-          zb* dz = CS + (long)(rbase + i * 16) + (long)col * p.scn;
-          if (((uintptr_t)dz & 15) == 0) {
-            uint4* dst = (uint4*)dz;
-            dst[0] = make_uint4(v0.hi, v0.lo, v1.hi, v1.lo);
-            dst[1] = make_uint4(v2.hi, v2.lo, v3.hi, v3.lo);
-          } else {
-            dz[0] = v0;
-            dz[1] = v1;
-            dz[2] = v2;
-            dz[3] = v3;
+          f0[j] = f1[j] = make_float4(0.f, 0.f, 0.f, 0.f);
+          if (lf && cbase + j * 16 < p.n) {
+            const float4* fp = (const float4*)(F + 2 * (row + ccol[j]));
+            f0[j] = fp[0];
+            f1[j] = fp[1];
           }
         }
-    } else {
 #pragma unroll
-    for (int j = 0; j < TN; j++)
+        for (int j = 0; j < TN; j++) {
+          if (cbase + j * 16 >= p.n) continue;
+          const float fv[8] = {f0[j].x, f0[j].y, f0[j].z, f0[j].w, f1[j].x, f1[j].y, f1[j].z, f1[j].w};
+          zb h[4];
+          uint32_t t[4];
+          float dv[8];
+#pragma unroll
+          for (int q = 0; q < 4; q++) {
+            const double re = (double)cr[i][j][q], im = (double)ci[i][j][q];
+            const double ore = p.ar * re - p.ai * im, oim = p.ar * im + p.ai * re;  // alpha * AB
+            const double f_r = (double)fv[2 * q], f_i = (double)fv[2 * q + 1];
+            dv[2 * q] = (float)(f_r + ore);
+            dv[2 * q + 1] = (float)(f_i + oim);
+            const double sr = p.cf ? f_r + ore : ore, si = p.cf ? f_i + oim : oim;
+            if (CS3) split3_f((float)sr, (float)si, h[q], t[q]);
+            else h[q] = split_z((float)sr, (float)si);
+          }
+          uint4* dst = (uint4*)(CS + row + ccol[j]);
+          dst[0] = make_uint4(h[0].hi, h[0].lo, h[1].hi, h[1].lo);
+          dst[1] = make_uint4(h[2].hi, h[2].lo, h[3].hi, h[3].lo);
+          if (CS3) *(uint4*)(CS3 + row + ccol[j]) = make_uint4(t[0], t[1], t[2], t[3]);
+          if (D) {
+            float4* dd = (float4*)(D + 2 * (row + ccol[j]));
+            dd[0] = make_float4(dv[0], dv[1], dv[2], dv[3]);
+            dd[1] = make_float4(dv[4], dv[5], dv[6], dv[7]);
+          }
+        }
+      }
+      return;
+    }
+  }
+  if constexpr (!OSPLIT) {
+    if (C && !D && !has_beta && !(p.cf && F)) {  // C = alpha AB
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int q = 0; q < 4; q++) {
+          const int row = rbase + i * 16 + q;
+          if (row >= p.m) continue;
+          CZ* Cr = (CZ*)C + (long)row * p.scm;
+#pragma unroll
+          for (int j = 0; j < TN; j++) {
+            if (cbase + j * 16 >= p.n) continue;
+            const double re = (double)cr[i][j][q], im = (double)ci[i][j][q];
+            Cr[ccol[j]] = CZ{(DT)(p.ar * re - p.ai * im), (DT)(p.ar * im + p.ai * re)};
+          }
+        }
+      return;
+    }
+  }
+  // one block at a time, its F and C read before it is written
+#pragma unroll
+  for (int i = 0; i < TM; i++)
+#pragma unroll
+    for (int j = 0; j < TN; j++) {
+      const int col = cbase + j * 16;
+      if (col >= p.n) continue;
+      CZ fv[4], cv[4];
 #pragma unroll
       for (int q = 0; q < 4; q++) {
-        const int row = rbase + i * 16 + q, col = cbase + j * 16;
-        if (!(row < p.m && col < p.n)) continue;
+        const int row = rbase + i * 16 + q;
+        const long off = (long)row * p.scm + ccol[j];
+        const long foff = (p.sfm || p.sfn) ? (long)row * p.sfm + (long)col * p.sfn : off;
+        fv[q] = cv[q] = CZ{0, 0};
+        if ((D || p.cf) && F && row < p.m) fv[q] = ((const CZ*)F)[foff];
+        if (!OSPLIT && C && has_beta && row < p.m) cv[q] = ((const CZ*)C)[off];
+      }
+#pragma unroll
+      for (int q = 0; q < 4; q++) {
+        const int row = rbase + i * 16 + q;
+        if (row >= p.m) continue;
         const double re = (double)cr[i][j][q], im = (double)ci[i][j][q];
         const double ore = p.ar * re - p.ai * im, oim = p.ar * im + p.ai * re;  // alpha * AB
         double ocr = ore, oci = oim;                                             // + beta * C
         if (!OSPLIT && has_beta) {
-          const double cre = (double)vr[j][q], cim = (double)vi[j][q];
+          const double cre = (double)cv[q].re, cim = (double)cv[q].im;
           ocr += p.br * cre - p.bi * cim;
           oci += p.br * cim + p.bi * cre;
         }
-        const long off = 2 * ((long)row * p.scm + (long)col * p.scn);
-        const double f_r = (double)fr[j][q], f_i = (double)fi[j][q];
-        if (D) {
-          D[off] = (DT)(f_r + ore);
-          D[off + 1] = (DT)(f_i + oim);
-        }
+        const long off = (long)row * p.scm + ccol[j];
+        const double f_r = (double)fv[q].re, f_i = (double)fv[q].im;
+        if (D) ((CZ*)D)[off] = CZ{(DT)(f_r + ore), (DT)(f_i + oim)};
         if constexpr (OSPLIT) {
           if (CS) {
             const double sr = p.cf ? f_r + ore : ore, si = p.cf ? f_i + oim : oim;
@@ -464,17 +517,15 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
               zb h;
               uint32_t t;
               split3_f((float)sr, (float)si, h, t);
-              CS[off / 2] = h;
-              CS3[off / 2] = t;
+              CS[off] = h;
+              CS3[off] = t;
             } else {
-              CS[off / 2] = split_z((float)sr, (float)si);
+              CS[off] = split_z((float)sr, (float)si);
             }
           }
         } else if (C) {
-          C[off] = (DT)(p.cf ? ocr + f_r : ocr);
-          C[off + 1] = (DT)(p.cf ? oci + f_i : oci);
+          ((CZ*)C)[off] = CZ{(DT)(p.cf ? ocr + f_r : ocr), (DT)(p.cf ? oci + f_i : oci)};
         }
       }
     }
-  }
 }

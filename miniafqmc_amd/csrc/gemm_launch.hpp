@@ -25,6 +25,10 @@ constexpr RingCfg kRing[] = {
 constexpr RingCfg kRing3[] = {
     {128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {128, 128, 2, 2, 3}, {64, 64, 2, 2, 2}};
 constexpr int kNRing = 5;
+// relative rates with the chip full, by pieces: the HS potential, the bias
+// and the propagator products at 256 to 512 orbitals
+constexpr double kRingRate[] = {0.87, 1.0, 1.0, 1.02, 0.85};
+constexpr double kRingRate3[] = {0.95, 1.0, 1.0, 0.92, 0.93};
 
 // FP64 products (zgemm_f64_kernel): every operand order, tile candidates
 // (rows, complex columns, waves, LDS stages).

@@ -400,11 +400,11 @@ __global__ void third_piece_kernel(const zd* __restrict__ src, const zb* __restr
   }
 }
 
-// Batched transpose into three-piece split-BF16: in [b][R][C] (row stride C,
-// item stride R*C) -> out [b][C][R] (zb) and its third pieces out3, per
-// 32 x 32 tile through LDS; grid (C/32, R/32, b).
-template <class IT>
-__global__ __launch_bounds__(256) void transpose_split3_kernel(const IT* __restrict__ in, zb* __restrict__ out,
+// Batched transpose into split-BF16: in [b][R][C] (row stride C, item stride
+// R*C) -> out [b][C][R] (zb), with P3 as three pieces (the third ones to
+// out3), per 32 x 32 tile through LDS; grid (C/32, R/32, b).
+template <class IT, bool P3>
+__global__ __launch_bounds__(256) void transpose_split_kernel(const IT* __restrict__ in, zb* __restrict__ out,
                                                                uint32_t* __restrict__ out3, int R, int C)
 {
   __shared__ zd tile[32][33];
@@ -421,7 +421,8 @@ __global__ __launch_bounds__(256) void transpose_split3_kernel(const IT* __restr
     if (rr < R && cc < C) {
       const zd v = tile[tx][yy];
       const long o = item + (long)cc * R + rr;
-      split3_z(v.re, v.im, out[o], out3[o]);
+      if constexpr (P3) split3_z(v.re, v.im, out[o], out3[o]);
+      else out[o] = split_z((float)v.re, (float)v.im);
     }
   }
 }
