@@ -658,26 +658,23 @@ int gj_inverse_into(afqmc_ctx* c, zd* T, zd* Tinv, zd* det, long dq, long dr, in
   const int N = c->N;
   const long batch = 2L * c->nw;
   const long ms = (long)N * N;
-  if (N <= 16)
+  auto go = [&](auto rpl, auto nwv, auto cpw) {
+    constexpr int RPL = decltype(rpl)::value, NW = decltype(nwv)::value, CPW = decltype(cpw)::value;
     return launch(c, "gj_inverse", [&]() {
-      hipLaunchKernelGGL((gj_inverse_kernel<16, 8>), dim3(batch), dim3(128), 0, c->stream, T, Tinv, det, dq, dr, N, ms,
-                         flags, dc, ldet, lc);
+      hipLaunchKernelGGL((gj_inverse_kernel<RPL, NW, CPW>), dim3(batch), dim3(64 * NW), 0, c->stream, T, Tinv, det,
+                         dq, dr, N, ms, flags, dc, ldet, lc);
     });
-  if (N <= 32)
-    return launch(c, "gj_inverse", [&]() {
-      hipLaunchKernelGGL((gj_inverse_kernel<32, 8>), dim3(batch), dim3(256), 0, c->stream, T, Tinv, det, dq, dr, N, ms,
-                         flags, dc, ldet, lc);
-    });
-  if (N <= 64)
-    return launch(c, "gj_inverse", [&]() {
-      hipLaunchKernelGGL((gj_inverse_kernel<64, 8>), dim3(batch), dim3(512), 0, c->stream, T, Tinv, det, dq, dr, N, ms,
-                         flags, dc, ldet, lc);
-    });
-  if (N <= 128)
-    return launch(c, "gj_inverse", [&]() {
-      hipLaunchKernelGGL((gj_inverse_kernel<128, 8>), dim3(batch), dim3(1024), 0, c->stream, T, Tinv, det, dq, dr, N,
-                         ms, flags, dc, ldet, lc);
-    });
+  };
+  std::integral_constant<int, 1> i1;
+  std::integral_constant<int, 2> i2;
+  std::integral_constant<int, 4> i4;
+  std::integral_constant<int, 8> i8;
+  // one row per lane (two beyond 64), as many waves as the columns need
+  if (N <= 16) return go(i1, i4, i4);
+  if (N <= 32) return go(i1, i8, i4);
+  if (N <= 64) return go(i1, i8, i8);
+  if (N <= 96) return go(i2, std::integral_constant<int, 12>(), i8);
+  if (N <= 128) return go(i2, std::integral_constant<int, 16>(), i8);
   if (N <= GJ_GMAX) {
     // the working matrices do not fit one workgroup's registers: they stay
     // in global memory (allocated at the first call)

@@ -3,6 +3,8 @@
 #include "common.hpp"
 #include "fieldrng.hpp"
 
+#include <type_traits>
+
 // ---------------------------------------------------------------------------
 // Batched in-place Gauss-Jordan inverse + determinant of N x N complex
 // matrices, FP64.  Follows LAPACK's pivoting on the column-major view used by
@@ -13,12 +15,7 @@
 // the diagonal are those of the LU factorisation, so pivots and determinant
 // match getrf; the inverse equals getri's up to rounding.
 //
-// Thread (i, cg) of the NMAX*CG threads holds row i, columns cg + CG*t of X in
-// registers (NMAX/CG complex values).  Rows >= N are padded with the
-// identity.  Per elimination step: holders of column k publish |X(i,k)|, every
-// wave finds the pivot row p, rows p and k and column k go through LDS, and
-// each thread updates its own entries.  The signed pivots also give the
-// log-determinant (store_log_det).
+// The signed pivots also give the log-determinant (store_log_det).
 // batch b: input T + b*mstride; det written to det[(b/2)*dq + (b%2)*dr] and
 // to dcache[b] when dcache != null.
 // log det = sum_k log(pv_k), principal logs, imaginary part wrapped to
@@ -56,187 +53,272 @@ __device__ inline void store_log_det(const zd* pv, int N, bool singular, long b,
   }
 }
 
-// Wave argmax of (v, i) pairs, larger v first, then smaller i (an
-// associative, commutative choice, so any pairing order gives the same
-// pair): DPP moves within quads, half-rows and rows, then row broadcasts;
-// lane 63 holds the wave's pair, and i is returned in every lane.
-template <int CTRL, int RM> __device__ __forceinline__ void amx_step(double& bv, int& bi)
+// value of lane j (j the same in every lane) without going through LDS
+__device__ __forceinline__ double rdlane(double x, int j)
 {
-  const long long u = __double_as_longlong(bv);
-  const int lo = (int)u, hi = (int)(u >> 32);
-  const int olo = __builtin_amdgcn_update_dpp(lo, lo, CTRL, RM, 0xF, false);
-  const int ohi = __builtin_amdgcn_update_dpp(hi, hi, CTRL, RM, 0xF, false);
-  const int oi = __builtin_amdgcn_update_dpp(bi, bi, CTRL, RM, 0xF, false);
-  const double ov = __longlong_as_double((long long)(((unsigned long long)(unsigned)ohi << 32) | (unsigned)olo));
-  if (ov > bv || (ov == bv && oi < bi)) {
-    bv = ov;
-    bi = oi;
-  }
+  const long long v = __double_as_longlong(x);
+  const int lo = __builtin_amdgcn_readlane((int)(v & 0xffffffffLL), j);
+  const int hi = __builtin_amdgcn_readlane((int)(v >> 32), j);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
 }
-__device__ __forceinline__ int wave_argmax(double bv, int bi)
+__device__ __forceinline__ zd rdlane(zd x, int j) { return zd{rdlane(x.re, j), rdlane(x.im, j)}; }
+
+// Maximum of v over the wave, uniform: DPP moves within quads, half-rows and
+// rows, then row broadcasts (0 is the identity).
+template <int CTRL, int RM> __device__ __forceinline__ uint32_t umax_step(uint32_t v)
 {
-  amx_step<0xB1, 0xF>(bv, bi);   // quad_perm [1,0,3,2]
-  amx_step<0x4E, 0xF>(bv, bi);   // quad_perm [2,3,0,1]
-  amx_step<0x141, 0xF>(bv, bi);  // row_half_mirror
-  amx_step<0x140, 0xF>(bv, bi);  // row_mirror
-  amx_step<0x142, 0xA>(bv, bi);  // row_bcast15 into rows 1 and 3
-  amx_step<0x143, 0xC>(bv, bi);  // row_bcast31 into rows 2 and 3
-  return __builtin_amdgcn_readlane(bi, 63);
+  return max(v, (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, RM, 0xF, false));
+}
+__device__ __forceinline__ uint32_t wave_umax(uint32_t v)
+{
+  v = umax_step<0xB1, 0xF>(v);   // quad_perm [1,0,3,2]
+  v = umax_step<0x4E, 0xF>(v);   // quad_perm [2,3,0,1]
+  v = umax_step<0x141, 0xF>(v);  // row_half_mirror
+  v = umax_step<0x140, 0xF>(v);  // row_mirror
+  v = umax_step<0x142, 0xA>(v);  // row_bcast15 into rows 1 and 3
+  v = umax_step<0x143, 0xC>(v);  // row_bcast31 into rows 2 and 3
+  return (uint32_t)__builtin_amdgcn_readlane((int)v, 63);
 }
 
-template <int NMAX, int CG>
-__global__ __launch_bounds__(NMAX* CG) void gj_inverse_kernel(const zd* __restrict__ T, zd* __restrict__ Tinv,
-                                                               zd* __restrict__ det, long dq, long dr, int N,
-                                                               long mstride, int* __restrict__ info,
-                                                               zd* __restrict__ dcache, zd* __restrict__ ldet,
-                                                               zd* __restrict__ lcache)
+// 1 / b for a finite, nonzero b to about an ulp: b scaled by a power of two to
+// a largest component in [1/2, 1), |b|^2 inverted by the hardware's estimate
+// and two Newton steps (a third of the latency of two dependent divisions);
+// other b as zdiv gives it.
+__device__ __forceinline__ zd zrecip(zd b)
 {
-  constexpr int NC = NMAX / CG;
-  __shared__ double red[NMAX];
-  __shared__ zd prow[NMAX], oldk[NMAX], colk[NMAX], pv[NMAX];
-  __shared__ int perm[NMAX], dest[NMAX];
-  const int tid = threadIdx.x;
-  const int i = tid / CG, cg = tid % CG;
-  const int lane = tid & 63;
+  const int e = __builtin_amdgcn_frexp_exp(fmax(fabs(b.re), fabs(b.im)));
+  const double a = __builtin_amdgcn_ldexp(b.re, -e), c = __builtin_amdgcn_ldexp(b.im, -e);
+  const double d = fma(a, a, c * c);
+  if (!(d >= 0.25 && d <= 2.0)) return zdiv(zd{1.0, 0.0}, b);
+  double y = __builtin_amdgcn_rcp(d);
+  y = fma(y, fma(-d, y, 1.0), y);
+  y = fma(y, fma(-d, y, 1.0), y);
+  return zd{__builtin_amdgcn_ldexp(a * y, -e), __builtin_amdgcn_ldexp(-c * y, -e)};
+}
+
+// One workgroup per matrix.  Lane l holds row l (RPL = 2: rows l and l + 64) at
+// the CPW columns of its wave, column j = wave * CPW + c in register slot c, so
+// a step touches registers statically and a row never leaves its lane.  Rows
+// are not swapped: pos is the position LAPACK's interchanges would have
+// brought the row to, and a row is a pivot candidate while pos >= k.  A pivot
+// row is not scaled when it is chosen but once at the end (it is no candidate
+// any more, and the other rows' multipliers hold the reciprocal), so a step is
+// x += multiplier * pivot row in every lane, with multiplier 0 in the pivot
+// row's, and only column k's slot is set apart.
+//
+// Step k: the wave that owns column k finds the pivot row p (wave maximum of
+// |Re| + |Im|, the lowest position among equals), the pivot's reciprocal and
+// the multipliers -X(i,k)/piv of all rows and leaves them in LDS (two buffers
+// by step parity); after a barrier every wave takes row p's entries of its own
+// columns by readlane and updates its rows.  The owner of column k + 1 updates
+// that column first and searches it before its other columns, so one barrier
+// and one search chain bound a step.
+//
+// Bound: that chain (key maximum, reciprocal, LDS round trip, barrier: 0.5 to
+// 0.7 us a step with nothing else to do), and from 64 electrons on the
+// readlanes and FP64 FMAs of four waves per SIMD (0.9 us a step at 128), which
+// the owner's own columns keep from overlapping fully.  Measured (MI355X, us
+// per batch; before: the matrix split over the rows' threads, two barriers per
+// step, the pivot row read from LDS by all, a serial unscrambling of the
+// interchanges): 2048 x N = 128 3070 -> 1930, 512 x 96 541 -> 319, 512 x 64
+// 150 -> 90, 192 x 32 48 -> 29, 32 x 16 23 -> 17.  With the search, the
+// reciprocal and all updates but the searched column's taken out, 128 x N = 128
+// went from 230 to 93 us.
+template <int RPL, int NW, int CPW>
+__global__ __launch_bounds__(64 * NW) void gj_inverse_kernel(const zd* __restrict__ T, zd* __restrict__ Tinv,
+                                                             zd* __restrict__ det, long dq, long dr, int N,
+                                                             long mstride, int* __restrict__ info,
+                                                             zd* __restrict__ dcache, zd* __restrict__ ldet,
+                                                             zd* __restrict__ lcache)
+{
+  constexpr int NMAX = NW * CPW;  // columns
+  static_assert(CPW % 2 == 0, "buffers alternate by slot parity");
+  __shared__ zd gqs[2][64 * RPL];  // multipliers by row
+  __shared__ zd ipvs[2], pv[NMAX];
+  __shared__ int ctl[2];   // pivot row, or -1 when the pivot is zero
+  __shared__ int prow[NMAX];
+  const int tid = threadIdx.x, lane = tid & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const long b = blockIdx.x;
   const zd* Tb = T + b * mstride;
-  zd x[NC];
+  const int j0 = wave * CPW;
+  zd x[RPL][CPW];
+  int pos[RPL];
+  zd scale[RPL];  // reciprocal of the row's pivot
 #pragma unroll
-  for (int t = 0; t < NC; t++) {
-    int j = cg + CG * t;
-    if (i < N && j < N) x[t] = Tb[(long)j * N + i];  // X = T^T
-    else x[t] = zd{(i == j) ? 1.0 : 0.0, 0.0};
+  for (int q = 0; q < RPL; q++) {
+    const int i = lane + 64 * q;
+    pos[q] = i < N ? i : 0x7fffffff;
+    scale[q] = zd{1.0, 0.0};
+#pragma unroll
+    for (int c = 0; c < CPW; c++)
+      x[q][c] = (i < N && j0 + c < N) ? Tb[(long)(j0 + c) * N + i] : zd{0.0, 0.0};  // X = T^T
   }
-  zd dt{1.0, 0.0};
-  bool singular = false;
-  // Columns are eliminated in blocks of CG: block tk holds columns CG*tk ..
-  // CG*tk + CG - 1, one per thread of a row, all in register slot tk.  For the
-  // CG steps of a block that slot is moved to xc, a register addressed
-  // statically, so only xc needs the column-k special case; the other slots
-  // take the plain update (slot tk's copy is refreshed from xc at the end).
-  const int nblk = (N + CG - 1) / CG;
-  for (int tk = 0; tk < nblk && !singular; tk++) {
-    zd xc{0, 0};
+  // search column k (slot c of this wave) and publish the step
+  auto publish = [&](int k, auto cc) __attribute__((always_inline)) {
+    constexpr int c = decltype(cc)::value, st = c & 1;
+    // keys: the high word of |Re| + |Im| plus 1 (nonnegative doubles order as
+    // their bits), 0 for rows that are no candidates and for NaN; the low
+    // words decide among equal high words, then the position
+    uint32_t hi[RPL], lo[RPL], m = 0;
 #pragma unroll
-    for (int t = 0; t < NC; t++)
-      if (t == tk) xc = x[t];
-    const int jc = cg + CG * tk;  // the column xc holds
+    for (int q = 0; q < RPL; q++) {
+      const double v = zcabs1(x[q][c]);
+      const unsigned long long u = (unsigned long long)__double_as_longlong(v);
+      hi[q] = (pos[q] >= k && pos[q] < N && v == v) ? (uint32_t)(u >> 32) + 1u : 0u;
+      lo[q] = (uint32_t)u;
+      m = max(m, hi[q]);
+    }
+    m = wave_umax(m);
+    unsigned long long cand[RPL];
+    int n = 0;
 #pragma unroll
-    for (int ck = 0; ck < CG; ck++) {
-      const int k = CG * tk + ck;
-      if (k >= N) break;
-      const bool own = (cg == ck);  // xc holds column k
-      if (own) {
-        red[i] = (i >= k) ? zcabs1(xc) : -1.0;
-        colk[i] = xc;
-      }
-      __syncthreads();
-      double bv = -2.0;
-      int bi = 0;
+    for (int q = 0; q < RPL; q++) {
+      // no candidate compares (all NaN): the row at position k
+      cand[q] = m ? __ballot(hi[q] == m) : __ballot(pos[q] == k);
+      n += __popcll(cand[q]);
+    }
+    if (n > 1) {
+      uint32_t ml = 0;
 #pragma unroll
-      for (int q = lane; q < NMAX; q += 64) {
-        double v = red[q];
-        if (v > bv) { bv = v; bi = q; }
-      }
-      const int p = wave_argmax(bv, bi);
-      if (i == p) {
+      for (int q = 0; q < RPL; q++)
+        if (hi[q] == m) ml = max(ml, lo[q]);
+      ml = wave_umax(ml);
+      n = 0;
 #pragma unroll
-        for (int t = 0; t < NC; t++) prow[cg + CG * t] = x[t];
-        prow[jc] = xc;  // after slot tk's stale copy: the later store wins
-        if (own) pv[k] = (p != k) ? zd{-xc.re, -xc.im} : xc;  // signed pivot
-      }
-      if (i == k && p != k) {
-#pragma unroll
-        for (int t = 0; t < NC; t++) oldk[cg + CG * t] = x[t];
-        oldk[jc] = xc;
-      }
-      if (tid == 0) perm[k] = p;
-      __syncthreads();
-      const zd piv = prow[k];
-      if (piv.re == 0.0 && piv.im == 0.0) {
-        singular = true;
-        dt = zd{0.0, 0.0};
-        break;
-      }
-      dt = zmul(dt, (p != k) ? zd{-piv.re, -piv.im} : piv);
-      const zd ipv = zdiv(zd{1.0, 0.0}, piv);
-      if (i == k) {
-        // new row k = pivot row / piv; column k holds 1/piv
-#pragma unroll
-        for (int t = 0; t < NC; t++) x[t] = zmul(prow[cg + CG * t], ipv);
-        xc = own ? ipv : zmul(prow[jc], ipv);
-      } else {
-        const bool swapped_in = (i == p);  // p != k here since i != k
-        if (swapped_in) {
-#pragma unroll
-          for (int t = 0; t < NC; t++) x[t] = oldk[cg + CG * t];
-          xc = oldk[jc];
-        }
-        // X(i,k) of the row now at i: the swapped-in row takes old row k's,
-        // from oldk (written between this step's barriers), not colk[k],
-        // which row k's owner overwrites at the start of the next step with
-        // no barrier in between (row k may sit in another wave)
-        const zd f = swapped_in ? oldk[k] : colk[i];
-        const zd gq = zmul(zd{-f.re, -f.im}, ipv);  // -X(i,k)/piv
-#pragma unroll
-        for (int t = 0; t < NC; t++) {
-          const zd pr = prow[cg + CG * t];
-          const double xr = x[t].re, xi = x[t].im;
-          x[t].re = xr + gq.re * pr.re - gq.im * pr.im;
-          x[t].im = xi + gq.re * pr.im + gq.im * pr.re;
-        }
-        // column k: X(i,k) = -X(i,k)/piv, i.e. 0 + gq * 1
-        const zd pc = prow[jc];
-        const double xr = own ? 0.0 : xc.re, xi = own ? 0.0 : xc.im;
-        const double pr_r = own ? 1.0 : pc.re, pr_i = own ? 0.0 : pc.im;
-        xc.re = xr + gq.re * pr_r - gq.im * pr_i;
-        xc.im = xi + gq.re * pr_i + gq.im * pr_r;
+      for (int q = 0; q < RPL; q++) {
+        cand[q] = __ballot(hi[q] == m && lo[q] == ml);
+        n += __popcll(cand[q]);
       }
     }
+    int p = -1;
+    if (n == 1) {
 #pragma unroll
-    for (int t = 0; t < NC; t++)
-      if (t == tk) x[t] = xc;
+      for (int q = 0; q < RPL; q++)
+        if (cand[q]) p = (__ffsll((long long)cand[q]) - 1) + 64 * q;
+    } else {
+      int best = 0x7fffffff;
+#pragma unroll
+      for (int q = 0; q < RPL; q++)
+        for (unsigned long long s = cand[q]; s; s &= s - 1) {
+          const int l = __ffsll((long long)s) - 1;
+          const int ps = __builtin_amdgcn_readlane(pos[q], l);
+          if (ps < best) {
+            best = ps;
+            p = l + 64 * q;
+          }
+        }
+    }
+    zd piv = rdlane(x[0][c], p & 63);
+    int pp = __builtin_amdgcn_readlane(pos[0], p & 63);
+    if constexpr (RPL == 2) {
+      if (p >= 64) {
+        piv = rdlane(x[1][c], p - 64);
+        pp = __builtin_amdgcn_readlane(pos[1], p - 64);
+      }
+    }
+    const bool zero = piv.re == 0.0 && piv.im == 0.0;
+    const zd ipv = zrecip(piv);
+#pragma unroll
+    for (int q = 0; q < RPL; q++)
+      gqs[st][lane + 64 * q] = lane + 64 * q == p ? zd{0.0, 0.0} : zmul(zd{-x[q][c].re, -x[q][c].im}, ipv);
+    if (lane == 0) {
+      ctl[st] = zero ? -1 : p;
+      ipvs[st] = ipv;
+      prow[k] = p;
+      pv[k] = pp != k ? zd{-piv.re, -piv.im} : piv;  // signed pivot
+    }
+  };
+  if (wave == 0) publish(0, std::integral_constant<int, 0>());
+  __syncthreads();
+  zd dt{1.0, 0.0};
+  bool singular = false;
+  const int nblk = (N + CPW - 1) / CPW;
+  for (int kb = 0; kb < nblk && !singular; kb++) {
+    // wave kb owns the block's columns
+    auto step = [&](auto cc) __attribute__((always_inline)) {
+      constexpr int c = decltype(cc)::value, st = c & 1, c1 = (c + 1) % CPW;
+      const int k = kb * CPW + c;
+      if (k >= N || singular) return;
+      const int pl = ctl[st];
+      const zd ipv = ipvs[st], spv = pv[k];
+      zd gq[RPL];
+#pragma unroll
+      for (int q = 0; q < RPL; q++) gq[q] = gqs[st][lane + 64 * q];
+      const int p = __builtin_amdgcn_readfirstlane(pl);
+      if (p < 0) {
+        singular = true;
+        dt = zd{0.0, 0.0};
+        return;
+      }
+      // positions: the pivot row to k, the row there to the pivot's
+      int pp = __builtin_amdgcn_readlane(pos[0], p & 63);
+      if constexpr (RPL == 2)
+        if (p >= 64) pp = __builtin_amdgcn_readlane(pos[1], p - 64);
+#pragma unroll
+      for (int q = 0; q < RPL; q++) {
+        const bool mine = lane + 64 * q == p;
+        pos[q] = mine ? k : (pos[q] == k ? pp : pos[q]);
+        if (mine) scale[q] = ipv;
+      }
+      auto update = [&](int s, bool colk) __attribute__((always_inline)) {
+        // row p's entry of the slot
+        zd pr;
+        if constexpr (RPL == 2) pr = p >= 64 ? rdlane(x[1][s], p - 64) : rdlane(x[0][s], p);
+        else pr = rdlane(x[0][s], p);
+#pragma unroll
+        for (int q = 0; q < RPL; q++) {
+          const double xr = x[q][s].re, xi = x[q][s].im;
+          x[q][s].re = xr + gq[q].re * pr.re - gq[q].im * pr.im;
+          x[q][s].im = xi + gq[q].re * pr.im + gq[q].im * pr.re;
+          if (colk) x[q][s] = lane + 64 * q == p ? zd{1.0, 0.0} : gq[q];
+        }
+        __builtin_amdgcn_sched_barrier(0);  // one slot at a time: bounds the live registers
+      };
+      const int k1 = k + 1;
+      // the search chain ahead of the other waves' updates
+      if (wave == k1 / CPW) __builtin_amdgcn_s_setprio(3);
+      update(c1, false);
+      if (k1 < N && wave == k1 / CPW) publish(k1, std::integral_constant<int, c1>());
+      __builtin_amdgcn_s_setprio(0);
+#pragma unroll
+      for (int s = 0; s < CPW; s++)
+        if (s != c1) update(s, s == c && wave == kb);
+      if (wave == 0) dt = zmul(dt, spv);
+      __syncthreads();
+    };
+    step(std::integral_constant<int, 0>());
+    step(std::integral_constant<int, 1>());
+    if constexpr (CPW > 2) {
+      step(std::integral_constant<int, 2>());
+      step(std::integral_constant<int, 3>());
+    }
+    if constexpr (CPW > 4) {
+      step(std::integral_constant<int, 4>());
+      step(std::integral_constant<int, 5>());
+      step(std::integral_constant<int, 6>());
+      step(std::integral_constant<int, 7>());
+    }
   }
   if (tid == 0) {
     if (singular && info) atomicAdd(info, 1);
     det[(b / 2) * dq + (b % 2) * dr] = dt;
     if (dcache) dcache[b] = dt;
   }
-  // the log-determinant last, when the matrix no longer occupies registers
-  if (!Tinv) {
-    store_log_det(pv, N, singular, b, ldet, lcache);
-    return;
-  }
-  if (singular) {
-    // leave a defined value: zeros
-    __syncthreads();
+  if (Tinv) {
+    // with the rows in LAPACK's positions the result would be the inverse of
+    // the interchanged matrix: its column k belongs to the row p chosen at
+    // step k, so T^-1[p_j][pos_i] = X(i, j)
 #pragma unroll
-    for (int t = 0; t < NC; t++) {
-      int j = cg + CG * t;
-      if (i < N && j < N) Tinv[b * mstride + (long)j * N + i] = zd{0, 0};
-    }
-    store_log_det(pv, N, singular, b, ldet, lcache);
-    return;
-  }
-  // undo the row interchanges as column interchanges in reverse order
-  __syncthreads();
-  if (tid == 0) {
-    for (int c = 0; c < N; c++) dest[c] = c;  // dest used as colmap first
-    for (int k = N - 1; k >= 0; k--) {
-      int pk = perm[k];
-      int tmp = dest[k];
-      dest[k] = dest[pk];
-      dest[pk] = tmp;
-    }
-    for (int c = 0; c < N; c++) perm[dest[c]] = c;  // perm now = inverse map
-  }
-  __syncthreads();
-  // Z(:, c) = Y(:, colmap[c]) -> Y column j goes to column perm[j];
-  // T^-1[a][b] = Z[b][a]
+    for (int q = 0; q < RPL; q++)
 #pragma unroll
-  for (int t = 0; t < NC; t++) {
-    int j = cg + CG * t;
-    if (i < N && j < N) Tinv[b * mstride + (long)perm[j] * N + i] = x[t];
+      for (int c = 0; c < CPW; c++) {
+        const int i = lane + 64 * q, j = j0 + c;
+        if (i < N && j < N) {
+          if (singular) Tinv[b * mstride + (long)j * N + i] = zd{0, 0};  // a defined value
+          else Tinv[b * mstride + (long)prow[j] * N + pos[q]] = zmul(x[q][c], scale[q]);
+        }
+      }
   }
   store_log_det(pv, N, singular, b, ldet, lcache);
 }

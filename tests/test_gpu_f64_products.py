@@ -98,3 +98,51 @@ def test_exchange_in_one_launch_vs_cholesky_form(require_gpu, mode, level, tol, 
     ref = ex.pop()
     for e in ex:
         assert np.abs(e - ref).max() <= tol * np.abs(ref).max()
+
+
+@pytest.mark.parametrize("N", [1, 2, 4, 5, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128])
+def test_batched_inverse_pivots(require_gpu, N):
+    """Overlap matrices with prescribed pivot choices (the trial is the first N
+    unit vectors, so a walker's top block is its overlap matrix): Gaussian
+    entries, rows in reverse order (an interchange at every step), entries of
+    exactly equal size (LAPACK takes the first), sizes 1e-200 and 1e200; inverse
+    and determinant against numpy."""
+    say("batched inverse", N)
+    M = N + 3
+    r = np.random.default_rng(N)
+
+    def cn(*shape):
+        return r.standard_normal(shape) + 1j * r.standard_normal(shape)
+
+    T = [cn(N, N), cn(N, N)[::-1] + 8 * np.eye(N)[::-1], 1e-200 * cn(N, N), 1e200 * cn(N, N)]
+    h = np.array([[1.0]])
+    while h.shape[0] < N:
+        h = np.block([[h, h], [h, -h]])
+    T.append((h[:N, :N] + 1j * np.tril(h[:N, :N])) if N > 1 else np.array([[1 + 1j]]))
+    s = m.make_system(M, N, 2, density=1.0, sigma_L=0.01, sigma_h=1.0, dt=0.005, seed=N)
+    s.trial_alpha[:] = np.eye(M, N)
+    s.trial_beta[:] = np.eye(M, N)
+    nw = len(T)
+    W = np.zeros((nw, 2, M, N), complex)
+    for w in range(nw):
+        W[w, 0, :N] = T[w].T  # T1[a][b] = W[b][a]
+        W[w, 1, :N] = cn(N, N) + 3 * np.eye(N)
+    W[:, :, N:] = 0.1
+    g = m.AfqmcSys(s, nw, "fp64_dense", dense_exchange=False)
+    g.set(nat.BUF_W, W)
+    g.set(nat.BUF_WDATA, np.zeros((nw, 8), complex))
+    G = g.calculate_mixed_density_matrix().reshape(2, N, M, nw)
+    ov = g.W_data[:, 2:4]
+    g.close()
+    for w in range(nw):
+        for sp in range(2):
+            A = W[w, sp, :N].T
+            sign, logd = np.linalg.slogdet(A / np.abs(A).max())
+            logd += N * np.log(np.abs(A).max())
+            inv = np.linalg.inv(A / np.abs(A).max()) / np.abs(A).max()
+            cond = np.linalg.cond(A / np.abs(A).max())
+            ref = inv @ W[w, sp].T
+            assert np.abs(G[sp, :, :, w] - ref).max() <= 1e-14 * N * cond * np.abs(ref).max()
+            if abs(logd) < 600:
+                det = sign * np.exp(logd)
+                assert abs(ov[w, sp] - det) <= 1e-13 * N * cond * abs(det)
