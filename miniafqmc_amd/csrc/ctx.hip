@@ -1871,10 +1871,14 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
         RET((zgemm<CP, LT_, GT, YT, true, true>(c, "energy_y_gemm", a, 2 * nw)));
       }
     }
+    // partials per walker-spin: enough workgroups for eight per CU
+    const int ngrp = (int)std::max<long>(1, std::min<long>(cnt, 2048 / (2L * nw)));
+    RET(need_vws(c, sizeof(zd) * (size_t)ngrp * 2 * nw));
     RET(launch(c, "energy_trace", [&]() {
-      hipLaunchKernelGGL((trace_sq_kernel<typename ztype<YT>::type>), dim3(2 * nw), dim3(256), 0, c->stream,
-                         (const typename ztype<YT>::type*)c->Ybuf, N, cnt, (long)cnt * per_item, c->e_exch_part, 1L,
-                         2 * nw);
+      hipLaunchKernelGGL((trace_sq_kernel<typename ztype<YT>::type>), dim3(2 * nw, ngrp), dim3(256), 0, c->stream,
+                         (const typename ztype<YT>::type*)c->Ybuf, N, cnt, (long)cnt * per_item, (zd*)c->vws, ngrp);
+      hipLaunchKernelGGL(add_parts_kernel, dim3((2 * nw + 255) / 256), dim3(256), 0, c->stream, (const zd*)c->vws,
+                         ngrp, c->e_exch_part, 2 * nw);
     }));
   }
   }

@@ -100,7 +100,7 @@ def test_exchange_in_one_launch_vs_cholesky_form(require_gpu, mode, level, tol, 
         assert np.abs(e - ref).max() <= tol * np.abs(ref).max()
 
 
-@pytest.mark.parametrize("N", [1, 2, 4, 5, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128])
+@pytest.mark.parametrize("N", [1, 2, 4, 5, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 256])
 def test_batched_inverse_pivots(require_gpu, N):
     """Overlap matrices with prescribed pivot choices (the trial is the first N
     unit vectors, so a walker's top block is its overlap matrix): Gaussian
