@@ -36,8 +36,8 @@ REFERENCE_TIMERS = (
     ("Overlap", ("ovlp_gemm", "gj_inverse")),
     ("Orthgonalization", ("ortho_gram", "ortho_chol_inv", "ortho_sign", "ortho_apply", "ortho_flags",
                           "lq_orthogonalize", "lq_fallback")),
-    ("Local Energy", ("energy_one", "energy_two", "energy_direct", "energy_exch_dot", "energy_pairsum",
-                      "energy_assemble", "energy_zero", "energy_trace", "energy_v_gemm", "energy_v_reduce", "energy_vx_gemm",
+    ("Local Energy", ("energy_exch_dot", "energy_assemble",
+                      "energy_zero", "energy_trace", "energy_v_gemm", "energy_v_reduce", "energy_vx_gemm",
                       "energy_y_gemm", "csrmm_vakbl", "g_transpose", "gc64_gemm", "convert", "g_split", "g_split3")),
 )
 

@@ -40,6 +40,7 @@ struct KStat {
 struct EvPair {
   std::string name;
   hipEvent_t a, b;
+  int count;
 };
 
 } // namespace
@@ -167,6 +168,8 @@ struct afqmc_ctx {
   bool allow_vx = true;
   zd* Gtmp = nullptr;     // FP64 G [nw][2NM] for the energy (CSR: transposed; mixed: FP64 copy)
   void* vws = nullptr;    // split-k partials of the bias contraction
+  int vws_pending = 0;    // slices there that the next fields kernel sums into vbias
+  double* xtmp = nullptr; // draws passed to afqmc_fields, [K][nw] (allocated at the first such call)
   size_t vws_bytes = 0;
   // orthogonalisation: Cholesky QR scratch (allocated at the first call)
   bool ortho_householder = false;  // always use the blocked Householder kernel
@@ -285,7 +288,9 @@ const Roctx& roctx()
   return r;
 }
 
-template <class F> int launch(afqmc_ctx* c, const char* name, F&& f)
+// count: what the statistics count it as (a kernel that runs several products
+// of the call-by-call form counts each).
+template <class F> int launch(afqmc_ctx* c, const char* name, F&& f, int count = 1)
 {
   const Roctx& rx = roctx();
   if (rx.push) rx.push(c->tuning ? (std::string("tune/") + name).c_str() : name);
@@ -307,7 +312,7 @@ template <class F> int launch(afqmc_ctx* c, const char* name, F&& f)
   if (e != hipSuccess) return fail(c, AFQMC_ERR_HIP, std::string(name) + ": " + hipGetErrorString(e));
   if (c->prof) {
     (void)hipEventRecord(b, c->stream);
-    c->pending.push_back({name, a, b});
+    c->pending.push_back({name, a, b, count});
   }
   return AFQMC_OK;
 }
@@ -320,7 +325,7 @@ void collect_events(afqmc_ctx* c)
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, p.a, p.b);
     auto& s = c->stats[p.name];
-    s.n++;
+    s.n += p.count;
     s.ms += ms;
     c->evpool.push_back(p.a);
     c->evpool.push_back(p.b);
@@ -778,15 +783,18 @@ int g_fp64(afqmc_ctx* c)
 }
 
 // ---------------------------------------------------------------------------
-int do_mdm(afqmc_ctx* c)
+// restore: W_data's overlaps from the last inverse when it is reused (a substep
+// leaves that to its fields kernel)
+int do_mdm(afqmc_ctx* c, bool restore = true)
 {
   const int M = c->M, N = c->N, nw = c->nw;
   if (c->t1inv_valid) {
     // the overlap step already inverted W^T conj(Psi) for these walkers
-    RET(launch(c, "det_restore", [&]() {
-      hipLaunchKernelGGL(det_restore_kernel, dim3((2 * nw + 255) / 256), dim3(256), 0, c->stream, c->Wd, c->dcache,
-                         c->Wl, c->lcache, nw);
-    }));
+    if (restore)
+      RET(launch(c, "det_restore", [&]() {
+        hipLaunchKernelGGL(det_restore_kernel, dim3((2 * nw + 255) / 256), dim3(256), 0, c->stream, c->Wd, c->dcache,
+                           c->Wl, c->lcache, nw);
+      }));
   } else {
     RET(overlap_matrices(c));
     RET(gj_inverse(c, c->T1, c->T1, c->Wd + 2, 8, 1));
@@ -854,7 +862,8 @@ long f64_chunk(long m, long n, long kt, int items, int smax)
 // products (spin, chunk of j) run as one batch into a workspace, summed in
 // chunk order.  (200 walkers, 999 vectors, N M = 15250: 12.6 ms unsplit in
 // 32 workgroups per spin.)
-int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const char* name, const char* rname)
+int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const char* name, const char* rname,
+                       bool defer)
 {
   const long NM = (long)c->N * c->M, nw = c->nw, K = c->K;
   const long chunk = f64_chunk(nw, K, NM, 2, 16);
@@ -879,6 +888,10 @@ int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const c
   a.sc2 = nw * K;
   a.bdiv = S;
   RET(zgemm64<zd>(c, name, a, 2 * S));
+  if (defer) {
+    c->vws_pending = 2 * S;
+    return AFQMC_OK;
+  }
   return launch(c, rname, [&]() {
     hipLaunchKernelGGL((zsum_slices_kernel<zd>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const zd*)c->vws,
                        out, nw * K, 2 * S);
@@ -892,11 +905,11 @@ int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const c
 template <int CP, class GT, class LT_>
 int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, const char* name,
                          const uint32_t* G3 = nullptr, const uint32_t* Lt3 = nullptr,
-                         const char* rname = "vbias_reduce")
+                         const char* rname = "vbias_reduce", bool defer = false)
 {
   const long NM = (long)c->N * c->M, nw = c->nw, K = c->K;
   if constexpr (CP == CP_F64) {
-    if (NM >= 512) return dense_contract_f64(c, (const zd*)Gp, (const zd*)Lt, out, name, rname);
+    if (NM >= 512) return dense_contract_f64(c, (const zd*)Gp, (const zd*)Lt, out, name, rname, defer);
   }
   const long tiles = ((nw + 127) / 128) * ((K + 63) / 64);
   int S = 1;
@@ -953,6 +966,10 @@ int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, 
   a.A3 = G3;  // third pieces with the same offsets
   a.B3 = Lt3;
   RET((zgemm<CP, GT, LT_, PT, true, true>(c, name, a, 2 * S)));
+  if (defer) {
+    c->vws_pending = 2 * S;
+    return AFQMC_OK;
+  }
   return launch(c, rname, [&]() {
     hipLaunchKernelGGL((zsum_slices_kernel<PZ>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const PZ*)c->vws, out,
                        nw * K, 2 * S);
@@ -962,12 +979,12 @@ int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, 
 // afqmc_sys::calculate_mixed_density_matrix(W, W_data, G, false)
 // (mixed_density_matrix.hpp:93-101): G_s = conj(A_s) Gc_s per walker and
 // spin, [2*M*M][nw] walker-last.  FP64_CSR mode.
-int do_mdm_full(afqmc_ctx* c)
+int do_mdm_full(afqmc_ctx* c, bool restore = true)
 {
   const int M = c->M, N = c->N, nw = c->nw;
   const long MM = (long)M * M, MN = (long)M * N;
   if (!c->Gfull) RET(dalloc(c, &c->Gfull, 2 * MM * nw));
-  RET(do_mdm(c));
+  RET(do_mdm(c, restore));
   // columns (k, w) of one spin side by side: one M x M*nw product per spin
   F64Args a = f64args(M, M * nw, N);
   a.A = c->trial;  // A(i, a) = trialwfn_s[i][a]
@@ -1002,7 +1019,7 @@ int do_vbias_full(afqmc_ctx* c)
 // FP64_CSR bias product with SpvnT kept dense: vbias[K][nw] = SpvnT[K][2NM] G
 // on FP64 MFMA, the long sum split into S chunks (a batched GEMM into a
 // workspace, then summed in FP64 in chunk order).
-int dense_csr_vbias(afqmc_ctx* c)
+int dense_csr_vbias(afqmc_ctx* c, bool defer)
 {
   const long NAK = 2L * c->N * c->M, nw = c->nw, K = c->K;
   const long chunk = f64_chunk(K, nw, NAK, 1, 32);
@@ -1034,52 +1051,67 @@ int dense_csr_vbias(afqmc_ctx* c)
   a.C = c->vws;
   a.sc2 = K * nw;
   RET(zgemm64<zd>(c, "vbias_gemm", a, S));
+  if (defer) {
+    c->vws_pending = S;
+    return AFQMC_OK;
+  }
   return launch(c, "vbias_reduce", [&]() {
     hipLaunchKernelGGL((zsum_slices_kernel<zd>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const zd*)c->vws,
                        c->vbias, nw * K, S);
   });
 }
 
-int do_vbias(afqmc_ctx* c)
+// defer: the partial products of a split contraction stay in the workspace for
+// the fields kernel that follows (vws_pending)
+int do_vbias(afqmc_ctx* c, bool defer = false)
 {
   const int nw = c->nw, K = c->K, NAK = 2 * c->N * c->M;
+  const char* rn = "vbias_reduce";
   if (c->mode == AFQMC_FP64_CSR) {
-    if (c->sptd) return dense_csr_vbias(c);
+    if (c->sptd) return dense_csr_vbias(c, defer);
     zd one{1, 0}, zero{0, 0};
     return csrmm_n(c, "csrmm_vbias", K, NAK, c->spt_nnz, c->spt_rp, c->spt_col, c->spt_val, (const zd*)c->G,
                    (long)nw, c->vbias, (long)nw, one, zero, true);
   }
   if (c->mode == AFQMC_FP64_DENSE)
-    return dense_contract_vbias<CP_F64, double, double>(c, c->G, c->Lt, c->vbias, "vbias_gemm");
+    return dense_contract_vbias<CP_F64, double, double>(c, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
+                                                        defer);
   if (c->mode == AFQMC_MIXED_FP32)
-    return dense_contract_vbias<CP_F32, float, float>(c, c->G, c->Lt, c->vbias, "vbias_gemm");
+    return dense_contract_vbias<CP_F32, float, float>(c, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
+                                                      defer);
   if (c->three & 1)
-    return dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, c->G, c->Lt, c->vbias, "vbias_gemm", c->tp_G, c->tp_Lt);
-  return dense_contract_vbias<CP_BF16X3, bfs, bfs>(c, c->G, c->Lt, c->vbias, "vbias_gemm");
+    return dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, c->G, c->Lt, c->vbias, "vbias_gemm", c->tp_G, c->tp_Lt, rn,
+                                                     defer);
+  return dense_contract_vbias<CP_BF16X3, bfs, bfs>(c, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
+                                                   defer);
 }
 
 // Draws of the fields phase: xdev (a device block [K][nw]; with xslice !=
 // null the staged block and *xslice its substep index) or, when xdev is null,
 // generated on the device from (field_seed, substep or *xslice, walker).
-int do_fields(afqmc_ctx* c, const double* xdev, long substep, const long* xslice = nullptr)
+// pre: what the substep leaves to this kernel.
+int do_fields(afqmc_ctx* c, const double* xdev, long substep, const long* xslice = nullptr, FieldPre pre = FieldPre{})
 {
   const int nw = c->nw, K = c->K;
   FieldSrc src{xdev, xslice, substep, c->field_seed};
+  pre.slices = c->vws;
+  pre.ns = c->vws_pending;
+  c->vws_pending = 0;
   if (c->mode == AFQMC_FP64_CSR)
     return launch(c, "fields", [&]() {
-      hipLaunchKernelGGL((fields_wlast_kernel<zd>), dim3((nw + 63) / 64), dim3(1024), 0, c->stream, K, nw, c->vbias,
-                         src, (zd*)c->X, c->hybridW, c->flags + 1);
+      hipLaunchKernelGGL((fields_wlast_kernel<zd>), dim3((nw + 15) / 16), dim3(1024), 0, c->stream, K, nw, c->vbias,
+                         src, (zd*)c->X, c->hybridW, c->flags + 1, pre);
     });
   return launch(c, "fields", [&]() {
     if (!c->mixed)
-      hipLaunchKernelGGL((fields_wfirst_kernel<zd>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
-                         (zd*)c->X, c->hybridW, c->flags + 1, (uint32_t*)nullptr);
+      hipLaunchKernelGGL((fields_wfirst_kernel<zd, zd>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
+                         (zd*)c->X, c->hybridW, c->flags + 1, (uint32_t*)nullptr, pre);
     else if (c->bsplit)
-      hipLaunchKernelGGL((fields_wfirst_kernel<zb>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
-                         (zb*)c->X, c->hybridW, c->flags + 1, c->tp_X);
+      hipLaunchKernelGGL((fields_wfirst_kernel<zb, zf>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
+                         (zb*)c->X, c->hybridW, c->flags + 1, c->tp_X, pre);
     else
-      hipLaunchKernelGGL((fields_wfirst_kernel<zf>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
-                         (zf*)c->X, c->hybridW, c->flags + 1, (uint32_t*)nullptr);
+      hipLaunchKernelGGL((fields_wfirst_kernel<zf, zf>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
+                         (zf*)c->X, c->hybridW, c->flags + 1, (uint32_t*)nullptr, pre);
   });
 }
 
@@ -1439,7 +1471,7 @@ int do_propagate(afqmc_ctx* c)
     a.N = c->N;
     a.nw = c->nw;
     a.ncb = 0;
-    return launch(c, "prop_fused", [&]() { prop_small_launch(c->stream, a, fmt); });
+    return launch(c, "prop_fused", [&]() { prop_small_launch(c->stream, a, fmt); }, 8);
   }
   if (fused_prop_ok(c)) return propagate_fused(c);
   if (c->mode == AFQMC_FP64_CSR) return propagate_f64(c, c->vHSw);
@@ -1738,10 +1770,6 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
   const int M = c->M, N = c->N, K = c->K, nw = c->nw;
   const long NM = (long)N * M;
   const double inv_dt = 1.0 / c->dt_sys;
-  RET(launch(c, "energy_zero", [&]() {
-    (void)hipMemsetAsync(c->e_direct, 0, sizeof(zd) * nw, c->stream);
-    (void)hipMemsetAsync(c->e_exch_part, 0, sizeof(zd) * 2 * nw, c->stream);
-  }));
   // direct term: v(w,n) = sum Lt G ; direct = sum_n v^2 / dt
   if constexpr (CPV == CP_BF16X6) {
     // three pieces of the split G (built for the exchange) and of Lt
@@ -1751,10 +1779,6 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     RET((dense_contract_vbias<CPV, GT, LVT>(c, Gp, Lv, c->e_v, "energy_v_gemm", nullptr, nullptr,
                                             "energy_v_reduce")));
   }
-  RET(launch(c, "energy_direct", [&]() {
-    hipLaunchKernelGGL((sumsq_kernel<zd>), dim3(nw), dim3(256), 0, c->stream, K, c->e_v, 1L, (long)K, c->e_direct,
-                       inv_dt);
-  }));
   bool one = false;
   if constexpr (std::is_same<GT, double>::value && (CP == CP_F64 || CP == CP_BF16X3 || CP == CP_BF16X6)) {
     one = c->Vx && exch_one_ok<CP>(c);
@@ -1818,6 +1842,8 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
   } else {
   // exchange: Y_n,s = Lt_s(n) G_s^T (N x N), sum_ab Y_ab Y_ba, for all
   // walker-spin pairs at once over chunks of nq vectors
+  RET(launch(c, "energy_zero",
+             [&]() { (void)hipMemsetAsync(c->e_exch_part, 0, sizeof(zd) * 2 * nw, c->stream); }));
   const long per_item = (long)N * N;
   const long ycap = (long)(c->ybuf_bytes / sizeof(typename ztype<YT>::type));
   const int nq = (int)std::max<long>(1, std::min<long>(K, ycap / (2L * nw * per_item)));
@@ -1882,18 +1908,10 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     }));
   }
   }
-  RET(launch(c, "energy_pairsum", [&]() {
-    hipLaunchKernelGGL(pairsum_kernel, dim3((nw + 255) / 256), dim3(256), 0, c->stream, c->e_exch_part, c->e_exch, nw);
-  }));
-  // one-body: e1 = sum_i G(w,i) haj(i)
-  RET(launch(c, "energy_one", [&]() {
-    hipLaunchKernelGGL((coldot_kernel<typename ztype<GT>::type, zd>), dim3(nw), dim3(256), 0, c->stream, (int)(2 * NM),
-                       (const typename ztype<GT>::type*)Gp, 1L, 2 * NM, (const zd*)c->haj, 1L, 0L, c->e_one, 1L, 1.0,
-                       0);
-  }));
   return launch(c, "energy_assemble", [&]() {
-    hipLaunchKernelGGL(energy_assemble_kernel, dim3((nw + 255) / 256), dim3(256), 0, c->stream, c->Wd, c->e_direct,
-                       c->e_exch, c->e_one, nw);
+    hipLaunchKernelGGL((energy_finish_kernel<typename ztype<GT>::type>), dim3(nw), dim3(256), 0, c->stream, K, c->e_v,
+                       inv_dt, (int)(2 * NM), (const typename ztype<GT>::type*)Gp, c->haj, c->e_exch_part, c->e_direct,
+                       c->e_exch, c->e_one, c->Wd);
   });
 }
 
@@ -1994,18 +2012,10 @@ int do_energy(afqmc_ctx* c, double* eav_out)
                   (long)nw, c->Gcloc, (long)nw, one, zero));
       // E2 = sum G.(Vakbl G) lands in the direct slot (exchange slot zero),
       // so E_L = E2/2 + E1 as energy.hpp:93-100
-      RET(launch(c, "energy_two", [&]() {
-        (void)hipMemsetAsync(c->e_exch, 0, sizeof(zd) * nw, c->stream);
-        hipLaunchKernelGGL((coldot_kernel<zd, zd>), dim3(nw), dim3(256), 0, c->stream, (int)NAK, (const zd*)c->G,
-                           (long)nw, 1L, (const zd*)c->Gcloc, (long)nw, 1L, c->e_direct, 1L, 1.0, 0);
-      }));
-      RET(launch(c, "energy_one", [&]() {
-        hipLaunchKernelGGL((coldot_kernel<zd, zd>), dim3(nw), dim3(256), 0, c->stream, (int)NAK, (const zd*)c->G,
-                           (long)nw, 1L, (const zd*)c->haj, 1L, 0L, c->e_one, 1L, 1.0, 0);
-      }));
       RET(launch(c, "energy_assemble", [&]() {
-        hipLaunchKernelGGL(energy_assemble_kernel, dim3((nw + 255) / 256), dim3(256), 0, c->stream, c->Wd,
-                           c->e_direct, c->e_exch, c->e_one, nw);
+        hipLaunchKernelGGL(energy_vakbl_kernel, dim3((nw + 15) / 16), dim3(1024), 0, c->stream, (int)NAK, nw,
+                           (const zd*)c->G, (const zd*)c->Gcloc, (const zd*)c->haj, c->e_direct, c->e_exch, c->e_one,
+                           c->Wd);
       }));
     } else {
       const void* G = c->G;
@@ -2083,17 +2093,27 @@ int check_flags(afqmc_ctx* c)
 int substep_body(afqmc_ctx* c, const double* xdev, long substep, int do_ortho_, double dt,
                  const long* xslice = nullptr)
 {
+  // the overlaps are saved (from the reused inverse's determinants, if it is)
+  // and the bias's partial sums joined in the fields kernel: nothing between
+  // the density matrix and the new overlaps reads either
+  FieldPre pre{};
+  pre.Wd = c->Wd;
+  pre.Wl = c->Wl;
+  if (c->t1inv_valid) {
+    pre.dcache = c->dcache;
+    pre.lcache = c->lcache;
+  }
+  c->vws_pending = 0;
   if (c->transposed) {
-    RET(do_mdm(c));
-    RET(do_vbias(c));
+    RET(do_mdm(c, false));
+    RET(do_vbias(c, true));
   } else {
-    RET(do_mdm_full(c));
+    RET(do_mdm_full(c, false));
     RET(do_vbias_full(c));
   }
-  RET(do_fields(c, xdev, substep, xslice));
+  RET(do_fields(c, xdev, substep, xslice, pre));
   RET(do_vhs(c));
   RET(do_propagate(c));
-  RET(do_save_overlaps(c));
   RET(do_overlaps(c));
   RET(do_weights(c, nullptr, dt));
   if (do_ortho_) {
@@ -2924,22 +2944,17 @@ int afqmc_fields(afqmc_ctx* c, const double* x, long substep)
   NEED_SYSTEM(c);
   const long KW = (long)c->K * c->nw;
   const double* xdev = nullptr;
-  double* tmp = nullptr;
   if (x) {
-    RET(dalloc(c, &tmp, KW));
-    HIPCHK(c, hipMemcpyAsync(tmp, x, sizeof(double) * KW, hipMemcpyHostToDevice, c->stream));
-    xdev = tmp;
+    if (!c->xtmp) RET(dalloc(c, &c->xtmp, KW));
+    HIPCHK(c, hipMemcpyAsync(c->xtmp, x, sizeof(double) * KW, hipMemcpyHostToDevice, c->stream));
+    xdev = c->xtmp;
   } else {
     if (!have_fields(c, substep)) return fail(c, AFQMC_ERR_STATE, "no staged fields for substep");
     xdev = stage_at(c, substep);
   }
-  int r = do_fields(c, xdev, substep);
-  if (r == AFQMC_OK) r = check_flags(c);
-  if (tmp) {
-    (void)hipStreamSynchronize(c->stream);
-    dfree(c, tmp);
-  }
-  return r;
+  c->vws_pending = 0;  // vbias is complete between calls
+  RET(do_fields(c, xdev, substep));
+  return check_flags(c);
 }
 int afqmc_vhs(afqmc_ctx* c)
 {

@@ -848,23 +848,63 @@ __device__ inline void field_term(zd b, double xr, zd& h, zd& Xo)
   Xo = zd{xr - b.im, b.re};
 }
 
+// What a substep leaves to its fields kernel, which has a thread for every
+// bias entry and walker anyway: the sum of the bias contraction's ns partial
+// products (into vb, in order), and the saved overlaps (save_overlaps_kernel),
+// taken from the last inverse's determinants where the density matrix reused
+// it (dcache, lcache: det_restore_kernel).  Zero: neither.
+struct FieldPre {
+  const void* slices;  // [ns][nw*K]
+  int ns;
+  zd* Wd;              // not null: save the overlaps
+  zd* Wl;
+  const zd* dcache;    // null: from W_data
+  const zd* lcache;
+};
+
+__device__ inline void save_overlaps_row(zd* d, zd* l, const zd* dc, const zd* lc)
+{
+  d[5] = d[4];
+  d[6] = dc ? dc[0] : d[2];
+  d[7] = dc ? dc[1] : d[3];
+  l[2] = lc ? lc[0] : l[0];
+  l[3] = lc ? lc[1] : l[1];
+}
+__device__ inline void field_pre_save(const FieldPre& p, long w)
+{
+  save_overlaps_row(p.Wd + w * 8, p.Wl + w * 4, p.dcache ? p.dcache + 2 * w : nullptr,
+                    p.lcache ? p.lcache + 2 * w : nullptr);
+}
+// bias entry o (of tot), summed from the slices and stored when there are any
+template <class PZ> __device__ inline zd field_bias(const FieldPre& p, zd* vb, long o, long tot)
+{
+  if (!p.ns) return vb[o];
+  const PZ* s = (const PZ*)p.slices + o;
+  zd a{0.0, 0.0};
+#pragma unroll 4
+  for (int q = 0; q < p.ns; q++) a = zadd(a, to_zd(s[(long)q * tot]));
+  vb[o] = a;
+  return a;
+}
+
 // Walker-first layouts (vbias, X [nw][K]): one workgroup per walker, the
 // lanes along n (coalesced), each thread a pair (2j, 2j+1) of draws at a
 // time; fixed-order block reduction of hybridW.
-template <class XT>
-__global__ __launch_bounds__(256) void fields_wfirst_kernel(int K, int nw, const zd* __restrict__ vb, FieldSrc src,
+template <class XT, class PZ>
+__global__ __launch_bounds__(256) void fields_wfirst_kernel(int K, int nw, zd* __restrict__ vb, FieldSrc src,
                                                             XT* __restrict__ X, zd* __restrict__ hybridW,
-                                                            int* __restrict__ nonfinite,
-                                                            uint32_t* __restrict__ X3 = nullptr)
+                                                            int* __restrict__ nonfinite, uint32_t* __restrict__ X3,
+                                                            FieldPre pre)
 {
   __shared__ zd part[4];
   const int w = blockIdx.x;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
   const long sub = src.xslice ? *src.xslice : src.substep;
   const double* x = src.x ? src.x + (src.xslice ? sub * (long)K * nw : 0L) : nullptr;
-  const zd* vbw = vb + (long)w * K;
+  const long tot = (long)nw * K, o0 = (long)w * K;
   XT* Xw = X + (long)w * K;
   uint32_t* X3w = X3 ? X3 + (long)w * K : nullptr;
+  if (pre.Wd && threadIdx.x == 0) field_pre_save(pre, w);
   // split X with its third pieces (three-piece split-BF16), else as XT
   auto put = [&](int n, zd o) {
     if constexpr (std::is_same<XT, zb>::value) {
@@ -887,10 +927,10 @@ __global__ __launch_bounds__(256) void fields_wfirst_kernel(int K, int nw, const
       afqmc_rng::field_pair(src.seed, sub, w, n, xa, xb);
     }
     zd o;
-    field_term(vbw[n], xa, h, o);
+    field_term(field_bias<PZ>(pre, vb, o0 + n, tot), xa, h, o);
     put(n, o);
     if (n + 1 < K) {
-      field_term(vbw[n + 1], xb, h, o);
+      field_term(field_bias<PZ>(pre, vb, o0 + n + 1, tot), xb, h, o);
       put(n + 1, o);
     }
   }
@@ -905,22 +945,24 @@ __global__ __launch_bounds__(256) void fields_wfirst_kernel(int K, int nw, const
 }
 
 // Walker-last layout (vbias, X [K][nw], the FP64 CSR mode): one workgroup per
-// 64 walkers (lanes), its 16 waves taking pairs (2j, 2j+1) of n in turn;
-// fixed-order reduction over the waves.
+// 16 walkers, its 64 groups of 16 lanes taking pairs (2j, 2j+1) of n in turn;
+// fixed-order reduction over the groups.
 template <class XT>
-__global__ __launch_bounds__(1024) void fields_wlast_kernel(int K, int nw, const zd* __restrict__ vb, FieldSrc src,
+__global__ __launch_bounds__(1024) void fields_wlast_kernel(int K, int nw, zd* __restrict__ vb, FieldSrc src,
                                                             XT* __restrict__ X, zd* __restrict__ hybridW,
-                                                            int* __restrict__ nonfinite)
+                                                            int* __restrict__ nonfinite, FieldPre pre)
 {
-  __shared__ zd part[16][64];
-  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
-  const int w = blockIdx.x * 64 + lane;
+  __shared__ zd part[64][16];
+  const int lw = threadIdx.x & 15, grp = threadIdx.x >> 4;
+  const int w = blockIdx.x * 16 + lw;
   const long sub = src.xslice ? *src.xslice : src.substep;
   const double* x = src.x ? src.x + (src.xslice ? sub * (long)K * nw : 0L) : nullptr;
+  const long tot = (long)nw * K;
   zd h{0, 0};
   bool bad = false;
   if (w < nw) {
-    for (int n = 2 * wv; n < K; n += 32) {
+    if (pre.Wd && grp == 0) field_pre_save(pre, w);
+    for (int n = 2 * grp; n < K; n += 128) {
       double xa, xb = 0.0;
       if (x) {
         xa = x[(long)n * nw + w];
@@ -930,22 +972,22 @@ __global__ __launch_bounds__(1024) void fields_wlast_kernel(int K, int nw, const
         afqmc_rng::field_pair(src.seed, sub, w, n, xa, xb);
       }
       zd o;
-      field_term(vb[(long)n * nw + w], xa, h, o);
+      field_term(field_bias<zd>(pre, vb, (long)n * nw + w, tot), xa, h, o);
       from_zd(o, X[(long)n * nw + w]);
       if (n + 1 < K) {
-        field_term(vb[(long)(n + 1) * nw + w], xb, h, o);
+        field_term(field_bias<zd>(pre, vb, (long)(n + 1) * nw + w, tot), xb, h, o);
         from_zd(o, X[(long)(n + 1) * nw + w]);
       }
     }
   }
   if (bad) atomicOr(nonfinite, 1);
-  part[wv][lane] = h;
+  part[grp][lw] = h;
   __syncthreads();
-  if (wv == 0 && w < nw) {
-    zd t = part[0][lane];
-    for (int q = 1; q < 16; q++) t = zadd(t, part[q][lane]);
-    hybridW[w] = t;
+  for (int s = 32; s >= 1; s >>= 1) {
+    if (grp < s) part[grp][lw] = zadd(part[grp][lw], part[grp + s][lw]);
+    __syncthreads();
   }
+  if (grp == 0 && w < nw) hybridW[w] = part[0][lw];
 }
 
 // W_data[:,5] = W_data[:,4]; W_data[:,6..7] = W_data[:,2..3]; the
@@ -954,13 +996,7 @@ __global__ void save_overlaps_kernel(zd* __restrict__ Wd, zd* __restrict__ Wl, i
 {
   int w = blockIdx.x * blockDim.x + threadIdx.x;
   if (w >= nw) return;
-  zd* d = Wd + (long)w * 8;
-  d[5] = d[4];
-  d[6] = d[2];
-  d[7] = d[3];
-  zd* l = Wl + (long)w * 4;
-  l[2] = l[0];
-  l[3] = l[1];
+  save_overlaps_row(Wd + (long)w * 8, Wl + (long)w * 4, nullptr, nullptr);
 }
 
 // weights / hybrid energy / Eshift (src/miniapps/miniafqmc_base.cpp:317-327).
@@ -1701,47 +1737,86 @@ __global__ void add_parts_kernel(const zd* __restrict__ part, int ng, zd* __rest
   out[q] = a;
 }
 
-// out[w] = part[2w] + part[2w+1] (the two spins)
-__global__ void pairsum_kernel(const zd* __restrict__ part, zd* __restrict__ out, int nw)
+// The local energy's last step, one workgroup per walker: the Coulomb sum
+// direct = inv_dt * sum_n v(w,n)^2, the exchange from its two spins, the
+// one-body term sum_i G(w,i) haj(i), and W_data[w][0] = (direct - exch)/2 +
+// e1 (energy.hpp:93-100 in the Cholesky form).  G and v walker-first.
+template <class GZ>
+__global__ __launch_bounds__(256) void energy_finish_kernel(int K, const zd* __restrict__ v, double inv_dt, int n,
+                                                            const GZ* __restrict__ G, const zd* __restrict__ haj,
+                                                            const zd* __restrict__ exch_part, zd* __restrict__ direct,
+                                                            zd* __restrict__ exch, zd* __restrict__ one,
+                                                            zd* __restrict__ Wd)
 {
-  int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w < nw) out[w] = zadd(part[2 * w], part[2 * w + 1]);
-}
-
-// direct term: out[w] += sum_n v(n,w)^2 where v(n,w) at v[n*vsn + w*vsw]
-template <class VT>
-__global__ __launch_bounds__(256) void sumsq_kernel(int K, const VT* __restrict__ v, long vsn, long vsw,
-                                                    zd* __restrict__ out, double scale)
-{
-  __shared__ zd sh[256];
-  const int w = blockIdx.x;
-  zd acc{0, 0};
-  for (int n = threadIdx.x; n < K; n += 256) {
-    const zd x = to_zd(v[(long)n * vsn + (long)w * vsw]);
-    acc.re += x.re * x.re - x.im * x.im;
-    acc.im += 2.0 * x.re * x.im;
+  __shared__ zd sh[2][256];
+  const int w = blockIdx.x, tid = threadIdx.x;
+  zd a{0, 0}, b{0, 0};
+  for (int i = tid; i < K; i += 256) {
+    const zd x = v[(long)w * K + i];
+    a.re += x.re * x.re - x.im * x.im;
+    a.im += 2.0 * x.re * x.im;
   }
-  sh[threadIdx.x] = acc;
+  for (int i = tid; i < n; i += 256) {
+    const zd g = to_zd(G[(long)w * n + i]), h = haj[i];
+    b.re += g.re * h.re - g.im * h.im;
+    b.im += g.re * h.im + g.im * h.re;
+  }
+  sh[0][tid] = a;
+  sh[1][tid] = b;
   __syncthreads();
   for (int s = 128; s > 0; s >>= 1) {
-    if (threadIdx.x < s) sh[threadIdx.x] = zadd(sh[threadIdx.x], sh[threadIdx.x + s]);
+    if (tid < s) {
+      sh[0][tid] = zadd(sh[0][tid], sh[0][tid + s]);
+      sh[1][tid] = zadd(sh[1][tid], sh[1][tid + s]);
+    }
     __syncthreads();
   }
-  if (threadIdx.x == 0) {
-    out[w].re += scale * sh[0].re;
-    out[w].im += scale * sh[0].im;
+  if (tid == 0) {
+    const zd d{inv_dt * sh[0][0].re, inv_dt * sh[0][0].im};
+    const zd x = zadd(exch_part[2 * w], exch_part[2 * w + 1]);
+    direct[w] = d;
+    exch[w] = x;
+    one[w] = sh[1][0];
+    Wd[(long)w * 8] = zadd(zd{0.5 * (d.re - x.re), 0.5 * (d.im - x.im)}, sh[1][0]);
   }
 }
 
-// E_L assembly for the Cholesky form:
-// Wd[w][0] = 0.5*(direct[w] - exch[w]) + e1[w]
-__global__ void energy_assemble_kernel(zd* __restrict__ Wd, const zd* __restrict__ direct,
-                                       const zd* __restrict__ exch, const zd* __restrict__ e1, int nw)
+// The same with Vakbl (energy.hpp:93-100): direct = sum_i G(i,w) Y(i,w) with
+// Y = Vakbl G, no exchange; G and Y walker-last, one workgroup per 16 walkers.
+__global__ __launch_bounds__(1024) void energy_vakbl_kernel(int n, int nw, const zd* __restrict__ G,
+                                                            const zd* __restrict__ Y, const zd* __restrict__ haj,
+                                                            zd* __restrict__ direct, zd* __restrict__ exch,
+                                                            zd* __restrict__ one, zd* __restrict__ Wd)
 {
-  int w = blockIdx.x * blockDim.x + threadIdx.x;
-  if (w >= nw) return;
-  zd e2{0.5 * (direct[w].re - exch[w].re), 0.5 * (direct[w].im - exch[w].im)};
-  Wd[(long)w * 8] = zadd(e2, e1[w]);
+  __shared__ zd sh[2][64][16];
+  const int lw = threadIdx.x & 15, grp = threadIdx.x >> 4;
+  const int w = blockIdx.x * 16 + lw;
+  zd a{0, 0}, b{0, 0};
+  if (w < nw)
+    for (int i = grp; i < n; i += 64) {
+      const zd g = G[(long)i * nw + w], y = Y[(long)i * nw + w], h = haj[i];
+      a.re += g.re * y.re - g.im * y.im;
+      a.im += g.re * y.im + g.im * y.re;
+      b.re += g.re * h.re - g.im * h.im;
+      b.im += g.re * h.im + g.im * h.re;
+    }
+  sh[0][grp][lw] = a;
+  sh[1][grp][lw] = b;
+  __syncthreads();
+  for (int s = 32; s >= 1; s >>= 1) {
+    if (grp < s) {
+      sh[0][grp][lw] = zadd(sh[0][grp][lw], sh[0][grp + s][lw]);
+      sh[1][grp][lw] = zadd(sh[1][grp][lw], sh[1][grp + s][lw]);
+    }
+    __syncthreads();
+  }
+  if (grp == 0 && w < nw) {
+    const zd d = sh[0][0][lw], e1 = sh[1][0][lw];
+    direct[w] = d;
+    exch[w] = zd{0, 0};
+    one[w] = e1;
+    Wd[(long)w * 8] = zadd(zd{0.5 * d.re, 0.5 * d.im}, e1);
+  }
 }
 
 // ---------------------------------------------------------------------------
