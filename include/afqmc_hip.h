@@ -165,7 +165,9 @@ typedef enum {
   /* AFQMC_FP64_CSR with the transposed bias, set before afqmc_upload_system:
    * 1 (default) keeps a dense copy of the half-rotated SpvnT when at least
    * half of its entries are stored (those under the cutoff are zero) and
-   * runs the bias product on FP64 MFMA; 0 always runs the CSR product.  No
+   * runs the bias product on FP64 MFMA, and likewise keeps Vakbl dense in
+   * place of its CSR form when at least half of it is stored (its rows'
+   * columns ascending); 0 always runs the CSR products.  No
    * counterpart in the reference (its csrmm is the only form). */
   AFQMC_OPT_CSR_DENSE = 11,
   /* nonzero (AFQMC_MIXED_BF16 at energy levels 1-2, set before the system

@@ -85,6 +85,7 @@ struct afqmc_ctx {
   int* v_col = nullptr;
   zd* v_val = nullptr;
   long long v_nnz = 0;
+  zd* vkd = nullptr;  // Vakbl dense, [2NM][2NM], when at least half of it is stored (AFQMC_OPT_CSR_DENSE)
   void* Ld = nullptr;  // dense modes: [K][M*M]  (zd or zf)
   void* Lt = nullptr;  // [2][K][N*M] (zd or zf); scaled by sqrt(dt)
   zd* Lt64 = nullptr;  // mixed modes with energy_level >= 1: Lt in FP64
@@ -849,12 +850,13 @@ int need_vws(afqmc_ctx* c, size_t bytes)
 }
 
 // Chunks of a k sum of length kt whose output is m x n: enough 64 x 64 tiles
-// for four workgroups per CU, each chunk at least 256 long and a multiple of
-// the k-tile, at most smax of them; the last one may be shorter.
+// for four workgroups per CU, each chunk at least 128 long (16 steps of the
+// k loop: below that its first loads dominate) and a multiple of the k-tile,
+// at most smax of them; the last one may be shorter.
 long f64_chunk(long m, long n, long kt, int items, int smax)
 {
   const long tiles = ((m + 63) / 64) * ((n + 63) / 64) * items;
-  const long s = std::max<long>(1, std::min<long>(std::min<long>(smax, kt / 256), (1024 + tiles - 1) / tiles));
+  const long s = std::max<long>(1, std::min<long>(std::min<long>(smax, kt / 128), (1024 + tiles - 1) / tiles));
   return (((kt + s - 1) / s) + 7) / 8 * 8;
 }
 
@@ -1099,8 +1101,13 @@ int do_fields(afqmc_ctx* c, const double* xdev, long substep, const long* xslice
   c->vws_pending = 0;
   if (c->mode == AFQMC_FP64_CSR)
     return launch(c, "fields", [&]() {
-      hipLaunchKernelGGL((fields_wlast_kernel<zd>), dim3((nw + 15) / 16), dim3(1024), 0, c->stream, K, nw, c->vbias,
-                         src, (zd*)c->X, c->hybridW, c->flags + 1, pre);
+      // few walkers: four a workgroup, so that more than one CU reads
+      if (nw <= 64)
+        hipLaunchKernelGGL((fields_wlast_kernel<zd, 4>), dim3((nw + 3) / 4), dim3(1024), 0, c->stream, K, nw, c->vbias,
+                           src, (zd*)c->X, c->hybridW, c->flags + 1, pre);
+      else
+        hipLaunchKernelGGL((fields_wlast_kernel<zd, 16>), dim3((nw + 15) / 16), dim3(1024), 0, c->stream, K, nw,
+                           c->vbias, src, (zd*)c->X, c->hybridW, c->flags + 1, pre);
     });
   return launch(c, "fields", [&]() {
     if (!c->mixed)
@@ -2006,7 +2013,34 @@ int do_energy(afqmc_ctx* c, double* eav_out)
   const int nw = c->nw, N = c->N, M = c->M;
   const long NAK = 2L * N * M;
   if (c->mode == AFQMC_FP64_CSR) {
-    if (c->v_rp) {
+    if (c->vkd) {
+      // Y(w, i) = sum_j G(w, j) Vakbl(i, j) on FP64 MFMA, split over j
+      const long chunk = f64_chunk(nw, NAK, NAK, 1, 16);
+      const int S = (int)((NAK + chunk - 1) / chunk);
+      const long gsw = g_wfirst(c) ? NAK : 1, gsi = g_wfirst(c) ? 1 : nw;
+      RET(need_vws(c, sizeof(zd) * (size_t)S * nw * NAK));
+      F64Args a = f64args(nw, (int)NAK, (int)chunk);
+      a.ktot = NAK;
+      a.bdiv = S;
+      a.A = c->G;
+      a.sam = gsw;
+      a.sak = gsi;
+      a.sa2 = chunk * gsi;
+      a.B = c->vkd;
+      a.sbn = NAK;
+      a.sbk = 1;
+      a.sb2 = chunk;
+      a.C = c->vws;
+      a.scm = NAK;
+      a.scn = 1;
+      a.sc2 = nw * NAK;
+      RET(zgemm64<zd>(c, "energy_y_gemm", a, S));
+      RET(launch(c, "energy_assemble", [&]() {
+        hipLaunchKernelGGL(energy_vakbl_dense_kernel, dim3(nw), dim3(512), 0, c->stream, (int)NAK, nw,
+                           (const zd*)c->G, gsw, gsi, (const zd*)c->vws, S, (const zd*)c->haj, c->e_direct, c->e_exch,
+                           c->e_one, c->Wd);
+      }));
+    } else if (c->v_rp) {
       zd one{1, 0}, zero{0, 0};
       RET(csrmm_n(c, "csrmm_vakbl", (int)NAK, (int)NAK, c->v_nnz, c->v_rp, c->v_col, c->v_val, (const zd*)c->G,
                   (long)nw, c->Gcloc, (long)nw, one, zero));
@@ -2684,6 +2718,36 @@ int afqmc_upload_system(afqmc_ctx* c, const double* trial_alpha, const double* t
       HIPCHK(c, hipMemcpyAsync(c->v_col, vakbl->col + vakbl->rowptr[0], sizeof(int) * vn, hipMemcpyHostToDevice, st));
       HIPCHK(c, hipMemcpyAsync(c->v_val, vakbl->val + 2 * (long)vakbl->rowptr[0], sizeof(zd) * vn, hipMemcpyHostToDevice, st));
       c->v_nnz = vn;
+      // as SpvnT: rows at least half full make a dense product (not when
+      // entries repeat, which csrmm adds up), which reads no more bytes and
+      // runs on MFMA: 1024 x 1024, 16 walkers 288 -> 43 us.  The dense form
+      // takes the CSR form's place, so that little more memory is held.
+      bool dense = c->csr_dense && 2.0 * vn >= (double)vr * vr;
+      for (long r = 0; r < vr && dense; r++)
+        for (int q = rp0[r] + 1; q < rp0[r + 1]; q++)
+          if (vcol[q] <= vcol[q - 1]) {
+            dense = false;
+            break;
+          }
+      if (dense) {
+        size_t fr = 0, tot_ = 0;
+        HIPCHK(c, hipMemGetInfo(&fr, &tot_));
+        dense = sizeof(zd) * (size_t)vr * vr + ((size_t)2 << 30) <= fr;
+      }
+      if (dense) {
+        RET(dalloc(c, &c->vkd, (size_t)vr * vr));
+        HIPCHK(c, hipMemsetAsync(c->vkd, 0, sizeof(zd) * (size_t)vr * vr, st));
+        RET(launch(c, "csr_densify", [&]() {
+          hipLaunchKernelGGL(csr_densify_rows_kernel, dim3((unsigned)((vr + 3) / 4)), dim3(256), 0, st, (int)vr, c->v_rp,
+                             c->v_col, c->v_val, c->vkd, vr);
+        }));
+        HIPCHK(c, hipStreamSynchronize(st));
+        dfree(c, c->v_rp);
+        dfree(c, c->v_col);
+        dfree(c, c->v_val);
+        c->v_rp = c->v_col = nullptr;
+        c->v_val = nullptr;
+      }
       RET(dalloc(c, &c->Gcloc, 2 * NM * c->nw));
       HIPCHK(c, hipStreamSynchronize(st));
       dfree(c, Lt64);

@@ -945,16 +945,17 @@ __global__ __launch_bounds__(256) void fields_wfirst_kernel(int K, int nw, zd* _
 }
 
 // Walker-last layout (vbias, X [K][nw], the FP64 CSR mode): one workgroup per
-// 16 walkers, its 64 groups of 16 lanes taking pairs (2j, 2j+1) of n in turn;
-// fixed-order reduction over the groups.
-template <class XT>
+// LW walkers, its 1024 / LW groups of LW lanes taking pairs (2j, 2j+1) of n in
+// turn; fixed-order reduction over the groups.
+template <class XT, int LW>
 __global__ __launch_bounds__(1024) void fields_wlast_kernel(int K, int nw, zd* __restrict__ vb, FieldSrc src,
                                                             XT* __restrict__ X, zd* __restrict__ hybridW,
                                                             int* __restrict__ nonfinite, FieldPre pre)
 {
-  __shared__ zd part[64][16];
-  const int lw = threadIdx.x & 15, grp = threadIdx.x >> 4;
-  const int w = blockIdx.x * 16 + lw;
+  constexpr int NG = 1024 / LW;
+  __shared__ zd part[NG][LW];
+  const int lw = threadIdx.x % LW, grp = threadIdx.x / LW;
+  const int w = blockIdx.x * LW + lw;
   const long sub = src.xslice ? *src.xslice : src.substep;
   const double* x = src.x ? src.x + (src.xslice ? sub * (long)K * nw : 0L) : nullptr;
   const long tot = (long)nw * K;
@@ -962,7 +963,7 @@ __global__ __launch_bounds__(1024) void fields_wlast_kernel(int K, int nw, zd* _
   bool bad = false;
   if (w < nw) {
     if (pre.Wd && grp == 0) field_pre_save(pre, w);
-    for (int n = 2 * grp; n < K; n += 128) {
+    for (int n = 2 * grp; n < K; n += 2 * NG) {
       double xa, xb = 0.0;
       if (x) {
         xa = x[(long)n * nw + w];
@@ -983,7 +984,7 @@ __global__ __launch_bounds__(1024) void fields_wlast_kernel(int K, int nw, zd* _
   if (bad) atomicOr(nonfinite, 1);
   part[grp][lw] = h;
   __syncthreads();
-  for (int s = 32; s >= 1; s >>= 1) {
+  for (int s = NG / 2; s >= 1; s >>= 1) {
     if (grp < s) part[grp][lw] = zadd(part[grp][lw], part[grp + s][lw]);
     __syncthreads();
   }
@@ -1781,7 +1782,47 @@ __global__ __launch_bounds__(256) void energy_finish_kernel(int K, const zd* __r
   }
 }
 
-// The same with Vakbl (energy.hpp:93-100): direct = sum_i G(i,w) Y(i,w) with
+// The same with Vakbl kept dense: Y = Vakbl G as ns partial products
+// [ns][nw][n] (summed in order), one workgroup per walker; G(w, i) at
+// G[w * gsw + i * gsi].
+__global__ __launch_bounds__(512) void energy_vakbl_dense_kernel(int n, int nw, const zd* __restrict__ G, long gsw,
+                                                                 long gsi, const zd* __restrict__ Y, int ns,
+                                                                 const zd* __restrict__ haj, zd* __restrict__ direct,
+                                                                 zd* __restrict__ exch, zd* __restrict__ one,
+                                                                 zd* __restrict__ Wd)
+{
+  __shared__ zd sh[2][512];
+  const int w = blockIdx.x, tid = threadIdx.x;
+  zd a{0, 0}, b{0, 0};
+  for (int i = tid; i < n; i += 512) {
+    zd y{0, 0};
+#pragma unroll 4
+    for (int q = 0; q < ns; q++) y = zadd(y, Y[((long)q * nw + w) * n + i]);
+    const zd g = G[w * gsw + i * gsi], h = haj[i];
+    a.re += g.re * y.re - g.im * y.im;
+    a.im += g.re * y.im + g.im * y.re;
+    b.re += g.re * h.re - g.im * h.im;
+    b.im += g.re * h.im + g.im * h.re;
+  }
+  sh[0][tid] = a;
+  sh[1][tid] = b;
+  __syncthreads();
+  for (int s = 256; s > 0; s >>= 1) {
+    if (tid < s) {
+      sh[0][tid] = zadd(sh[0][tid], sh[0][tid + s]);
+      sh[1][tid] = zadd(sh[1][tid], sh[1][tid + s]);
+    }
+    __syncthreads();
+  }
+  if (tid == 0) {
+    direct[w] = sh[0][0];
+    exch[w] = zd{0, 0};
+    one[w] = sh[1][0];
+    Wd[(long)w * 8] = zadd(zd{0.5 * sh[0][0].re, 0.5 * sh[0][0].im}, sh[1][0]);
+  }
+}
+
+// The same with Vakbl in CSR (energy.hpp:93-100): direct = sum_i G(i,w) Y(i,w) with
 // Y = Vakbl G, no exchange; G and Y walker-last, one workgroup per 16 walkers.
 __global__ __launch_bounds__(1024) void energy_vakbl_kernel(int n, int nw, const zd* __restrict__ G,
                                                             const zd* __restrict__ Y, const zd* __restrict__ haj,

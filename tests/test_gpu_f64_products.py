@@ -100,6 +100,37 @@ def test_exchange_in_one_launch_vs_cholesky_form(require_gpu, mode, level, tol, 
         assert np.abs(e - ref).max() <= tol * np.abs(ref).max()
 
 
+@pytest.mark.parametrize("M,N,nw", [(9, 3, 5), (24, 6, 64), (37, 19, 67)])
+def test_vakbl_dense_vs_csr(require_gpu, M, N, nw):
+    """Vakbl kept dense gives the CSR product's energy terms; one whose entries
+    repeat (each stored as two halves) keeps the CSR product, which adds them."""
+    say("Vakbl dense", M, N, nw)
+    s = m.make_system(M, N, 32, density=0.7, sigma_L=0.05, sigma_h=1.0, dt=0.005, seed=M * N, with_vakbl=True)
+    full = s.vakbl
+    twice = m.Csr(full.nrows, full.ncols, (2 * full.rowptr).astype(full.rowptr.dtype), np.repeat(full.col, 2),
+                  np.repeat(full.val, 2) / 2)
+    assert 2 * full.nnz >= full.nrows**2
+    W = walkers(s, nw, seed=nw)
+    Wd = np.zeros((nw, 8), complex)
+    Wd[:, 1] = 1.0
+    got = []
+    for v, dense in ((full, False), (full, True), (twice, True)):
+        s.vakbl = v
+        g = m.AfqmcSys(s, nw, "fp64_csr", csr_dense=dense)
+        g.set(nat.BUF_W, W)
+        g.set(nat.BUF_WDATA, Wd)
+        g.calculate_mixed_density_matrix()
+        g.profile(True)
+        g.calculate_energy()
+        names = set(g.kernel_stats())
+        g.profile(False)
+        got.append(np.concatenate([g.energy_terms(), g.W_data[:, :1]], axis=1))
+        g.close()
+        assert ("csrmm_vakbl" in names) == (not dense or v is twice), sorted(names)
+    for e in got[1:]:
+        assert np.abs(e - got[0]).max() <= 1e-12 * np.abs(got[0]).max()
+
+
 @pytest.mark.parametrize("N", [1, 2, 4, 5, 15, 16, 17, 31, 32, 33, 63, 64, 65, 95, 96, 97, 127, 128, 129, 160, 256])
 def test_batched_inverse_pivots(require_gpu, N):
     """Overlap matrices with prescribed pivot choices (the trial is the first N
