@@ -667,8 +667,12 @@ int gj_inverse_into(afqmc_ctx* c, zd* T, zd* Tinv, zd* det, long dq, long dr, in
   auto go = [&](auto rpl, auto nwv, auto cpw) {
     constexpr int RPL = decltype(rpl)::value, NW = decltype(nwv)::value, CPW = decltype(cpw)::value;
     return launch(c, "gj_inverse", [&]() {
-      hipLaunchKernelGGL((gj_inverse_kernel<RPL, NW, CPW>), dim3(batch), dim3(64 * NW), 0, c->stream, T, Tinv, det,
-                         dq, dr, N, ms, flags, dc, ldet, lc);
+      if (c->mixed)
+        hipLaunchKernelGGL((gj_inverse_kernel<RPL, NW, CPW, true>), dim3(batch), dim3(64 * NW), 0, c->stream, T, Tinv,
+                           det, dq, dr, N, ms, flags, dc, ldet, lc);
+      else
+        hipLaunchKernelGGL((gj_inverse_kernel<RPL, NW, CPW, false>), dim3(batch), dim3(64 * NW), 0, c->stream, T, Tinv,
+                           det, dq, dr, N, ms, flags, dc, ldet, lc);
     });
   };
   std::integral_constant<int, 1> i1;
@@ -686,8 +690,12 @@ int gj_inverse_into(afqmc_ctx* c, zd* T, zd* Tinv, zd* det, long dq, long dr, in
     // in global memory (allocated at the first call)
     if (!c->gjwork) RET(dalloc(c, &c->gjwork, (size_t)batch * ms));
     return launch(c, "gj_inverse", [&]() {
-      hipLaunchKernelGGL(gj_inverse_global_kernel, dim3(batch), dim3(1024), 0, c->stream, T, Tinv, c->gjwork, det, dq,
-                         dr, N, ms, flags, dc, ldet, lc);
+      if (c->mixed)
+        hipLaunchKernelGGL(gj_inverse_global_kernel<true>, dim3(batch), dim3(1024), 0, c->stream, T, Tinv, c->gjwork,
+                           det, dq, dr, N, ms, flags, dc, ldet, lc);
+      else
+        hipLaunchKernelGGL(gj_inverse_global_kernel<false>, dim3(batch), dim3(1024), 0, c->stream, T, Tinv, c->gjwork,
+                           det, dq, dr, N, ms, flags, dc, ldet, lc);
     });
   }
   return fail(c, AFQMC_ERR_UNSUPPORTED, "N > 256 electrons per spin is not supported by the batched inverse");

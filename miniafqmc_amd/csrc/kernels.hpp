@@ -124,7 +124,15 @@ __device__ __forceinline__ zd zrecip(zd b)
 // 150 -> 90, 192 x 32 48 -> 29, 32 x 16 23 -> 17.  With the search, the
 // reciprocal and all updates but the searched column's taken out, 128 x N = 128
 // went from 230 to 93 us.
-template <int RPL, int NW, int CPW>
+//
+// SCALED (the mixed modes): the pivot row is scaled as it is chosen, by its
+// one lane after the other rows' updates, with the reciprocal by division.
+// That is the elimination's textbook rounding; the mixed modes round T^-1 to
+// FP32, where an ulp of FP64 now and then turns an FP32 rounding and with it
+// everything the walker does afterwards, so their bits do not follow the
+// faster form (2048 x N = 128 2390 us against 2080, 512 x 96 385 against 321,
+// 512 x 64 117 against 96, one box).
+template <int RPL, int NW, int CPW, bool SCALED>
 __global__ __launch_bounds__(64 * NW) void gj_inverse_kernel(const zd* __restrict__ T, zd* __restrict__ Tinv,
                                                              zd* __restrict__ det, long dq, long dr, int N,
                                                              long mstride, int* __restrict__ info,
@@ -218,7 +226,7 @@ __global__ __launch_bounds__(64 * NW) void gj_inverse_kernel(const zd* __restric
       }
     }
     const bool zero = piv.re == 0.0 && piv.im == 0.0;
-    const zd ipv = zrecip(piv);
+    const zd ipv = SCALED ? zdiv(zd{1.0, 0.0}, piv) : zrecip(piv);
 #pragma unroll
     for (int q = 0; q < RPL; q++)
       gqs[st][lane + 64 * q] = lane + 64 * q == p ? zd{0.0, 0.0} : zmul(zd{-x[q][c].re, -x[q][c].im}, ipv);
@@ -259,7 +267,7 @@ __global__ __launch_bounds__(64 * NW) void gj_inverse_kernel(const zd* __restric
       for (int q = 0; q < RPL; q++) {
         const bool mine = lane + 64 * q == p;
         pos[q] = mine ? k : (pos[q] == k ? pp : pos[q]);
-        if (mine) scale[q] = ipv;
+        if (!SCALED && mine) scale[q] = ipv;
       }
       auto update = [&](int s, bool colk) __attribute__((always_inline)) {
         // row p's entry of the slot
@@ -275,15 +283,35 @@ __global__ __launch_bounds__(64 * NW) void gj_inverse_kernel(const zd* __restric
         }
         __builtin_amdgcn_sched_barrier(0);  // one slot at a time: bounds the live registers
       };
+      // the pivot row's entry of one slot, or of all others
+      auto rescale = [&](int s0, bool only) __attribute__((always_inline)) {
+        if constexpr (SCALED) {
+          auto row = [&](auto qc) __attribute__((always_inline)) {
+            constexpr int q = decltype(qc)::value;
+            if (lane == (p & 63)) {
+#pragma unroll
+              for (int s = 0; s < CPW; s++)
+                if ((s == s0) == only) {
+                  x[q][s] = zmul(x[q][s], ipv);
+                  __builtin_amdgcn_sched_barrier(0);
+                }
+            }
+          };
+          if (RPL == 2 && p >= 64) row(std::integral_constant<int, RPL - 1>());
+          else row(std::integral_constant<int, 0>());
+        }
+      };
       const int k1 = k + 1;
       // the search chain ahead of the other waves' updates
       if (wave == k1 / CPW) __builtin_amdgcn_s_setprio(3);
       update(c1, false);
+      rescale(c1, true);
       if (k1 < N && wave == k1 / CPW) publish(k1, std::integral_constant<int, c1>());
       __builtin_amdgcn_s_setprio(0);
 #pragma unroll
       for (int s = 0; s < CPW; s++)
         if (s != c1) update(s, s == c && wave == kb);
+      rescale(c1, false);
       if (wave == 0) dt = zmul(dt, spv);
       __syncthreads();
     };
@@ -316,7 +344,7 @@ __global__ __launch_bounds__(64 * NW) void gj_inverse_kernel(const zd* __restric
         const int i = lane + 64 * q, j = j0 + c;
         if (i < N && j < N) {
           if (singular) Tinv[b * mstride + (long)j * N + i] = zd{0, 0};  // a defined value
-          else Tinv[b * mstride + (long)prow[j] * N + pos[q]] = zmul(x[q][c], scale[q]);
+          else Tinv[b * mstride + (long)prow[j] * N + pos[q]] = SCALED ? x[q][c] : zmul(x[q][c], scale[q]);
         }
       }
   }
@@ -332,13 +360,15 @@ __global__ __launch_bounds__(64 * NW) void gj_inverse_kernel(const zd* __restric
 // written in its own step and every thread reads its entries (one or two
 // addresses a wave) while the others' rows change: one barrier per step.  The
 // threads of column k + 1 leave its new values in LDS, where every wave finds
-// the next pivot for itself.
+// the next pivot for itself.  SCALED as in the register kernel: the row's own
+// threads scale it in the following step (2450 against 2340 us at N = 160).
 //
 // Bound: the caches behind the L2 (the matrix is read and written once a
 // step; 128 matrices of 410 KB move 7 TB/s).  Measured (MI355X): 128 matrices
 // of N = 160 2.88 -> 2.30 ms (before: four barriers per step and a 64-bit
 // division by N per entry).
 constexpr int GJ_GMAX = 256;
+template <bool SCALED>
 __global__ __launch_bounds__(1024) void gj_inverse_global_kernel(const zd* __restrict__ T, zd* __restrict__ Tinv,
                                                                  zd* __restrict__ work, zd* __restrict__ det, long dq,
                                                                  long dr, int N, long mstride, int* __restrict__ info,
@@ -367,7 +397,7 @@ __global__ __launch_bounds__(1024) void gj_inverse_global_kernel(const zd* __res
     }
   __syncthreads();
   zd dt{1.0, 0.0}, scale{1.0, 0.0};
-  bool singular = false;
+  bool singular = false, last = false;  // last: row i was the last step's pivot row
   for (int k = 0; k < N; k++) {
     const zd* ck = colk[k & 1];
     // pivot: |Re| + |Im| largest, the lowest position among equals (keys as
@@ -415,11 +445,10 @@ __global__ __launch_bounds__(1024) void gj_inverse_global_kernel(const zd* __res
       pv[k] = spv;
       perm[k] = p;
     }
-    const zd ipv = zrecip(piv);
+    const zd ipv = SCALED ? zdiv(zd{1.0, 0.0}, piv) : zrecip(piv);
 #pragma unroll
     for (int q = 0; q < Q; q++) pos[q] = lane + 64 * q == p ? k : (pos[q] == k ? pp : pos[q]);
     mypos = i == p ? k : (mypos == k ? pp : mypos);
-    if (i == p) scale = ipv;
     const zd f = ck[i];
     const zd gq = i == p ? zd{0.0, 0.0} : zmul(zd{-f.re, -f.im}, ipv);
     if (active) {
@@ -429,14 +458,17 @@ __global__ __launch_bounds__(1024) void gj_inverse_global_kernel(const zd* __res
       for (int j = jg; j < N; j += G) {
         const long o = (long)j * N;
         zd x = Xi[o];
+        if (SCALED && last) x = zmul(x, scale);
         const zd pr = Xp[o];
         x.re = x.re + gq.re * pr.re - gq.im * pr.im;
         x.im = x.im + gq.re * pr.im + gq.im * pr.re;
         if (j == k) x = i == p ? zd{1.0, 0.0} : gq;
         if (i != p || j == k) Xi[o] = x;
-        if (j == k + 1) colk[(k + 1) & 1][i] = x;
+        if (j == k + 1) colk[(k + 1) & 1][i] = SCALED && i == p ? zmul(x, ipv) : x;
       }
     }
+    last = i == p;
+    if (last) scale = ipv;
     __syncthreads();
   }
   if (tid == 0) {
@@ -450,7 +482,7 @@ __global__ __launch_bounds__(1024) void gj_inverse_global_kernel(const zd* __res
   // T^-1[p_j][pos_i] = X(i, j) / pivot of row i, zeros when singular
   for (int j = jg; j < N; j += G) {
     if (singular) Ob[(long)j * N + i] = zd{0, 0};
-    else Ob[(long)perm[j] * N + mypos] = zmul(X[(long)j * N + i], scale);
+    else Ob[(long)perm[j] * N + mypos] = !SCALED || last ? zmul(X[(long)j * N + i], scale) : X[(long)j * N + i];
   }
 }
 

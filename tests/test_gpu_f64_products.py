@@ -177,3 +177,34 @@ def test_batched_inverse_pivots(require_gpu, N):
             if abs(logd) < 600:
                 det = sign * np.exp(logd)
                 assert abs(ov[w, sp] - det) <= 1e-13 * N * cond * abs(det)
+
+
+@pytest.mark.parametrize("N", [1, 3, 16, 17, 32, 33, 64, 65, 96, 97, 128, 129, 160, 256])
+def test_batched_inverse_mixed_modes(require_gpu, N):
+    """The mixed modes' inverse (pivot rows scaled as they are chosen):
+    determinants in FP64, and G within the FP32 rounding of its operands and
+    of a sum of N products; with interchanges at random and at every step."""
+    say("batched inverse, mixed", N)
+    M, nw = N + 3, 3
+    r = np.random.default_rng(100 + N)
+    s = m.make_system(M, N, 2, density=1.0, sigma_L=0.01, sigma_h=1.0, dt=0.005, seed=N)
+    s.trial_alpha[:] = np.eye(M, N)
+    s.trial_beta[:] = np.eye(M, N)
+    W = 0.1 * (r.standard_normal((nw, 2, M, N)) + 1j * r.standard_normal((nw, 2, M, N)))
+    W[:, 0, :N] += np.eye(N)
+    W[:, 1, :N] += np.eye(N)[::-1]
+    g = m.AfqmcSys(s, nw, "mixed_fp32", dense_exchange=False)
+    g.set(nat.BUF_W, W)
+    g.set(nat.BUF_WDATA, np.zeros((nw, 8), complex))
+    G = g.calculate_mixed_density_matrix().reshape(2, N, M, nw)
+    ov = g.W_data[:, 2:4]
+    g.close()
+    for w in range(nw):
+        for sp in range(2):
+            A = W[w, sp, :N].T
+            inv, cond = np.linalg.inv(A), np.linalg.cond(A)
+            bound = 2 * (2 * N + 4) * 2.0**-24 * (np.abs(inv) @ np.abs(W[w, sp].T))
+            ref = inv @ W[w, sp].T
+            assert np.all(np.abs(G[sp, :, :, w] - ref) <= bound + 1e-14 * N * cond * np.abs(ref).max())
+            det = np.linalg.det(A)
+            assert abs(ov[w, sp] - det) <= 1e-13 * N * cond * abs(det)
