@@ -131,8 +131,11 @@ typedef enum {
    * straight into a ring of LDS stages by 16-byte direct loads, and the
    * others as 1; 1 stages the split-BF16 left operand (and a right one that
    * allows it) by direct loads into two LDS stages; 0 passes every operand
-   * through registers.  All give the same results bit for bit.  May be
-   * changed at any time.  No counterpart in the reference. */
+   * through registers.  All give the same results bit for bit.
+   * AFQMC_MIXED_FP32: 2 runs the products of FP32 operands with k contiguous
+   * and even, and the exchange, through the ring, 1 and 0 through registers
+   * (the same walkers bit for bit; the exchange's sums in another order).
+   * May be changed at any time.  No counterpart in the reference. */
   AFQMC_OPT_DIRECT_LDS = 6,
   /* 0 (default): each GEMM call site runs the tile shape the autotuner
    * (afqmc_tune) or the size heuristic picked; k > 0 forces candidate k of

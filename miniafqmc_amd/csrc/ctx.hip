@@ -416,9 +416,17 @@ bool ring_ok(const afqmc_ctx* c, const ZGemmArgs& a)
          ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.B & 15) == 0 && !a.conjb;
 }
 
+// FP32 operands: whole 16-byte chunks of two complex
+bool ringf_ok(const afqmc_ctx* c, const ZGemmArgs& a)
+{
+  return c->gemm_adma && c->gemm_ring && a.sak == 1 && a.sbk == 1 && a.k > 0 && a.k % 2 == 0 && !a.ktri &&
+         a.sam % 2 == 0 && a.sa1 % 2 == 0 && a.sa2 % 2 == 0 && a.sbn % 2 == 0 && a.sb1 % 2 == 0 && a.sb2 % 2 == 0 &&
+         ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.B & 15) == 0 && !a.conjb;
+}
+
 template <class OT, int NP> int ring_run(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch, int ri)
 {
-  const RingCfg t = NP == 3 ? kRing3[ri] : kRing[ri];
+  const RingCfg t = ring_cfg<NP>(ri);
   a.MT = (a.m + t.BM - 1) / t.BM;
   a.NT = (a.n + t.BN - 1) / t.BN;
   const long tiles = (long)a.MT * a.NT * batch;
@@ -431,9 +439,9 @@ template <int NP> int ring_default(const ZGemmArgs& a, int batch)
 {
   int best = 0;
   double tb = 1e300;
-  for (int i = 0; i < kNRing; i++) {
-    const RingCfg t = NP == 3 ? kRing3[i] : kRing[i];
-    const double rate = NP == 3 ? kRingRate3[i] : kRingRate[i];
+  for (int i = 0; i < ring_count<NP>(); i++) {
+    const RingCfg t = ring_cfg<NP>(i);
+    const double rate = ring_rate<NP>(i);
     const double tiles = (double)((a.m + t.BM - 1) / t.BM) * ((a.n + t.BN - 1) / t.BN) * batch;
     const double percu = std::ceil(tiles / 256.0);
     // four waves alone on a CU leave gaps (eight are two per SIMD)
@@ -451,12 +459,12 @@ template <class OT, int NP = 2> int zgemm_ring(afqmc_ctx* c, const char* name, c
   char keyb[160];
   std::snprintf(keyb, sizeof(keyb), "%s/ring%d/%d/%d/%d/%d", name, NP, a.m, a.n, a.k, batch);
   const std::string key(keyb);
-  if (c->force_cfg > 0 && c->force_cfg <= kNRing) return ring_run<OT, NP>(c, name, a, batch, c->force_cfg - 1);
+  if (c->force_cfg > 0 && c->force_cfg <= ring_count<NP>()) return ring_run<OT, NP>(c, name, a, batch, c->force_cfg - 1);
   auto it = c->tune.find(key);
   if (it != c->tune.end() && !c->tuning) return ring_run<OT, NP>(c, name, a, batch, it->second);
   if (!c->tuning) return ring_run<OT, NP>(c, name, a, batch, ring_default<NP>(a, batch));
   int best = ring_default<NP>(a, batch);
-  RET(tune_tiles(c, kNRing, best, [&](int ri) { return ring_run<OT, NP>(c, name, a, batch, ri); }));
+  RET(tune_tiles(c, ring_count<NP>(), best, [&](int ri) { return ring_run<OT, NP>(c, name, a, batch, ri); }));
   c->tune[key] = best;
   return ring_run<OT, NP>(c, name, a, batch, best);
 }
@@ -592,6 +600,9 @@ int zgemm(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch)
   } else {
   if constexpr (CP == CP_BF16X3 && std::is_same<AT, bfs>::value && std::is_same<BT, bfs>::value && AK && BK) {
     if (ring_ok(c, a)) return zgemm_ring<OT>(c, name, a, batch);
+  }
+  if constexpr (CP == CP_F32 && std::is_same<AT, float>::value && std::is_same<BT, float>::value && AK && BK) {
+    if (ringf_ok(c, a)) return zgemm_ring<OT, 0>(c, name, a, batch);
   }
   char keyb[160];
   std::snprintf(keyb, sizeof(keyb), "%s/%d/%d/%d/%d/%d/%d%d", name, CP, a.m, a.n, a.k, batch, (int)AK, (int)BK);
@@ -1170,10 +1181,10 @@ int do_vhs(afqmc_ctx* c)
   a.n = (int)MM;
   a.k = K;
   if (c->mode == AFQMC_FP64_DENSE) return zgemm<CP_F64, double, double, double, true, false>(c, "vhs_gemm", a, 1);
-  if (c->mode == AFQMC_MIXED_FP32) return zgemm<CP_F32, float, float, float, true, false>(c, "vhs_gemm", a, 1);
-  // split-BF16: Ld stored [M*M][K]
+  // mixed modes: Ld stored [M*M][K]
   a.sbn = K;
   a.sbk = 1;
+  if (c->mode == AFQMC_MIXED_FP32) return zgemm<CP_F32, float, float, float, true, true>(c, "vhs_gemm", a, 1);
   // vHS's third pieces, only when a Horner step of the three-piece
   // propagator reads them (bits 1-6 of the step mask)
   c->vhs3 = c->tp_vHS && (c->three_steps & 0x7E);
@@ -1680,19 +1691,21 @@ int do_ortho(afqmc_ctx* c)
 // which bounds their FP32 accumulation.
 // Measured per energy: 256 orbitals, 256 walkers, three pieces 7.1 -> 2.56 ms
 // (1290 TFLOP/s of MFMA), in FP64 12.4 -> 9.0 ms (61 TFLOP/s); 384 orbitals,
-// 256 walkers, two pieces 15.2 + 1.4 -> 6.6 ms.
+// 256 walkers, two pieces 15.2 + 1.4 -> 6.6 ms; 192 orbitals, 128 walkers, FP32
+// 4.46 -> 0.80 ms.
 constexpr long kF64ExchChunk = 2048;
 
 template <int CP> bool exch_one_ok(const afqmc_ctx* c)
 {
   if (CP == CP_F64) return true;
   const long NM = (long)c->N * c->M;
+  if (CP == CP_F32) return NM % 2 == 0 && c->gemm_adma && c->gemm_ring;
   if (NM % 16) return false;
   return CP == CP_BF16X6 || (CP == CP_BF16X3 && c->gemm_adma && c->gemm_ring);
 }
 
 // G: FP64 [nw][2NM]; Gs (and Gs3): its split forms
-template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const zb* Gs, const uint32_t* Gs3)
+template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const void* Gs, const uint32_t* Gs3)
 {
   const long NM = (long)c->N * c->M, nw = c->nw;
   ExchArgs x;
@@ -1704,19 +1717,20 @@ template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const zb* Gs, const ui
   // workgroups per CU where the smaller tiles give them
   int best = 0;
   double tb = 1e300;
-  constexpr int n = CP == CP_F64 ? kNF64 : kNRing;
+  constexpr int NP = CP == CP_BF16X6 ? 3 : CP == CP_F32 ? 0 : 2;
+  constexpr int n = CP == CP_F64 ? kNF64 : ring_count<NP>();
   constexpr double rate64[] = {57.4, 62.7, 63.9};
   constexpr double rateb[] = {0.86, 1.0, 1.0, 0.9, 0.55};
   auto dims = [&](int i, int& BM, int& BN) {
-    BM = CP == CP_F64 ? kF64[i % kNF64].BM : CP == CP_BF16X6 ? kRing3[i].BM : kRing[i].BM;
-    BN = CP == CP_F64 ? kF64[i % kNF64].BN : CP == CP_BF16X6 ? kRing3[i].BN : kRing[i].BN;
+    BM = CP == CP_F64 ? kF64[i % kNF64].BM : ring_cfg<NP>(i).BM;
+    BN = CP == CP_F64 ? kF64[i % kNF64].BN : ring_cfg<NP>(i).BN;
   };
   for (int i = 0; i < n; i++) {
     int BM, BN;
     dims(i, BM, BN);
     const double tiles = 2.0 * ((nw + BM - 1) / BM) * exch_items(NM, x.xch, BN);
     const double percu = std::ceil(tiles / 256.0);
-    const double t = percu * BM * BN / ((CP == CP_F64 ? rate64[i % kNF64] : rateb[i]) * (percu < 2.0 ? 0.7 : 1.0));
+    const double t = percu * BM * BN / ((CP == CP_F64 ? rate64[i % kNF64] : NP == 0 ? ring_rate<NP>(i) : rateb[i]) * (percu < 2.0 ? 0.7 : 1.0));
     if (t < tb) {
       tb = t;
       best = i;
@@ -1767,7 +1781,7 @@ template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const zb* Gs, const ui
     a.NT = 1;
     a.x = x;
     RET(launch(c, "energy_vx_gemm",
-               [&]() { ring_exch_launch<CP == CP_BF16X6 ? 3 : 2>(c->stream, a, grid, best); }));
+               [&]() { ring_exch_launch<NP>(c->stream, a, grid, best); }));
   }
   return launch(c, "energy_exch_dot", [&]() {
     hipLaunchKernelGGL(exch_sum_kernel, dim3((unsigned)((nw + 15) / 16), 2), dim3(256), 0, c->stream, x.part, x.xt,
@@ -1795,7 +1809,7 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
                                             "energy_v_reduce")));
   }
   bool one = false;
-  if constexpr (std::is_same<GT, double>::value && (CP == CP_F64 || CP == CP_BF16X3 || CP == CP_BF16X6)) {
+  if constexpr (std::is_same<GT, double>::value && (CP == CP_F64 || CP == CP_F32 || CP == CP_BF16X3 || CP == CP_BF16X6)) {
     one = c->Vx && exch_one_ok<CP>(c);
     if (one) {
       if (CP == CP_BF16X3) {
@@ -1804,6 +1818,14 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
         RET(launch(c, "g_split", [&]() {
           hipLaunchKernelGGL((zconvert_kernel<zd, zb>), dim3(nblk(2 * NM * nw, 256)), dim3(256), 0, c->stream,
                              (const zd*)Gp, c->G3, 2 * NM * nw);
+        }));
+      }
+      if (CP == CP_F32) {
+        // G in FP32 (a split complex has as many bytes)
+        if (!c->G3) RET(dalloc(c, &c->G3, 2 * (size_t)NM * nw));
+        RET(launch(c, "g_split", [&]() {
+          hipLaunchKernelGGL((zconvert_kernel<zd, zf>), dim3(nblk(2 * NM * nw, 256)), dim3(256), 0, c->stream,
+                             (const zd*)Gp, (zf*)c->G3, 2 * NM * nw);
         }));
       }
       RET(exch_one<CP>(c, (const zd*)Gp, c->G3, c->G3l));
@@ -2781,15 +2803,16 @@ int afqmc_upload_system(afqmc_ctx* c, const double* trial_alpha, const double* t
       RET(dalloc(c, &Ld32, K * MM));
       RET(dalloc(c, &Lt32, 2 * K * NM));
       RET(launch(c, "convert", [&]() {
+        // Ld is stored transposed, [M*M][K]: the vHS GEMM reads it with k
+        // contiguous and stages it straight into LDS
         if (c->bsplit) {
-          // split-BF16 Ld is stored transposed, [M*M][K]: the vHS GEMM reads
-          // it with k contiguous and stages it straight into LDS
           hipLaunchKernelGGL((ztranspose_kernel<zd, zb>), dim3((unsigned)((MM + 31) / 32), (unsigned)((K + 31) / 32)),
                              dim3(256), 0, st, Ld64, (zb*)Ld32, (int)K, (int)MM, MM, K);
           hipLaunchKernelGGL((zconvert_kernel<zd, zb>), dim3(nblk(2 * K * NM, 256)), dim3(256), 0, st, Lt64,
                              (zb*)Lt32, 2 * K * NM);
         } else {
-          hipLaunchKernelGGL((zconvert_kernel<zd, zf>), dim3(nblk(K * MM, 256)), dim3(256), 0, st, Ld64, Ld32, K * MM);
+          hipLaunchKernelGGL((ztranspose_kernel<zd, zf>), dim3((unsigned)((MM + 31) / 32), (unsigned)((K + 31) / 32)),
+                             dim3(256), 0, st, Ld64, Ld32, (int)K, (int)MM, MM, K);
           hipLaunchKernelGGL((zconvert_kernel<zd, zf>), dim3(nblk(2 * K * NM, 256)), dim3(256), 0, st, Lt64, Lt32,
                              2 * K * NM);
         }

@@ -45,6 +45,16 @@
 //
 // NP = 1 (one piece, 8 significant bits): the same two-piece tiles are staged
 // and only the hi words enter the MFMAs, h*h alone.
+//
+// NP = 0: FP32 operands (zf, as many bytes as a split complex) on
+// v_mfma_f32_16x16x4_f32, in zgemm_kernel's order: per group of four k,
+// ascending, a_re b then a_im (i b).  Bound: the matrix cores (one MFMA takes
+// 32 cycles of its SIMD for 2048 flops); what the register-staged kernel lost
+// was time waiting on memory and on address arithmetic.  k may end anywhere
+// at an even number: a chunk past it is read again from the last one and its
+// fragments are zeroed.  Same bits; 192 orbitals, 128 walkers: HS potential 521
+// -> 259 us (112 TFLOP/s; a large library product reaches 150), bias 207 -> 124,
+// exchange of one energy 4.46 (ten launches and dots) -> 0.80 ms.
 #pragma once
 #include "gemm.hpp"
 
@@ -65,7 +75,8 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 // BM rows x BN complex columns per workgroup, WM x WN waves, STAGES k-tiles
 // of 16 complex in LDS.  OT: output element (double, float, or bfs for split
 // output).  Launch conditions (checked by the host): A and B split-BF16, unit
-// k stride, rows and batch offsets 16-byte aligned, k % 16 == 0, no conj(B);
+// k stride, rows and batch offsets 16-byte aligned, k % 16 == 0 (k % 2 == 0 with
+// NP = 0), no conj(B);
 // NP = 3 also third-piece rows 16-byte aligned.
 // XD: the exchange energy (ExchArgs): the tile's product, rounded to FP32 as
 // the stored form was, is dotted with the FP64 G of the same walkers and rows
@@ -86,7 +97,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
   constexpr int LPT = AL + BL + AL3 + BL3;
   // one stage in uint2 units: the two-piece tiles, then the third pieces
   constexpr int STG = (BM + BN) * KT + (NP == 3 ? (BM + BN) * KT / 2 : 0);
-  static_assert(NP >= 1 && NP <= 3, "one, two or three pieces");
+  static_assert(NP >= 0 && NP <= 3, "FP32 or one, two or three pieces");
   static_assert(NP != 3 || ((BM * C3) % NT == 0 && (BN * C3) % NT == 0), "third-piece tiles must split evenly");
   static_assert(NP != 3 || (WTM % 32 == 0 && WTN % 32 == 0), "third pieces pair 16-row blocks within a wave tile");
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be a multiple of 16");
@@ -171,7 +182,11 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
     pb3[i] = B3 + (long)min(n0 + row3(u), pn - 1) * p.sbn + 4 * chunk3(u);
   }
   const int w0 = __builtin_amdgcn_readfirstlane(wave);
+  // largest k0 whose chunk lies inside (FP32 only; the same chunk of every row
+  // is a thread's, as NT / 8 rows are a multiple of 16)
+  const int klast = kend - 2 - 2 * ((tid & 7) ^ b16::swz(tid >> 3));
   auto issue = [&](uint2* st, int k0) __attribute__((always_inline)) {
+    if constexpr (NP == 0) k0 = min(k0, klast);
 #pragma unroll
     for (int i = 0; i < AL; i++)
       __builtin_amdgcn_global_load_lds((const void*)(pa[i] + k0),
@@ -219,11 +234,53 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
   // loop instead, which keeps the register count of eight-wave tiles within
   // the budget)
   constexpr int TNF = NP == 3 ? 1 : TN;
-  struct Frags {
+  struct FragsB {
     uint4 ah[TM], al[TM], b0[TNF], b1[TNF];
     uint4 a3[NP == 3 ? TM : 1];
   };
-  auto read = [&](const uint2* st, Frags& f) __attribute__((always_inline)) {
+  struct FragsF {
+    zf a[4][TM], b[4][TN];
+  };
+  using Frags = typename std::conditional<NP == 0, FragsF, FragsB>::type;
+  // FP32: lane group g takes k = 4 kq + g
+  auto readf = [&](const uint2* st, int k0, FragsF& f) __attribute__((always_inline)) {
+    const zf* tz = (const zf*)st;
+#pragma unroll
+    for (int kq = 0; kq < 4; kq++) {
+      const int o = 2 * ((2 * kq + (g >> 1)) ^ sw) + (g & 1);
+      const bool in = k0 + 4 * kq + g < kend;
+#pragma unroll
+      for (int i = 0; i < TM; i++) {
+        const zf v = tz[(arow + 16 * i) * KT + o];
+        f.a[kq][i] = zf{in ? v.re : 0.f, in ? v.im : 0.f};
+      }
+#pragma unroll
+      for (int j = 0; j < TN; j++) {
+        const zf v = tz[(brow + 16 * j) * KT + o];
+        f.b[kq][j] = zf{in ? v.re : 0.f, in ? v.im : 0.f};
+      }
+    }
+  };
+  auto mfmasf = [&](const FragsF& f) __attribute__((always_inline)) {
+#pragma unroll
+    for (int kq = 0; kq < 4; kq++) {
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          cr[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[kq][i].re, f.b[kq][j].re, cr[i][j], 0, 0, 0);
+          ci[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[kq][i].re, f.b[kq][j].im, ci[i][j], 0, 0, 0);
+        }
+#pragma unroll
+      for (int i = 0; i < TM; i++)
+#pragma unroll
+        for (int j = 0; j < TN; j++) {
+          cr[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[kq][i].im, -f.b[kq][j].im, cr[i][j], 0, 0, 0);
+          ci[i][j] = __builtin_amdgcn_mfma_f32_16x16x4f32(f.a[kq][i].im, f.b[kq][j].re, ci[i][j], 0, 0, 0);
+        }
+    }
+  };
+  auto read = [&](const uint2* st, FragsB& f) __attribute__((always_inline)) {
     const uint4* t4 = (const uint4*)st;  // 8 uint4 per tile row
 #pragma unroll
     for (int i = 0; i < TM; i++) {
@@ -248,7 +305,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
       for (int i = 0; i < TM; i++) f.a3[i] = t3[(arow3 + 16 * (i >> 1)) * 8 + ((i & 1) ? c1 : c0)];
     }
   };
-  auto mfmas = [&](const Frags& f, const uint2* st) __attribute__((always_inline)) {
+  auto mfmas = [&](const FragsB& f, const uint2* st) __attribute__((always_inline)) {
     // real part: (b_re, -b_im); imaginary part: (b_im, b_re)
     auto ng = [](uint32_t w) { return w ^ 0x80000000u; };
     auto rt = [](uint32_t w) { return __builtin_amdgcn_alignbit(w, w, 16u); };
@@ -331,10 +388,14 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
       // a bare barrier: a workgroup fence here would wait for the later
       // tiles' loads too
       __builtin_amdgcn_s_barrier();
-      read(cs, f);
+      if constexpr (NP == 0) readf(cs, c * KT, f);
+      else read(cs, f);
     }
     if (j < nk) issue(in_, j * KT);
-    if (c >= 0) mfmas(f, cs);
+    if (c >= 0) {
+      if constexpr (NP == 0) mfmasf(f);
+      else mfmas(f, cs);
+    }
   };
   for (int j = 0; j < nk + STAGES - 1; j += STAGES) {
     step(std::integral_constant<int, 0>(), j);

@@ -29,6 +29,19 @@ constexpr int kNRing = 5;
 // and the propagator products at 256 to 512 orbitals
 constexpr double kRingRate[] = {0.87, 1.0, 1.0, 1.02, 0.85};
 constexpr double kRingRate3[] = {0.95, 1.0, 1.0, 0.92, 0.93};
+// FP32 operands, small tiles: three to five workgroups a CU cover each other's
+// barriers (HS potential at 300 orbitals, 128 walkers, 1200 vectors: 111, 117
+// and 111 TFLOP/s; 128 x 64 and 128 x 128 with eight waves 110 and 104, a third
+// stage of 64 x 64 or a fourth of 32 x 32 no gain)
+constexpr RingCfg kRingF[] = {{32, 32, 2, 2, 3}, {64, 64, 2, 2, 2}, {64, 32, 2, 2, 3}};
+constexpr int kNRingF = 3;
+constexpr double kRingRateF[] = {0.95, 1.0, 0.95};
+template <int NP> constexpr int ring_count() { return NP == 0 ? kNRingF : kNRing; }
+template <int NP> constexpr RingCfg ring_cfg(int i) { return NP == 0 ? kRingF[i] : NP == 3 ? kRing3[i] : kRing[i]; }
+template <int NP> constexpr double ring_rate(int i)
+{
+  return NP == 0 ? kRingRateF[i] : NP == 3 ? kRingRate3[i] : kRingRate[i];
+}
 
 // FP64 products (zgemm_f64_kernel): every operand order, tile candidates
 // (rows, complex columns, waves, LDS stages).

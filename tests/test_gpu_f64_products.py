@@ -179,6 +179,31 @@ def test_batched_inverse_pivots(require_gpu, N):
                 assert abs(ov[w, sp] - det) <= 1e-13 * N * cond * abs(det)
 
 
+@pytest.mark.parametrize("M,N,K,nw", [(8, 2, 4, 1), (50, 7, 62, 5), (51, 6, 62, 5), (64, 16, 100, 33),
+                                      (90, 30, 150, 128), (200, 40, 134, 70)])
+def test_f32_ring_matches_register_staged(require_gpu, M, N, K, nw):
+    """FP32 products by direct LDS loads (every tile) against the kernel that
+    stages through registers: the walkers are the same bits after two substeps
+    (k that is no multiple of a k-tile, odd M), the energy terms, whose
+    exchange is summed in another order, agree to FP64 rounding."""
+    say("f32 ring", M, N, K, nw)
+    s = m.make_system(M, N, K, density=0.5, sigma_L=0.03, sigma_h=1.0, dt=0.005, seed=7)
+    x = m.fields_block(5, K, nw, 0, 2)
+    got = []
+    for direct, tile in ((0, 0), (2, 0), (2, 1), (2, 2), (2, 3)):
+        g = m.AfqmcSys(s, nw, "mixed_fp32")
+        nat.check(nat.lib.afqmc_set_option(g.ctx, nat.OPT_DIRECT_LDS, float(direct)))
+        g.set_tile(tile)
+        g.init_walkers()
+        g.stage_fields(x)
+        g.run(1, 2, 1, s.dt)
+        got.append((g.W, g.energy_terms()))
+        g.close()
+    for W, e in got[1:]:
+        assert np.array_equal(W, got[0][0])
+        assert np.abs(e - got[0][1]).max() <= 1e-14 * np.abs(got[0][1]).max()
+
+
 @pytest.mark.parametrize("N", [1, 3, 16, 17, 32, 33, 64, 65, 96, 97, 128, 129, 160, 256])
 def test_batched_inverse_mixed_modes(require_gpu, N):
     """The mixed modes' inverse (pivot rows scaled as they are chosen):
