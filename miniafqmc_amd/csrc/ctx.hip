@@ -12,6 +12,7 @@
 //     Lt [2][K][N*M] (spin-major).
 #include "afqmc_hip.h"
 #include "common.hpp"
+#include "download.hpp"
 #include "gemm_launch.hpp"
 #include "kernels.hpp"
 #include "prop_small.hpp"
@@ -178,6 +179,7 @@ struct afqmc_ctx {
   bool gemm_adma = true;           // split-BF16 GEMMs stage A by direct global -> LDS loads
   bool gemm_ring = true;           // ... and both operands through a ring of LDS stages where they allow
   long graph_gen = 0;              // bumped whenever captured substeps become stale
+  hipEvent_t pin_ev[dl::kSlots] = {};  // of the chunks of a download
   long exch_chunk = 2048;          // dense exchange: columns per accumulation chunk (0: one pass)
   zd* oU = nullptr;   // [2nw][N][N] R^{-1}
   zd* oX = nullptr;   // [2][2nw][M][N] the two Cholesky QR passes
@@ -251,6 +253,81 @@ void dfree(afqmc_ctx* c, void* p)
   auto it = std::find(c->allocs.begin(), c->allocs.end(), p);
   if (it != c->allocs.end()) c->allocs.erase(it);
   (void)hipFree(p);
+}
+
+// bytes of device memory to host memory, complete on return (download.hpp).
+// Less than 64 KB, and destinations that the runtime knows (pinned, device),
+// take its copy.
+int download(afqmc_ctx* c, void* host, const void* dev, size_t bytes)
+{
+  auto plain = [&]() -> int {
+    HIPCHK(c, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, c->stream));
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    return AFQMC_OK;
+  };
+  if (bytes < (64u << 10)) return plain();
+  hipPointerAttribute_t at;
+  if (hipPointerGetAttributes(&at, host) != hipSuccess) (void)hipGetLastError();
+  else if (at.type != hipMemoryTypeUnregistered) return plain();
+  for (auto& e : c->pin_ev)
+    if (!e) HIPCHK(c, hipEventCreateWithFlags(&e, hipEventDisableTiming));
+  // the stream's work first, so that no thread waits for it
+  HIPCHK(c, hipStreamSynchronize(c->stream));
+  auto j = std::make_shared<dl::Job>();
+  j->host = (char*)host;
+  j->bytes = bytes;
+  j->parts = std::min<size_t>(8, (bytes + 8 * dl::kPart - 1) / (8 * dl::kPart));
+  j->chunk = j->parts * dl::kPart;
+  j->n = (bytes + j->chunk - 1) / j->chunk;
+  j->slots = std::min<size_t>(j->n, dl::kSlots);
+  j->helpers = bytes < (1u << 20) ? 0 : bytes < (24u << 20) ? 3 : 7;
+  for (auto& d : j->done) d = 0;
+  const dl::Ring ring = dl::pool().take(j->slots * j->chunk);
+  if (!ring.p) return plain();
+  j->pin = ring.p;
+  if (j->helpers) dl::pool().add(j);
+  hipError_t err = hipSuccess;
+  size_t sent = 0, landed = 0;
+  auto copied = [&](size_t ch) {  // out of the slot, up to and including chunk ch
+    return j->done[ch % j->slots].load(std::memory_order_acquire) >= (ch / j->slots + 1) * j->parts;
+  };
+  while (!j->exhausted()) {
+    while (sent < j->n && (sent < j->slots || copied(sent - j->slots)) && err == hipSuccess) {
+      const size_t s = sent % j->slots, o = sent * j->chunk;
+      hipLaunchKernelGGL(copy_out_kernel, dim3(256), dim3(256), 0, c->stream, (const char*)dev + o,
+                         ring.d + s * j->chunk, std::min(j->chunk, bytes - o));
+      err = hipGetLastError();
+      if (err == hipSuccess) err = hipEventRecord(c->pin_ev[s], c->stream);
+      sent++;
+    }
+    if (err != hipSuccess) break;
+    if (landed < sent) {
+      // wait for the next chunk only when there is nothing to copy
+      const hipEvent_t ev = c->pin_ev[landed % j->slots];
+      err = j->step() ? hipEventQuery(ev) : hipEventSynchronize(ev);
+      if (err == hipSuccess) j->ready.store(++landed, std::memory_order_release);
+      else if (err == hipErrorNotReady) {
+        (void)hipGetLastError();
+        err = hipSuccess;
+      }
+      if (err != hipSuccess) break;
+    } else if (!j->step()) {
+      std::this_thread::yield();
+    }
+  }
+  // no part is taken any more; wait for those that were
+  const size_t taken = std::min(j->next.exchange(j->n * j->parts), j->n * j->parts);
+  if (j->helpers) dl::pool().remove(j);
+  for (;;) {
+    size_t d = 0;
+    for (auto& q : j->done) d += q.load(std::memory_order_acquire);
+    if (d >= taken) break;
+    std::this_thread::yield();
+  }
+  if (err != hipSuccess) (void)hipStreamSynchronize(c->stream);
+  dl::pool().give(ring);
+  if (err != hipSuccess) return fail(c, AFQMC_ERR_HIP, std::string("download: ") + hipGetErrorString(err));
+  return AFQMC_OK;
 }
 
 hipEvent_t get_event(afqmc_ctx* c)
@@ -2328,6 +2405,7 @@ int afqmc_ctx_create(int nmo, int naea, int nchol, int nwalk, int mode, afqmc_ct
     delete c;
     return AFQMC_ERR_HIP;
   }
+  dl::pool().user(1);  // until afqmc_ctx_destroy
   const long M = nmo, N = naea, K = nchol, nw = nwalk;
   const long MN = M * N, MM = M * M;
   const size_t zs = c->mixed ? sizeof(zf) : sizeof(zd);
@@ -2385,8 +2463,11 @@ int afqmc_ctx_destroy(afqmc_ctx* c)
     (void)hipEventDestroy(p.b);
   }
   for (auto e : c->evpool) (void)hipEventDestroy(e);
+  for (auto e : c->pin_ev)
+    if (e) (void)hipEventDestroy(e);
   for (void* p : c->allocs) (void)hipFree(p);
   if (c->stream) (void)hipStreamDestroy(c->stream);
+  dl::pool().user(-1);
   delete c;
   return AFQMC_OK;
 }
@@ -2886,8 +2967,8 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
   const long MN = M * N, MM = M * M, NAK = 2 * MN;
   hipStream_t st = c->stream;
   auto raw = [&](void* dev, size_t bytes) -> int {
-    if (to_device) HIPCHK(c, hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st));
-    else HIPCHK(c, hipMemcpyAsync(host, dev, bytes, hipMemcpyDeviceToHost, st));
+    if (!to_device) return download(c, host, dev, bytes);
+    HIPCHK(c, hipMemcpyAsync(dev, host, bytes, hipMemcpyHostToDevice, st));
     HIPCHK(c, hipStreamSynchronize(st));
     return AFQMC_OK;
   };
@@ -2921,10 +3002,8 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
     } else {
       if (is32) {
         t32.resize(tmp.size());
-        HIPCHK(c, hipMemcpyAsync(t32.data(), dev, sizeof(zf) * t32.size(), hipMemcpyDeviceToHost, st));
-        if (!t3.empty())
-          HIPCHK(c, hipMemcpyAsync(t3.data(), dev3, sizeof(uint32_t) * t3.size(), hipMemcpyDeviceToHost, st));
-        HIPCHK(c, hipStreamSynchronize(st));
+        RET(download(c, t32.data(), dev, sizeof(zf) * t32.size()));
+        if (!t3.empty()) RET(download(c, t3.data(), dev3, sizeof(uint32_t) * t3.size()));
         for (size_t i = 0; i < tmp.size(); i++) {
           if (c->bsplit) {
             uint32_t w[2];
@@ -2939,8 +3018,7 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
           }
         }
       } else {
-        HIPCHK(c, hipMemcpyAsync(tmp.data(), dev, sizeof(zd) * tmp.size(), hipMemcpyDeviceToHost, st));
-        HIPCHK(c, hipStreamSynchronize(st));
+        RET(download(c, tmp.data(), dev, sizeof(zd) * tmp.size()));
       }
       htranspose(tmp.data(), (zd*)host, nw, R);
     }

@@ -486,6 +486,16 @@ __global__ __launch_bounds__(1024) void gj_inverse_global_kernel(const zd* __res
   }
 }
 
+// n bytes of device memory (16-byte aligned) to mapped host memory: the
+// downloads' copy (the runtime's takes a copy engine, whose first use by a
+// stream can cost 8 ms).
+__global__ __launch_bounds__(256) void copy_out_kernel(const char* __restrict__ in, char* __restrict__ out, size_t n)
+{
+  const size_t n16 = n / 16, i0 = blockIdx.x * (size_t)256 + threadIdx.x;
+  for (size_t i = i0; i < n16; i += gridDim.x * (size_t)256) ((uint4*)out)[i] = ((const uint4*)in)[i];
+  if (i0 < n % 16) out[n16 * 16 + i0] = in[n16 * 16 + i0];
+}
+
 // Three-piece split-BF16 of n complex values: (h, m) to hm (a zb per
 // element; may alias the input when IT is zf, each element being read before
 // its slot is written by the same thread) and the third pieces to l.
