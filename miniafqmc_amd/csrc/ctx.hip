@@ -59,6 +59,11 @@ struct afqmc_ctx {
   // system
   zd* trial = nullptr;   // [2][M][N] conj(Psi)
   zd* propg = nullptr;   // [M][M]
+  // row lengths of the split-BF16 operands with k contiguous, in elements: X,
+  // Ld [..][ldk], propg32, vHS and the propagator's terms [..][ldm].  Odd M
+  // (beyond the one-kernel propagator) and K are padded to pairs, the direct
+  // loads' 16 bytes; the pad is never used.  Other modes: M and K.
+  int ldm = 0, ldk = 0;
   void* propg32 = nullptr; // [M][M] in the contraction format (mixed: zf, or zb when split)
   zd* haj = nullptr;     // [2N][M]
   int* sp_rp = nullptr;
@@ -488,8 +493,8 @@ template <int CP> int default_cfg(const ZGemmArgs& a)
 
 bool ring_ok(const afqmc_ctx* c, const ZGemmArgs& a)
 {
-  return c->gemm_adma && c->gemm_ring && a.sak == 1 && a.sbk == 1 && a.k % 16 == 0 && a.sam % 2 == 0 &&
-         a.sa1 % 2 == 0 && a.sa2 % 2 == 0 && a.sbn % 2 == 0 && a.sb1 % 2 == 0 && a.sb2 % 2 == 0 &&
+  return c->gemm_adma && c->gemm_ring && a.sak == 1 && a.sbk == 1 && a.k > 0 && (a.k % 2 == 0 || a.kpad) &&
+         a.sam % 2 == 0 && a.sa1 % 2 == 0 && a.sa2 % 2 == 0 && a.sbn % 2 == 0 && a.sb1 % 2 == 0 && a.sb2 % 2 == 0 &&
          ((uintptr_t)a.A & 15) == 0 && ((uintptr_t)a.B & 15) == 0 && !a.conjb;
 }
 
@@ -676,7 +681,10 @@ int zgemm(afqmc_ctx* c, const char* name, ZGemmArgs a, int batch)
     return zgemm_ring<OT, 1>(c, name, a, batch);
   } else {
   if constexpr (CP == CP_BF16X3 && std::is_same<AT, bfs>::value && std::is_same<BT, bfs>::value && AK && BK) {
-    if (ring_ok(c, a)) return zgemm_ring<OT>(c, name, a, batch);
+    // whole k-tiles need no masks; sums that end inside one take the form that
+    // masks its rest (its own figures: gemm_b16.hpp)
+    if (ring_ok(c, a))
+      return a.k % 16 ? zgemm_ring<OT, 4>(c, name, a, batch) : zgemm_ring<OT, 2>(c, name, a, batch);
   }
   if constexpr (CP == CP_F32 && std::is_same<AT, float>::value && std::is_same<BT, float>::value && AK && BK) {
     if (ringf_ok(c, a)) return zgemm_ring<OT, 0>(c, name, a, batch);
@@ -1012,30 +1020,6 @@ int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, 
   const long tiles = ((nw + 127) / 128) * ((K + 63) / 64);
   int S = 1;
   while (S < 16 && 2 * S * tiles < 2048 && NM % (2 * S) == 0 && (NM / (2 * S)) % 64 == 0) S *= 2;
-  if (S == 1) {
-    for (int sp = 0; sp < 2; sp++) {
-      ZGemmArgs a = gargs();
-      a.A = zadv<GT>(Gp, sp * NM);
-      a.sam = 2 * NM;
-      a.sak = 1;
-      a.B = zadv<LT_>(Lt, sp * K * NM);
-      a.sbn = NM;
-      a.sbk = 1;
-      a.C = out;
-      a.scm = K;
-      a.scn = 1;
-      a.m = (int)nw;
-      a.n = (int)K;
-      a.k = (int)NM;
-      a.br = sp == 0 ? 0.0 : 1.0;
-      if (G3) {
-        a.A3 = G3 + sp * NM;
-        a.B3 = Lt3 + sp * K * NM;
-      }
-      RET((zgemm<CP, GT, LT_, double, true, true>(c, name, a, 1)));
-    }
-    return AFQMC_OK;
-  }
   // partials in FP32 for the FP32/BF16 contractions, FP64 otherwise
   using PT = typename std::conditional<CP == CP_F64, double, float>::type;
   using PZ = typename ztype<PT>::type;
@@ -1208,13 +1192,13 @@ int do_fields(afqmc_ctx* c, const double* xdev, long substep, const long* xslice
   return launch(c, "fields", [&]() {
     if (!c->mixed)
       hipLaunchKernelGGL((fields_wfirst_kernel<zd, zd>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
-                         (zd*)c->X, c->hybridW, c->flags + 1, (uint32_t*)nullptr, pre);
+                         (zd*)c->X, c->hybridW, c->flags + 1, (uint32_t*)nullptr, pre, K);
     else if (c->bsplit)
       hipLaunchKernelGGL((fields_wfirst_kernel<zb, zf>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
-                         (zb*)c->X, c->hybridW, c->flags + 1, c->tp_X, pre);
+                         (zb*)c->X, c->hybridW, c->flags + 1, c->tp_X, pre, c->ldk);
     else
       hipLaunchKernelGGL((fields_wfirst_kernel<zf, zf>), dim3(nw), dim3(256), 0, c->stream, K, nw, c->vbias, src,
-                         (zf*)c->X, c->hybridW, c->flags + 1, (uint32_t*)nullptr, pre);
+                         (zf*)c->X, c->hybridW, c->flags + 1, (uint32_t*)nullptr, pre, K);
   });
 }
 
@@ -1262,6 +1246,11 @@ int do_vhs(afqmc_ctx* c)
   a.sbn = K;
   a.sbk = 1;
   if (c->mode == AFQMC_MIXED_FP32) return zgemm<CP_F32, float, float, float, true, true>(c, "vhs_gemm", a, 1);
+  // split rows padded to pairs (ldk, ldm)
+  a.sam = a.sbn = c->ldk;
+  a.kpad = 1;
+  a.n = c->M * c->ldm;
+  a.scm = a.n;
   // vHS's third pieces, only when a Horner step of the three-piece
   // propagator reads them (bits 1-6 of the step mask)
   c->vhs3 = c->tp_vHS && (c->three_steps & 0x7E);
@@ -1353,7 +1342,7 @@ template <int CP, class ST, class TT, class PT, class VT>
 int propagate_chain(afqmc_ctx* c, const void* P, const void* V)
 {
   const int M = c->M, N = c->N, nw = c->nw;
-  const long MN = (long)M * N, MM = (long)M * M;
+  const long MN = (long)M * N;
   auto base = [&]() {
     ZGemmArgs a = gargs();
     a.sam = M;
@@ -1376,6 +1365,7 @@ int propagate_chain(afqmc_ctx* c, const void* P, const void* V)
   {
     ZGemmArgs a = base();
     a.A = P;
+    a.sam = c->ldm;
     a.B = c->W;
     a.C = c->S;
     RET((zgemm<CP, PT, double, ST, true, false>(c, "prop_pw", a, 2 * nw)));
@@ -1388,7 +1378,8 @@ int propagate_chain(afqmc_ctx* c, const void* P, const void* V)
   for (int k = 6; k >= 1; k--) {
     ZGemmArgs a = base();
     a.A = V;
-    a.sa1 = MM;
+    a.sam = c->ldm;
+    a.sa1 = (long)M * c->ldm;
     a.sa2 = 0;
     a.B = prev;
     if (k < 6) {  // U_{k+1} transposed; U_7 = S row-major
@@ -1412,6 +1403,7 @@ int propagate_chain(afqmc_ctx* c, const void* P, const void* V)
   {
     ZGemmArgs a = base();
     a.A = P;
+    a.sam = c->ldm;
     a.B = prev;
     a.sbn = M;
     a.sbk = 1;
@@ -1437,7 +1429,7 @@ int propagate_chain(afqmc_ctx* c, const void* P, const void* V)
 int propagate_split(afqmc_ctx* c)
 {
   const int M = c->M, N = c->N, nw = c->nw;
-  const long MN = (long)M * N, MM = (long)M * M;
+  const long MN = (long)M * N, ldm = c->ldm;
   const dim3 tgrid((unsigned)((N + 31) / 32), (unsigned)((M + 31) / 32), (unsigned)(2 * nw));
   const bool opt3 = (c->three & 4) != 0;
   // product j in launch order: 0 P W, 7-k the Horner step k, 7 P U
@@ -1448,25 +1440,27 @@ int propagate_split(afqmc_ctx* c)
   RET(launch(c, "prop_split_w", [&]() {
     if (opt3)
       hipLaunchKernelGGL((transpose_split_kernel<zd, true>), tgrid, dim3(256), 0, c->stream, (const zd*)c->W, Tb,
-                         c->tp_Tb, M, N);
+                         c->tp_Tb, M, N, ldm);
     else
       hipLaunchKernelGGL((transpose_split_kernel<zd, false>), tgrid, dim3(256), 0, c->stream, (const zd*)c->W, Tb,
-                         (uint32_t*)nullptr, M, N);
+                         (uint32_t*)nullptr, M, N, ldm);
   }));
-  // m = M rows against n columns of M (terms [column][M])
+  // m = M rows against n columns of M (terms [column][ldm], ldm: M padded to
+  // pairs)
   auto base = [&](int n) {
     ZGemmArgs a = gargs();
     a.A = c->propg32;
     a.A3 = c->tp_P;
-    a.sam = M;
+    a.sam = ldm;
     a.sak = 1;
-    a.sbn = M;
+    a.sbn = ldm;
     a.sbk = 1;
     a.m = M;
     a.n = n;
     a.k = M;
+    a.kpad = 1;
     a.scm = 1;
-    a.scn = M;
+    a.scn = ldm;
     return a;
   };
   {  // S = P W: U_7 = S split (third pieces when U_6's product takes three)
@@ -1489,9 +1483,9 @@ int propagate_split(afqmc_ctx* c)
     ZGemmArgs a = base(2 * N);
     a.A = c->vHS;
     a.A3 = c->tp_vHS;
-    a.sa1 = MM;
-    a.sb1 = 2 * MN;
-    a.sc1 = 2 * MN;
+    a.sa1 = M * ldm;
+    a.sb1 = 2 * N * ldm;
+    a.sc1 = 2 * N * ldm;
     a.B = prev;
     a.B3 = prev3;
     a.C = bufs[k & 1];
@@ -1521,8 +1515,8 @@ int propagate_split(afqmc_ctx* c)
   }
   // the register-staged kernel (AFQMC_OPT_DIRECT_LDS below 2) takes a batch
   a.n = N;
-  a.sb1 = 2 * MN;
-  a.sb2 = MN;
+  a.sb1 = 2 * N * ldm;
+  a.sb2 = N * ldm;
   a.sc1 = 2 * MN;
   a.sc2 = MN;
   a.bdiv = 2;
@@ -1581,7 +1575,7 @@ int do_propagate(afqmc_ctx* c)
   if (c->mode == AFQMC_FP64_DENSE) return propagate_f64(c, (const zd*)c->vHS);
   if (c->mode == AFQMC_MIXED_FP32)
     return propagate_chain<CP_F32, float, float, float, float>(c, c->propg32, c->vHS);
-  if (c->gemm_adma && c->gemm_ring && c->M % 16 == 0) return propagate_split(c);
+  if (c->gemm_adma && c->gemm_ring && c->ldm % 2 == 0) return propagate_split(c);
   return propagate_chain<CP_BF16X3, float, bfs, bfs, bfs>(c, c->propg32, c->vHS);
 }
 
@@ -1777,8 +1771,8 @@ template <int CP> bool exch_one_ok(const afqmc_ctx* c)
   if (CP == CP_F64) return true;
   const long NM = (long)c->N * c->M;
   if (CP == CP_F32) return NM % 2 == 0 && c->gemm_adma && c->gemm_ring;
-  if (NM % 16) return false;
-  return CP == CP_BF16X6 || (CP == CP_BF16X3 && c->gemm_adma && c->gemm_ring);
+  if (CP == CP_BF16X6) return NM % 16 == 0;
+  return CP == CP_BF16X3 && NM % 2 == 0 && c->exch_chunk % 2 == 0 && c->gemm_adma && c->gemm_ring;
 }
 
 // G: FP64 [nw][2NM]; Gs (and Gs3): its split forms
@@ -1795,7 +1789,7 @@ template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const void* Gs, const 
   int best = 0;
   double tb = 1e300;
   constexpr int NP = CP == CP_BF16X6 ? 3 : CP == CP_F32 ? 0 : 2;
-  constexpr int n = CP == CP_F64 ? kNF64 : ring_count<NP>();
+  constexpr int n = CP == CP_F64 ? kNF64 : NP == 0 ? ring_count<NP>() : kNExch;
   constexpr double rate64[] = {57.4, 62.7, 63.9};
   constexpr double rateb[] = {0.86, 1.0, 1.0, 0.9, 0.55};
   auto dims = [&](int i, int& BM, int& BN) {
@@ -1858,7 +1852,13 @@ template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const void* Gs, const 
     a.NT = 1;
     a.x = x;
     RET(launch(c, "energy_vx_gemm",
-               [&]() { ring_exch_launch<NP>(c->stream, a, grid, best); }));
+               [&]() {
+                 // chunks or the block ending inside a k-tile mask its rest
+                 if constexpr (NP == 2) {
+                   if ((NM | x.xch) % 16) return ring_exch_launch<4>(c->stream, a, grid, best);
+                 }
+                 ring_exch_launch<NP>(c->stream, a, grid, best);
+               }));
   }
   return launch(c, "energy_exch_dot", [&]() {
     hipLaunchKernelGGL(exch_sum_kernel, dim3((unsigned)((nw + 15) / 16), 2), dim3(256), 0, c->stream, x.part, x.xt,
@@ -2395,6 +2395,8 @@ int afqmc_ctx_create(int nmo, int naea, int nchol, int nwalk, int mode, afqmc_ct
   c->mode = mode;
   c->mixed = (mode == AFQMC_MIXED_FP32 || mode == AFQMC_MIXED_BF16);
   c->bsplit = (mode == AFQMC_MIXED_BF16);
+  c->ldm = c->bsplit && nmo > PS_MMAX ? nmo + (nmo & 1) : nmo;
+  c->ldk = c->bsplit ? nchol + (nchol & 1) : nchol;
   if (hipStreamCreateWithFlags(&c->stream, hipStreamNonBlocking) != hipSuccess) {
     delete c;
     return AFQMC_ERR_HIP;
@@ -2421,13 +2423,13 @@ int afqmc_ctx_create(int nmo, int naea, int nchol, int nwalk, int mode, afqmc_ct
   chk(dalloc(c, &c->Wl, nw * 4));
   chk(dalloc_bytes(c, &c->G, nw * 2 * MN * zs));
   chk(dalloc(c, &c->vbias, nw * K));
-  chk(dalloc_bytes(c, &c->X, nw * K * zs));
-  chk(dalloc_bytes(c, &c->vHS, nw * MM * zs));
+  chk(dalloc_bytes(c, &c->X, nw * c->ldk * zs));
+  chk(dalloc_bytes(c, &c->vHS, nw * M * c->ldm * zs));
   if (mode == AFQMC_FP64_CSR) chk(dalloc(c, &c->vHSw, nw * MM));
   chk(dalloc(c, &c->hybridW, nw));
-  chk(dalloc_bytes(c, &c->S, nw * 2 * MN * zs));
-  chk(dalloc_bytes(c, &c->Ta, nw * 2 * MN * zs));
-  chk(dalloc_bytes(c, &c->Tb, nw * 2 * MN * zs));
+  chk(dalloc_bytes(c, &c->S, nw * 2 * N * c->ldm * zs));
+  chk(dalloc_bytes(c, &c->Ta, nw * 2 * N * c->ldm * zs));
+  chk(dalloc_bytes(c, &c->Tb, nw * 2 * N * c->ldm * zs));
   chk(dalloc(c, &c->eshift, 1));
   chk(dalloc(c, &c->flags, 4));
   chk(dalloc(c, &c->e_direct, nw));
@@ -2603,11 +2605,11 @@ int afqmc_upload_system(afqmc_ctx* c, const double* trial_alpha, const double* t
   HIPCHK(c, hipMemcpyAsync(c->propg, propg1, sizeof(zd) * MM, hipMemcpyHostToDevice, st));
   HIPCHK(c, hipMemcpyAsync(c->haj, haj, sizeof(zd) * 2 * NM, hipMemcpyHostToDevice, st));
   if (c->mixed) {
-    RET(dalloc_bytes(c, &c->propg32, sizeof(zf) * MM));
+    RET(dalloc_bytes(c, &c->propg32, sizeof(zf) * M * c->ldm));
     RET(launch(c, "convert", [&]() {
       if (c->bsplit)
         hipLaunchKernelGGL((zconvert_kernel<zd, zb>), dim3(nblk(MM, 256)), dim3(256), 0, st, c->propg,
-                           (zb*)c->propg32, MM);
+                           (zb*)c->propg32, MM, (long)M, (long)c->ldm);
       else
         hipLaunchKernelGGL((zconvert_kernel<zd, zf>), dim3(nblk(MM, 256)), dim3(256), 0, st, c->propg,
                            (zf*)c->propg32, MM);
@@ -2881,14 +2883,16 @@ int afqmc_upload_system(afqmc_ctx* c, const double* trial_alpha, const double* t
     if (c->mixed) {
       zf* Ld32 = nullptr;
       zf* Lt32 = nullptr;
-      RET(dalloc(c, &Ld32, K * MM));
+      RET(dalloc(c, &Ld32, (long)c->ldk * M * c->ldm));
       RET(dalloc(c, &Lt32, 2 * K * NM));
       RET(launch(c, "convert", [&]() {
         // Ld is stored transposed, [M*M][K]: the vHS GEMM reads it with k
         // contiguous and stages it straight into LDS
         if (c->bsplit) {
+          if (c->ldm != M) (void)hipMemsetAsync(Ld32, 0, sizeof(zf) * c->ldk * M * c->ldm, st);  // the pad rows
           hipLaunchKernelGGL((ztranspose_kernel<zd, zb>), dim3((unsigned)((MM + 31) / 32), (unsigned)((K + 31) / 32)),
-                             dim3(256), 0, st, Ld64, (zb*)Ld32, (int)K, (int)MM, MM, K);
+                             dim3(256), 0, st, Ld64, (zb*)Ld32, (int)K, (int)MM, MM, (long)c->ldk,
+                             (int)M, c->ldm);
           hipLaunchKernelGGL((zconvert_kernel<zd, zb>), dim3(nblk(2 * K * NM, 256)), dim3(256), 0, st, Lt64,
                              (zb*)Lt32, 2 * K * NM);
         } else {
@@ -2973,23 +2977,26 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
     return AFQMC_OK;
   };
   // walker-last reference [R][nw] <-> walker-first device [nw][R] of type
-  // zd/zf/zb, with the third pieces in dev3 when the buffer has them
-  auto wlast = [&](void* dev, long R, bool is32, uint32_t* dev3 = nullptr) -> int {
+  // zd/zf/zb, with the third pieces in dev3 when the buffer has them; split
+  // rows of L elements may take Lp on the device (no third pieces then)
+  auto wlast = [&](void* dev, long R, bool is32, uint32_t* dev3 = nullptr, long L = 1, long Lp = 1) -> int {
     std::vector<zd> tmp((size_t)R * nw);
     std::vector<zf> t32;
+    const size_t nd = tmp.size() / L * Lp;
+    auto at = [&](size_t i) { return L == Lp ? i : i / L * Lp + i % L; };
     std::vector<uint32_t> t3(dev3 && c->bsplit ? tmp.size() : 0);
     if (to_device) {
       htranspose((const zd*)host, tmp.data(), R, nw);
       if (is32) {
-        t32.resize(tmp.size());
+        t32.assign(nd, zf{0.f, 0.f});
         for (size_t i = 0; i < tmp.size(); i++) {
           if (c->bsplit) {
             uint32_t w[2];
             host_split(tmp[i].re, tmp[i].im, w);
-            std::memcpy(&t32[i], w, sizeof(w));
+            std::memcpy(&t32[at(i)], w, sizeof(w));
             if (!t3.empty()) t3[i] = host_third(tmp[i].re, tmp[i].im, w);
           } else {
-            t32[i] = zf{(float)tmp[i].re, (float)tmp[i].im};
+            t32[at(i)] = zf{(float)tmp[i].re, (float)tmp[i].im};
           }
         }
         HIPCHK(c, hipMemcpyAsync(dev, t32.data(), sizeof(zf) * t32.size(), hipMemcpyHostToDevice, st));
@@ -3001,20 +3008,20 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
       HIPCHK(c, hipStreamSynchronize(st));
     } else {
       if (is32) {
-        t32.resize(tmp.size());
+        t32.resize(nd);
         RET(download(c, t32.data(), dev, sizeof(zf) * t32.size()));
         if (!t3.empty()) RET(download(c, t3.data(), dev3, sizeof(uint32_t) * t3.size()));
         for (size_t i = 0; i < tmp.size(); i++) {
           if (c->bsplit) {
             uint32_t w[2];
-            std::memcpy(w, &t32[i], sizeof(w));
+            std::memcpy(w, &t32[at(i)], sizeof(w));
             tmp[i] = host_merge(w);
             if (!t3.empty()) {
               tmp[i].re += (double)host_bf2f((uint16_t)(t3[i] & 0xffff));
               tmp[i].im += (double)host_bf2f((uint16_t)(t3[i] >> 16));
             }
           } else {
-            tmp[i] = zd{t32[i].re, t32[i].im};
+            tmp[i] = zd{t32[at(i)].re, t32[at(i)].im};
           }
         }
       } else {
@@ -3040,12 +3047,12 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
   case AFQMC_BUF_HYBRIDW: return raw(c->hybridW, sizeof(zd) * nw);
   case AFQMC_BUF_G: return g_wfirst(c) ? wlast(c->G, NAK, c->mixed, c->tp_G) : raw(c->G, sizeof(zd) * NAK * nw);
   case AFQMC_BUF_VBIAS: return d ? wlast(c->vbias, K, false) : raw(c->vbias, sizeof(zd) * K * nw);
-  case AFQMC_BUF_X: return d ? wlast(c->X, K, c->mixed, c->tp_X) : raw(c->X, sizeof(zd) * K * nw);
+  case AFQMC_BUF_X: return d ? wlast(c->X, K, c->mixed, c->tp_X, K, c->ldk) : raw(c->X, sizeof(zd) * K * nw);
   case AFQMC_BUF_VHS:
     if (d) {
       // an upload writes the third pieces; a read adds them only when the
       // last HS potential wrote them
-      RET(wlast(c->vHS, MM, c->mixed, (to_device || c->vhs3) ? c->tp_vHS : nullptr));
+      RET(wlast(c->vHS, MM, c->mixed, (to_device || c->vhs3) ? c->tp_vHS : nullptr, M, c->ldm));
       if (to_device) c->vhs3 = c->tp_vHS != nullptr;
       return AFQMC_OK;
     }

@@ -67,6 +67,9 @@ struct ZGemmArgs {
   // when cni is nonzero (columns of several batch items side by side)
   int cni;
   long scno;
+  // split-BF16 rows are padded to an even number of elements: an odd k may
+  // be read in pairs (the pad is never used)
+  int kpad;
   // XD mode of zgemm_b16dma_kernel: A, B at the spin and chunk (0, 0), m walkers
   ExchArgs x;
 };

@@ -55,6 +55,17 @@
 // fragments are zeroed.  Same bits; 192 orbitals, 128 walkers: HS potential 521
 // -> 259 us (112 TFLOP/s; a large library product reaches 150), bias 207 -> 124,
 // exchange of one energy 4.46 (ten launches and dots) -> 0.80 ms.
+//
+// NP = 4: two pieces with k ending anywhere.  Rows hold a whole number of
+// 16-byte chunks (k even, or odd rows padded to pairs); a chunk past the end is
+// read again from the last one, and in the last k-tile the words past it are
+// masked to zero, so pads and repeated chunks never enter a sum and the bits are
+// the register-staged kernel's, which took these sizes before and is bound by
+// its round trip through registers.  A form of its own, so that whole k-tiles
+// pay neither the per-lane chunk limit nor the masks.  Whole passes (orbitals /
+// electrons / vectors, walkers): 147 / 36 / 336, 90 6.37 -> 2.41 ms; 211 / 52 /
+// 501, 380 28.2 -> 15.3; 303 / 84 / 1002, 69 12.4 -> 3.37; 231 / 57 / 843, 433
+// 25.1 -> 20.3 (N M odd: the bias and the exchange stay on the other kernel).
 #pragma once
 #include "gemm.hpp"
 
@@ -75,8 +86,8 @@ __device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1
 // BM rows x BN complex columns per workgroup, WM x WN waves, STAGES k-tiles
 // of 16 complex in LDS.  OT: output element (double, float, or bfs for split
 // output).  Launch conditions (checked by the host): A and B split-BF16, unit
-// k stride, rows and batch offsets 16-byte aligned, k % 16 == 0 (k % 2 == 0 with
-// NP = 0), no conj(B);
+// k stride, rows and batch offsets 16-byte aligned, k % 16 == 0 (NP = 0 and 4:
+// k % 2 == 0 or rows padded to pairs), no conj(B);
 // NP = 3 also third-piece rows 16-byte aligned.
 // XD: the exchange energy (ExchArgs): the tile's product, rounded to FP32 as
 // the stored form was, is dotted with the FP64 G of the same walkers and rows
@@ -97,7 +108,8 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
   constexpr int LPT = AL + BL + AL3 + BL3;
   // one stage in uint2 units: the two-piece tiles, then the third pieces
   constexpr int STG = (BM + BN) * KT + (NP == 3 ? (BM + BN) * KT / 2 : 0);
-  static_assert(NP >= 0 && NP <= 3, "FP32 or one, two or three pieces");
+  static_assert(NP >= 0 && NP <= 4, "FP32, one, two or three pieces, two with any k");
+  constexpr bool ANYK = NP == 0 || NP == 4;
   static_assert(NP != 3 || ((BM * C3) % NT == 0 && (BN * C3) % NT == 0), "third-piece tiles must split evenly");
   static_assert(NP != 3 || (WTM % 32 == 0 && WTN % 32 == 0), "third pieces pair 16-row blocks within a wave tile");
   static_assert(WTM % 16 == 0 && WTN % 16 == 0, "wave tile must be a multiple of 16");
@@ -182,11 +194,11 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
     pb3[i] = B3 + (long)min(n0 + row3(u), pn - 1) * p.sbn + 4 * chunk3(u);
   }
   const int w0 = __builtin_amdgcn_readfirstlane(wave);
-  // largest k0 whose chunk lies inside (FP32 only; the same chunk of every row
+  // largest k0 whose chunk of two starts inside (the same chunk of every row
   // is a thread's, as NT / 8 rows are a multiple of 16)
-  const int klast = kend - 2 - 2 * ((tid & 7) ^ b16::swz(tid >> 3));
+  const int klast = ((kend - 1) & ~1) - 2 * ((tid & 7) ^ b16::swz(tid >> 3));
   auto issue = [&](uint2* st, int k0) __attribute__((always_inline)) {
-    if constexpr (NP == 0) k0 = min(k0, klast);
+    if constexpr (ANYK) k0 = min(k0, klast);
 #pragma unroll
     for (int i = 0; i < AL; i++)
       __builtin_amdgcn_global_load_lds((const void*)(pa[i] + k0),
@@ -280,7 +292,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
         }
     }
   };
-  auto read = [&](const uint2* st, FragsB& f) __attribute__((always_inline)) {
+  auto read = [&](const uint2* st, int k0, FragsB& f) __attribute__((always_inline)) {
     const uint4* t4 = (const uint4*)st;  // 8 uint4 per tile row
 #pragma unroll
     for (int i = 0; i < TM; i++) {
@@ -304,6 +316,22 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
 #pragma unroll
       for (int i = 0; i < TM; i++) f.a3[i] = t3[(arow3 + 16 * (i >> 1)) * 8 + ((i & 1) ? c1 : c0)];
     }
+    if constexpr (NP == 4) {
+      if (k0 + KT > kend) {  // the last tile: k = k0 + 4g + t past the end count as zero
+        const int kl = kend - k0 - 4 * g;
+        const uint32_t z0 = kl > 0 ? ~0u : 0u, z1 = kl > 1 ? ~0u : 0u, z2 = kl > 2 ? ~0u : 0u, z3 = kl > 3 ? ~0u : 0u;
+#pragma unroll
+        for (int i = 0; i < TM; i++) {
+          f.ah[i] = make_uint4(f.ah[i].x & z0, f.ah[i].y & z1, f.ah[i].z & z2, f.ah[i].w & z3);
+          f.al[i] = make_uint4(f.al[i].x & z0, f.al[i].y & z1, f.al[i].z & z2, f.al[i].w & z3);
+        }
+#pragma unroll
+        for (int j = 0; j < TNF; j++) {
+          f.b0[j] = make_uint4(f.b0[j].x & z0, f.b0[j].y & z0, f.b0[j].z & z1, f.b0[j].w & z1);
+          f.b1[j] = make_uint4(f.b1[j].x & z2, f.b1[j].y & z2, f.b1[j].z & z3, f.b1[j].w & z3);
+        }
+      }
+    }
   };
   auto mfmas = [&](const FragsB& f, const uint2* st) __attribute__((always_inline)) {
     // real part: (b_re, -b_im); imaginary part: (b_im, b_re)
@@ -324,7 +352,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
         const uint4 ih = make_uint4(rt(v0.x), rt(v0.z), rt(v1.x), rt(v1.z));
 #pragma unroll
         for (int i = 0; i < TM; i++) mm(i, j, f.ah[i], rh, ih);
-      } else if constexpr (NP == 2) {
+      } else if constexpr (NP == 2 || NP == 4) {
         const uint4 rh = make_uint4(ng(v0.x), ng(v0.z), ng(v1.x), ng(v1.z));
         const uint4 rl = make_uint4(ng(v0.y), ng(v0.w), ng(v1.y), ng(v1.w));
         const uint4 ih = make_uint4(rt(v0.x), rt(v0.z), rt(v1.x), rt(v1.z));
@@ -389,7 +417,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
       // tiles' loads too
       __builtin_amdgcn_s_barrier();
       if constexpr (NP == 0) readf(cs, c * KT, f);
-      else read(cs, f);
+      else read(cs, c * KT, f);
     }
     if (j < nk) issue(in_, j * KT);
     if (c >= 0) {

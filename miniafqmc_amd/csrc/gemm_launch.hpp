@@ -20,14 +20,16 @@ struct RingCfg {
   int BM, BN, WM, WN, S;
 };
 constexpr RingCfg kRing[] = {
-    {128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {256, 128, 4, 2, 3}, {64, 64, 2, 2, 2}};
+    {128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {256, 128, 4, 2, 3}, {64, 64, 2, 2, 2}, {32, 32, 2, 2, 4}};
 // three-piece operands take half as much LDS again per stage
 constexpr RingCfg kRing3[] = {
     {128, 128, 2, 2, 2}, {256, 128, 4, 2, 2}, {128, 256, 2, 4, 2}, {128, 128, 2, 2, 3}, {64, 64, 2, 2, 2}};
-constexpr int kNRing = 5;
+constexpr int kNRing = 6, kNRing3 = 5, kNExch = 5;
 // relative rates with the chip full, by pieces: the HS potential, the bias
 // and the propagator products at 256 to 512 orbitals
-constexpr double kRingRate[] = {0.87, 1.0, 1.0, 1.02, 0.85};
+// (the last tile is for long sums over few outputs, which leave most CUs idle
+// in 64 x 64 tiles: its rate lets it win where those fill half the chip or less)
+constexpr double kRingRate[] = {0.87, 1.0, 1.0, 1.02, 0.85, 0.42};
 constexpr double kRingRate3[] = {0.95, 1.0, 1.0, 0.92, 0.93};
 // FP32 operands, small tiles: three to five workgroups a CU cover each other's
 // barriers (HS potential at 300 orbitals, 128 walkers, 1200 vectors: 111, 117
@@ -36,7 +38,7 @@ constexpr double kRingRate3[] = {0.95, 1.0, 1.0, 0.92, 0.93};
 constexpr RingCfg kRingF[] = {{32, 32, 2, 2, 3}, {64, 64, 2, 2, 2}, {64, 32, 2, 2, 3}};
 constexpr int kNRingF = 3;
 constexpr double kRingRateF[] = {0.95, 1.0, 0.95};
-template <int NP> constexpr int ring_count() { return NP == 0 ? kNRingF : kNRing; }
+template <int NP> constexpr int ring_count() { return NP == 0 ? kNRingF : NP == 3 ? kNRing3 : kNRing; }
 template <int NP> constexpr RingCfg ring_cfg(int i) { return NP == 0 ? kRingF[i] : NP == 3 ? kRing3[i] : kRing[i]; }
 template <int NP> constexpr double ring_rate(int i)
 {

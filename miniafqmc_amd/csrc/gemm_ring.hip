@@ -20,6 +20,9 @@ template <class OT, int NP, bool XD> void ring_go(hipStream_t st, const ZGemmArg
   case 4:
     if constexpr (4 < ring_count<NP>()) return go(std::integral_constant<int, 4>());
     break;
+  case 5:
+    if constexpr (5 < ring_count<NP>() && !XD) return go(std::integral_constant<int, 5>());
+    break;
   }
   go(std::integral_constant<int, 0>());
 }
@@ -35,6 +38,7 @@ template <int NP> void ring_exch_launch(hipStream_t st, const ZGemmArgs& a, unsi
 }
 template void ring_exch_launch<0>(hipStream_t, const ZGemmArgs&, unsigned, int);
 template void ring_exch_launch<2>(hipStream_t, const ZGemmArgs&, unsigned, int);
+template void ring_exch_launch<4>(hipStream_t, const ZGemmArgs&, unsigned, int);
 template void ring_exch_launch<3>(hipStream_t, const ZGemmArgs&, unsigned, int);
 
 #define RING_LAUNCH(OT, NP) template void ring_launch<OT, NP>(hipStream_t, const ZGemmArgs&, unsigned, int);
@@ -44,6 +48,9 @@ RING_LAUNCH(bfs, 1)
 RING_LAUNCH(bfs, 2)
 RING_LAUNCH(float, 2)
 RING_LAUNCH(double, 2)
+RING_LAUNCH(bfs, 4)
+RING_LAUNCH(float, 4)
+RING_LAUNCH(double, 4)
 RING_LAUNCH(bfs, 3)
 RING_LAUNCH(float, 3)
 RING_LAUNCH(double, 3)

@@ -530,11 +530,11 @@ __global__ void third_piece_kernel(const zd* __restrict__ src, const zb* __restr
 }
 
 // Batched transpose into split-BF16: in [b][R][C] (row stride C, item stride
-// R*C) -> out [b][C][R] (zb), with P3 as three pieces (the third ones to
+// R*C) -> out [b][C][ldo] (zb), with P3 as three pieces (the third ones to
 // out3), per 32 x 32 tile through LDS; grid (C/32, R/32, b).
 template <class IT, bool P3>
 __global__ __launch_bounds__(256) void transpose_split_kernel(const IT* __restrict__ in, zb* __restrict__ out,
-                                                               uint32_t* __restrict__ out3, int R, int C)
+                                                               uint32_t* __restrict__ out3, int R, int C, long ldo)
 {
   __shared__ zd tile[32][33];
   const long item = (long)blockIdx.z * R * C;
@@ -549,7 +549,7 @@ __global__ __launch_bounds__(256) void transpose_split_kernel(const IT* __restri
     const int cc = bx + yy, rr = by + tx;
     if (rr < R && cc < C) {
       const zd v = tile[tx][yy];
-      const long o = item + (long)cc * R + rr;
+      const long o = ((long)blockIdx.z * C + cc) * ldo + rr;
       if constexpr (P3) split3_z(v.re, v.im, out[o], out3[o]);
       else out[o] = split_z((float)v.re, (float)v.im);
     }
@@ -763,10 +763,11 @@ __global__ __launch_bounds__(1024) void csrmm_win_kernel(int nrows, int nw, int 
 
 // ---------------------------------------------------------------------------
 // Tiled transpose of complex matrices: out[c][r] = in[r][c], in is R x Cc.
-// Output precision OT (double or float pairs).
+// Output precision OT (double or float pairs).  With ci, row c of the output
+// goes to row (c / ci) * co + c % ci.
 template <class IT, class OT>
 __global__ __launch_bounds__(256) void ztranspose_kernel(const IT* __restrict__ in, OT* __restrict__ out, int R,
-                                                         int Cc, long ldi, long ldo)
+                                                         int Cc, long ldi, long ldo, int ci = 0, int co = 0)
 {
   __shared__ zd tile[32][33];
   const int bx = blockIdx.x * 32, by = blockIdx.y * 32;
@@ -781,21 +782,22 @@ __global__ __launch_bounds__(256) void ztranspose_kernel(const IT* __restrict__ 
     if (rr < R && cc < Cc) {
       OT o;
       from_zd(tile[tx][yy], o);
-      out[(long)cc * ldo + rr] = o;
+      out[(ci ? (long)(cc / ci) * co + cc % ci : (long)cc) * ldo + rr] = o;
     }
   }
 }
 
-// elementwise precision conversion / copy of n complex values
+// elementwise precision conversion / copy of n complex values, rows of li
+// to rows lo apart where these differ
 template <class IT, class OT>
-__global__ void zconvert_kernel(const IT* __restrict__ in, OT* __restrict__ out, long n)
+__global__ void zconvert_kernel(const IT* __restrict__ in, OT* __restrict__ out, long n, long li = 0, long lo = 0)
 {
   long i = (long)blockIdx.x * blockDim.x + threadIdx.x;
   long st = (long)gridDim.x * blockDim.x;
   for (; i < n; i += st) {
     OT o;
     from_zd(to_zd(in[i]), o);
-    out[i] = o;
+    out[li != lo ? i / li * lo + i % li : i] = o;
   }
 }
 
@@ -929,14 +931,14 @@ template <class PZ> __device__ inline zd field_bias(const FieldPre& p, zd* vb, l
   return a;
 }
 
-// Walker-first layouts (vbias, X [nw][K]): one workgroup per walker, the
+// Walker-first layouts (vbias [nw][K], X [nw][ldk]): one workgroup per walker, the
 // lanes along n (coalesced), each thread a pair (2j, 2j+1) of draws at a
 // time; fixed-order block reduction of hybridW.
 template <class XT, class PZ>
 __global__ __launch_bounds__(256) void fields_wfirst_kernel(int K, int nw, zd* __restrict__ vb, FieldSrc src,
                                                             XT* __restrict__ X, zd* __restrict__ hybridW,
                                                             int* __restrict__ nonfinite, uint32_t* __restrict__ X3,
-                                                            FieldPre pre)
+                                                            FieldPre pre, int ldk)
 {
   __shared__ zd part[4];
   const int w = blockIdx.x;
@@ -944,7 +946,7 @@ __global__ __launch_bounds__(256) void fields_wfirst_kernel(int K, int nw, zd* _
   const long sub = src.xslice ? *src.xslice : src.substep;
   const double* x = src.x ? src.x + (src.xslice ? sub * (long)K * nw : 0L) : nullptr;
   const long tot = (long)nw * K, o0 = (long)w * K;
-  XT* Xw = X + (long)w * K;
+  XT* Xw = X + (long)w * ldk;
   uint32_t* X3w = X3 ? X3 + (long)w * K : nullptr;
   if (pre.Wd && threadIdx.x == 0) field_pre_save(pre, w);
   // split X with its third pieces (three-piece split-BF16), else as XT
