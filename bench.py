@@ -85,20 +85,9 @@ def csr_flops(name, nw, nnz_spvn, nnz_spvnT):
 
 def contraction_spins_per_launch(M, N, K, nw, mode=None):
     """Spin blocks per launch of the bias-shaped contraction (G against the
-    K Cholesky rows, the bias and the Coulomb term).  In FP64 one launch
-    covers both spins from N*M = 512 on.  Otherwise the library splits its
-    k = N*M range into S chunks, S doubling from 1 while 2*S*tiles < 2048
-    (tiles = ceil(nw/128) * ceil(K/64)) and N*M/(2S) stays a multiple of 64;
-    with S > 1 one launch covers both spins, otherwise each spin is its own
-    launch."""
-    NM = N * M
-    if mode == "fp64_dense":
-        return 2 if NM >= 512 else 1
-    tiles = -(-nw // 128) * -(-K // 64)
-    S = 1
-    while S < 16 and 2 * S * tiles < 2048 and NM % (2 * S) == 0 and (NM // (2 * S)) % 64 == 0:
-        S *= 2
-    return 2 if S > 1 else 1
+    K Cholesky rows, the bias and the Coulomb term): both, as batch items,
+    however the sum over N*M is split."""
+    return 2
 
 
 def kernel_flops(name, M, N, K, nw, mode=None):
