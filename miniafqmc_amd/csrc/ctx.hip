@@ -44,6 +44,12 @@ struct EvPair {
   int count;
 };
 
+// a device buffer that grows to the largest size asked for (need_work)
+struct Work {
+  void* p = nullptr;
+  size_t bytes = 0;
+};
+
 } // namespace
 
 struct afqmc_ctx {
@@ -174,10 +180,12 @@ struct afqmc_ctx {
   int one_steps = 0;
   bool allow_vx = true;
   zd* Gtmp = nullptr;     // FP64 G [nw][2NM] for the energy (CSR: transposed; mixed: FP64 copy)
-  void* vws = nullptr;    // split-k partials of the bias contraction
+  // split-k partials of the bias contraction; captured substeps hold its
+  // address, so it is theirs alone and growing it drops them
+  Work vws;
   int vws_pending = 0;    // slices there that the next fields kernel sums into vbias
+  Work ews;               // partial sums of the energy (never captured)
   double* xtmp = nullptr; // draws passed to afqmc_fields, [K][nw] (allocated at the first such call)
-  size_t vws_bytes = 0;
   // orthogonalisation: Cholesky QR scratch (allocated at the first call)
   bool ortho_householder = false;  // always use the blocked Householder kernel
   bool fused_prop = false;         // split-BF16 propagator in one kernel when the shapes allow
@@ -944,13 +952,21 @@ int do_overlaps(afqmc_ctx* c)
   return AFQMC_OK;
 }
 
-// A workspace of at least `bytes` for the partial sums of split contractions.
-int need_vws(afqmc_ctx* c, size_t bytes)
+void drop_graphs(afqmc_ctx* c);
+
+// Workspace w with at least `bytes`.  Captured substeps (the context's and
+// those of groups) read and write vws at the address it had: they are dropped
+// before it moves.
+int need_work(afqmc_ctx* c, Work& w, size_t bytes)
 {
-  if (c->vws_bytes >= bytes) return AFQMC_OK;
-  dfree(c, c->vws);
-  c->vws_bytes = bytes;
-  return dalloc_bytes(c, &c->vws, bytes);
+  if (w.bytes >= bytes) return AFQMC_OK;
+  if (&w == &c->vws) {
+    HIPCHK(c, hipStreamSynchronize(c->stream));
+    drop_graphs(c);
+  }
+  dfree(c, w.p);
+  w.bytes = bytes;
+  return dalloc_bytes(c, &w.p, bytes);
 }
 
 // Chunks of a k sum of length kt whose output is m x n: enough 64 x 64 tiles
@@ -968,13 +984,13 @@ long f64_chunk(long m, long n, long kt, int items, int smax)
 // products (spin, chunk of j) run as one batch into a workspace, summed in
 // chunk order.  (200 walkers, 999 vectors, N M = 15250: 12.6 ms unsplit in
 // 32 workgroups per spin.)
-int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const char* name, const char* rname,
-                       bool defer)
+int dense_contract_f64(afqmc_ctx* c, Work& ws, const zd* G, const zd* Lt, zd* out, const char* name,
+                       const char* rname, bool defer)
 {
   const long NM = (long)c->N * c->M, nw = c->nw, K = c->K;
   const long chunk = f64_chunk(nw, K, NM, 2, 16);
   const int S = (int)((NM + chunk - 1) / chunk);
-  RET(need_vws(c, sizeof(zd) * 2 * S * nw * K));
+  RET(need_work(c, ws, sizeof(zd) * 2 * S * nw * K));
   F64Args a = f64args((int)nw, (int)K, (int)chunk);
   a.ktot = NM;
   a.A = G;  // batch (spin, chunk)
@@ -987,7 +1003,7 @@ int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const c
   a.sbk = 1;
   a.sb1 = K * NM;
   a.sb2 = chunk;
-  a.C = c->vws;
+  a.C = ws.p;
   a.scm = K;
   a.scn = 1;
   a.sc1 = S * nw * K;
@@ -999,7 +1015,7 @@ int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const c
     return AFQMC_OK;
   }
   return launch(c, rname, [&]() {
-    hipLaunchKernelGGL((zsum_slices_kernel<zd>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const zd*)c->vws,
+    hipLaunchKernelGGL((zsum_slices_kernel<zd>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const zd*)ws.p,
                        out, nw * K, 2 * S);
   });
 }
@@ -1009,13 +1025,13 @@ int dense_contract_f64(afqmc_ctx* c, const zd* G, const zd* Lt, zd* out, const c
 // the 2S partial products (spin, chunk) run as one batched GEMM into a
 // workspace and are then summed in FP64.
 template <int CP, class GT, class LT_>
-int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, const char* name,
+int dense_contract_vbias(afqmc_ctx* c, Work& ws, const void* Gp, const void* Lt, zd* out, const char* name,
                          const uint32_t* G3 = nullptr, const uint32_t* Lt3 = nullptr,
                          const char* rname = "vbias_reduce", bool defer = false)
 {
   const long NM = (long)c->N * c->M, nw = c->nw, K = c->K;
   if constexpr (CP == CP_F64) {
-    if (NM >= 512) return dense_contract_f64(c, (const zd*)Gp, (const zd*)Lt, out, name, rname, defer);
+    if (NM >= 512) return dense_contract_f64(c, ws, (const zd*)Gp, (const zd*)Lt, out, name, rname, defer);
   }
   const long tiles = ((nw + 127) / 128) * ((K + 63) / 64);
   int S = 1;
@@ -1023,7 +1039,7 @@ int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, 
   // partials in FP32 for the FP32/BF16 contractions, FP64 otherwise
   using PT = typename std::conditional<CP == CP_F64, double, float>::type;
   using PZ = typename ztype<PT>::type;
-  RET(need_vws(c, sizeof(PZ) * 2 * S * nw * K));
+  RET(need_work(c, ws, sizeof(PZ) * 2 * S * nw * K));
   const long chunk = NM / S;
   ZGemmArgs a = gargs();
   a.A = Gp;  // batch b = (spin, chunk): A offset spin*NM + chunk*NM/S
@@ -1036,7 +1052,7 @@ int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, 
   a.sbk = 1;
   a.sb1 = K * NM;
   a.sb2 = chunk;
-  a.C = c->vws;
+  a.C = ws.p;
   a.scm = K;
   a.scn = 1;
   a.sc1 = S * nw * K;
@@ -1053,7 +1069,7 @@ int dense_contract_vbias(afqmc_ctx* c, const void* Gp, const void* Lt, zd* out, 
     return AFQMC_OK;
   }
   return launch(c, rname, [&]() {
-    hipLaunchKernelGGL((zsum_slices_kernel<PZ>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const PZ*)c->vws, out,
+    hipLaunchKernelGGL((zsum_slices_kernel<PZ>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const PZ*)ws.p, out,
                        nw * K, 2 * S);
   });
 }
@@ -1129,8 +1145,8 @@ int dense_csr_vbias(afqmc_ctx* c, bool defer)
     a.C = c->vbias;
     return zgemm64<zd>(c, "vbias_gemm", a, 1);
   }
-  RET(need_vws(c, sizeof(zd) * S * K * nw));
-  a.C = c->vws;
+  RET(need_work(c, c->vws, sizeof(zd) * S * K * nw));
+  a.C = c->vws.p;
   a.sc2 = K * nw;
   RET(zgemm64<zd>(c, "vbias_gemm", a, S));
   if (defer) {
@@ -1138,7 +1154,7 @@ int dense_csr_vbias(afqmc_ctx* c, bool defer)
     return AFQMC_OK;
   }
   return launch(c, "vbias_reduce", [&]() {
-    hipLaunchKernelGGL((zsum_slices_kernel<zd>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const zd*)c->vws,
+    hipLaunchKernelGGL((zsum_slices_kernel<zd>), dim3(nblk(nw * K, 256)), dim3(256), 0, c->stream, (const zd*)c->vws.p,
                        c->vbias, nw * K, S);
   });
 }
@@ -1156,15 +1172,15 @@ int do_vbias(afqmc_ctx* c, bool defer = false)
                    (long)nw, c->vbias, (long)nw, one, zero, true);
   }
   if (c->mode == AFQMC_FP64_DENSE)
-    return dense_contract_vbias<CP_F64, double, double>(c, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
-                                                        defer);
+    return dense_contract_vbias<CP_F64, double, double>(c, c->vws, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr,
+                                                        nullptr, rn, defer);
   if (c->mode == AFQMC_MIXED_FP32)
-    return dense_contract_vbias<CP_F32, float, float>(c, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
-                                                      defer);
+    return dense_contract_vbias<CP_F32, float, float>(c, c->vws, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr,
+                                                      rn, defer);
   if (c->three & 1)
-    return dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, c->G, c->Lt, c->vbias, "vbias_gemm", c->tp_G, c->tp_Lt, rn,
-                                                     defer);
-  return dense_contract_vbias<CP_BF16X3, bfs, bfs>(c, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
+    return dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, c->vws, c->G, c->Lt, c->vbias, "vbias_gemm", c->tp_G, c->tp_Lt,
+                                                     rn, defer);
+  return dense_contract_vbias<CP_BF16X3, bfs, bfs>(c, c->vws, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
                                                    defer);
 }
 
@@ -1176,7 +1192,7 @@ int do_fields(afqmc_ctx* c, const double* xdev, long substep, const long* xslice
 {
   const int nw = c->nw, K = c->K;
   FieldSrc src{xdev, xslice, substep, c->field_seed};
-  pre.slices = c->vws;
+  pre.slices = c->vws.p;
   pre.ns = c->vws_pending;
   c->vws_pending = 0;
   if (c->mode == AFQMC_FP64_CSR)
@@ -1879,10 +1895,10 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
   // direct term: v(w,n) = sum Lt G ; direct = sum_n v^2 / dt
   if constexpr (CPV == CP_BF16X6) {
     // three pieces of the split G (built for the exchange) and of Lt
-    RET((dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, c->G3, Lv, c->e_v, "energy_v_gemm", c->G3l, c->tp_Lt,
+    RET((dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, c->ews, c->G3, Lv, c->e_v, "energy_v_gemm", c->G3l, c->tp_Lt,
                                                    "energy_v_reduce")));
   } else {
-    RET((dense_contract_vbias<CPV, GT, LVT>(c, Gp, Lv, c->e_v, "energy_v_gemm", nullptr, nullptr,
+    RET((dense_contract_vbias<CPV, GT, LVT>(c, c->ews, Gp, Lv, c->e_v, "energy_v_gemm", nullptr, nullptr,
                                             "energy_v_reduce")));
   }
   bool one = false;
@@ -2013,11 +2029,11 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     }
     // partials per walker-spin: enough workgroups for eight per CU
     const int ngrp = (int)std::max<long>(1, std::min<long>(cnt, 2048 / (2L * nw)));
-    RET(need_vws(c, sizeof(zd) * (size_t)ngrp * 2 * nw));
+    RET(need_work(c, c->ews, sizeof(zd) * (size_t)ngrp * 2 * nw));
     RET(launch(c, "energy_trace", [&]() {
       hipLaunchKernelGGL((trace_sq_kernel<typename ztype<YT>::type>), dim3(2 * nw, ngrp), dim3(256), 0, c->stream,
-                         (const typename ztype<YT>::type*)c->Ybuf, N, cnt, (long)cnt * per_item, (zd*)c->vws, ngrp);
-      hipLaunchKernelGGL(add_parts_kernel, dim3((2 * nw + 255) / 256), dim3(256), 0, c->stream, (const zd*)c->vws,
+                         (const typename ztype<YT>::type*)c->Ybuf, N, cnt, (long)cnt * per_item, (zd*)c->ews.p, ngrp);
+      hipLaunchKernelGGL(add_parts_kernel, dim3((2 * nw + 255) / 256), dim3(256), 0, c->stream, (const zd*)c->ews.p,
                          ngrp, c->e_exch_part, 2 * nw);
     }));
   }
@@ -2125,7 +2141,7 @@ int do_energy(afqmc_ctx* c, double* eav_out)
       const long chunk = f64_chunk(nw, NAK, NAK, 1, 16);
       const int S = (int)((NAK + chunk - 1) / chunk);
       const long gsw = g_wfirst(c) ? NAK : 1, gsi = g_wfirst(c) ? 1 : nw;
-      RET(need_vws(c, sizeof(zd) * (size_t)S * nw * NAK));
+      RET(need_work(c, c->ews, sizeof(zd) * (size_t)S * nw * NAK));
       F64Args a = f64args(nw, (int)NAK, (int)chunk);
       a.ktot = NAK;
       a.bdiv = S;
@@ -2137,14 +2153,14 @@ int do_energy(afqmc_ctx* c, double* eav_out)
       a.sbn = NAK;
       a.sbk = 1;
       a.sb2 = chunk;
-      a.C = c->vws;
+      a.C = c->ews.p;
       a.scm = NAK;
       a.scn = 1;
       a.sc2 = nw * NAK;
       RET(zgemm64<zd>(c, "energy_y_gemm", a, S));
       RET(launch(c, "energy_assemble", [&]() {
         hipLaunchKernelGGL(energy_vakbl_dense_kernel, dim3(nw), dim3(512), 0, c->stream, (int)NAK, nw,
-                           (const zd*)c->G, gsw, gsi, (const zd*)c->vws, S, (const zd*)c->haj, c->e_direct, c->e_exch,
+                           (const zd*)c->G, gsw, gsi, (const zd*)c->ews.p, S, (const zd*)c->haj, c->e_direct, c->e_exch,
                            c->e_one, c->Wd);
       }));
     } else if (c->v_rp) {
@@ -2360,13 +2376,8 @@ int capture_prep(afqmc_ctx* c, int ortho)
   if (!c->transposed && !c->Gfull) RET(dalloc(c, &c->Gfull, 2L * c->M * c->M * c->nw));
   if (c->mode != AFQMC_FP64_CSR || c->sptd) {
     // the bias contraction's split-k workspace at its largest (at most 32
-    // chunks, also for the dense copy of SpvnT)
-    const size_t need = sizeof(zd) * 32 * (size_t)c->nw * c->K;
-    if (c->vws_bytes < need) {
-      dfree(c, c->vws);
-      c->vws_bytes = need;
-      RET(dalloc_bytes(c, &c->vws, need));
-    }
+    // chunks, also for the dense copy of SpvnT); nothing else uses it
+    RET(need_work(c, c->vws, sizeof(zd) * 32 * (size_t)c->nw * c->K));
   }
   if (!c->t1inv_valid) RET(do_overlaps(c));
   HIPCHK(c, hipStreamSynchronize(c->stream));
