@@ -17,6 +17,7 @@
 #include "kernels.hpp"
 #include "prop_small.hpp"
 #include "propagate.hpp"
+#include "workspace.hpp"
 
 #include <dlfcn.h>
 
@@ -42,12 +43,6 @@ struct EvPair {
   std::string name;
   hipEvent_t a, b;
   int count;
-};
-
-// a device buffer that grows to the largest size asked for (need_work)
-struct Work {
-  void* p = nullptr;
-  size_t bytes = 0;
 };
 
 } // namespace
@@ -148,8 +143,7 @@ struct afqmc_ctx {
   zd* e_exch_part = nullptr;  // [nw][2]
   zd* e_one = nullptr;
   zd* e_v = nullptr;      // [nw][K] direct-term contractions
-  void* Ybuf = nullptr;
-  size_t ybuf_bytes = 0;
+  Work ybuf;              // exchange: Y of a few vectors, Z [nw][NM] or the partials of the one-launch form
   // same-spin exchange block of Vakbl, dense [2][NM][NM] (scaled by dt), in
   // the contraction precision; null when it does not fit in device memory
   void* Vx = nullptr;
@@ -959,14 +953,15 @@ void drop_graphs(afqmc_ctx* c);
 // before it moves.
 int need_work(afqmc_ctx* c, Work& w, size_t bytes)
 {
-  if (w.bytes >= bytes) return AFQMC_OK;
-  if (&w == &c->vws) {
-    HIPCHK(c, hipStreamSynchronize(c->stream));
-    drop_graphs(c);
-  }
-  dfree(c, w.p);
-  w.bytes = bytes;
-  return dalloc_bytes(c, &w.p, bytes);
+  return work_grow(
+      w, bytes,
+      [&]() -> int {
+        if (&w != &c->vws) return AFQMC_OK;
+        HIPCHK(c, hipStreamSynchronize(c->stream));
+        drop_graphs(c);
+        return AFQMC_OK;
+      },
+      [&](void** p, size_t n) { return dalloc_bytes(c, p, n); }, [&](void* p) { dfree(c, p); });
 }
 
 // Chunks of a k sum of length kt whose output is m x n: enough 64 x 64 tiles
@@ -1829,14 +1824,8 @@ template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const void* Gs, const 
   const int MT = (int)((nw + BM - 1) / BM);
   x.xt = exch_items(NM, x.xch, BN);
   const size_t need = sizeof(zd) * 2 * (size_t)x.xt * nw;
-  if (c->ybuf_bytes < need) {
-    dfree(c, c->Ybuf);
-    c->Ybuf = nullptr;
-    c->ybuf_bytes = 0;
-    RET(dalloc_bytes(c, &c->Ybuf, need));
-    c->ybuf_bytes = need;
-  }
-  x.part = (zd*)c->Ybuf;
+  RET(need_work(c, c->ybuf, need));
+  x.part = (zd*)c->ybuf.p;
   const double inv_dt = 1.0 / c->dt_sys;
   const unsigned grid = exch_grid(x.xt, MT);
   if constexpr (CP == CP_F64) {
@@ -1934,6 +1923,7 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     // the triangle) and its dot with G is added in FP64, which bounds the
     // accumulation error of reduced-precision contractions.
     using ZT = typename ztype<YT>::type;
+    RET(need_work(c, c->ybuf, sizeof(ZT) * (size_t)nw * NM));
     const long ch = (c->exch_chunk > 0 && c->exch_chunk < NM) ? c->exch_chunk : NM;
     for (int sp = 0; sp < 2; sp++) {
       for (long q0 = 0; q0 < NM; q0 += ch) {
@@ -1945,7 +1935,7 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
         a.B = (const typename ztype<VXT>::type*)c->Vx + sp * NM * NM + q0 * NM + q0;
         a.sbn = NM;
         a.sbk = 1;
-        a.C = (ZT*)c->Ybuf + q0;
+        a.C = (ZT*)c->ybuf.p + q0;
         a.scm = NM;
         a.scn = 1;
         a.m = nw;
@@ -1965,7 +1955,7 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
         RET(launch(c, "energy_exch_dot", [&]() {
           hipLaunchKernelGGL((coldot_kernel<typename ztype<GT>::type, ZT>), dim3(nw), dim3(256), 0, c->stream,
                              (int)(NM - q0), (const typename ztype<GT>::type*)Gp + sp * NM + q0, 1L, 2 * NM,
-                             (const ZT*)c->Ybuf + q0, 1L, NM, c->e_exch_part + sp, 2L, 1.0, q0 > 0 ? 1 : 0);
+                             (const ZT*)c->ybuf.p + q0, 1L, NM, c->e_exch_part + sp, 2L, 1.0, q0 > 0 ? 1 : 0);
         }));
       }
     }
@@ -1975,7 +1965,8 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
   RET(launch(c, "energy_zero",
              [&]() { (void)hipMemsetAsync(c->e_exch_part, 0, sizeof(zd) * 2 * nw, c->stream); }));
   const long per_item = (long)N * N;
-  const long ycap = (long)(c->ybuf_bytes / sizeof(typename ztype<YT>::type));
+  RET(need_work(c, c->ybuf, sizeof(typename ztype<YT>::type) * 2 * (size_t)nw * per_item));  // one vector
+  const long ycap = (long)(c->ybuf.bytes / sizeof(typename ztype<YT>::type));
   const int nq = (int)std::max<long>(1, std::min<long>(K, ycap / (2L * nw * per_item)));
   for (int n0 = 0; n0 < K; n0 += nq) {
     const int cnt = std::min(nq, K - n0);
@@ -1991,7 +1982,7 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     a.sb1 = 2 * NM;
     a.sb2 = NM;
     a.bdiv = 2;
-    a.C = c->Ybuf;
+    a.C = c->ybuf.p;
     a.scm = N;
     a.scn = 1;
     a.sc1 = 2L * cnt * per_item;
@@ -2032,7 +2023,7 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     RET(need_work(c, c->ews, sizeof(zd) * (size_t)ngrp * 2 * nw));
     RET(launch(c, "energy_trace", [&]() {
       hipLaunchKernelGGL((trace_sq_kernel<typename ztype<YT>::type>), dim3(2 * nw, ngrp), dim3(256), 0, c->stream,
-                         (const typename ztype<YT>::type*)c->Ybuf, N, cnt, (long)cnt * per_item, (zd*)c->ews.p, ngrp);
+                         (const typename ztype<YT>::type*)c->ybuf.p, N, cnt, (long)cnt * per_item, (zd*)c->ews.p, ngrp);
       hipLaunchKernelGGL(add_parts_kernel, dim3((2 * nw + 255) / 256), dim3(256), 0, c->stream, (const zd*)c->ews.p,
                          ngrp, c->e_exch_part, 2 * nw);
     }));
@@ -2092,11 +2083,7 @@ template <class ZT> int maybe_vx(afqmc_ctx* c, const zd* Lt64, size_t zsize)
   const size_t need = bytes + ybytes + ((size_t)8 << 30);
   if (need > fr) return AFQMC_OK;
   RET(dalloc_bytes(c, &c->Vx, bytes));
-  if (c->ybuf_bytes < ybytes) {
-    dfree(c, c->Ybuf);
-    c->ybuf_bytes = ybytes;
-    RET(dalloc_bytes(c, &c->Ybuf, ybytes));
-  }
+  RET(need_work(c, c->ybuf, ybytes));
   if (std::is_same<ZT, zd>::value) return build_vx<double>(c, Lt64);
   if (std::is_same<ZT, zb>::value) return build_vx<bfs>(c, Lt64);
   return build_vx<float>(c, Lt64);
@@ -2119,11 +2106,7 @@ int maybe_vx3(afqmc_ctx* c, const zd* Lt64)
   RET(dalloc(c, &c->Vx3, 2 * (size_t)NM * NM));
   RET(dalloc(c, &c->G3, 2 * (size_t)NM * nw));
   RET(dalloc(c, &c->G3l, 2 * (size_t)NM * nw));
-  if (c->ybuf_bytes < ybytes) {
-    dfree(c, c->Ybuf);
-    c->ybuf_bytes = ybytes;
-    RET(dalloc_bytes(c, &c->Ybuf, ybytes));
-  }
+  RET(need_work(c, c->ybuf, ybytes));
   RET(build_vx<float>(c, Lt64));
   return launch(c, "vx_split3", [&]() {
     hipLaunchKernelGGL((split3_kernel<zf>), dim3(nblk(2 * NM * NM, 256)), dim3(256), 0, c->stream, (const zf*)c->Vx,
@@ -2448,8 +2431,7 @@ int afqmc_ctx_create(int nmo, int naea, int nchol, int nwalk, int mode, afqmc_ct
   chk(dalloc(c, &c->e_exch_part, 2 * nw));
   chk(dalloc(c, &c->e_one, nw));
   chk(dalloc(c, &c->e_v, nw * K));
-  c->ybuf_bytes = std::max<long>(2 * nw * N * N, std::min<long>(2 * nw * K * N * N, 1L << 25)) * sizeof(zd);
-  chk(dalloc_bytes(c, &c->Ybuf, c->ybuf_bytes));
+  chk(need_work(c, c->ybuf, std::max<long>(2 * nw * N * N, std::min<long>(2 * nw * K * N * N, 1L << 25)) * sizeof(zd)));
   if (r != AFQMC_OK) {
     afqmc_ctx_destroy(c);
     return r;
