@@ -191,7 +191,7 @@ struct afqmc_ctx {
   zd* oU = nullptr;   // [2nw][N][N] R^{-1}
   zd* oX = nullptr;   // [2][2nw][M][N] the two Cholesky QR passes
   int* ofail = nullptr;  // [2nw] matrices left to the Householder kernel
-  zd* Gcloc = nullptr;    // CSR mode Vakbl energy
+  zd* Gcloc = nullptr;    // Y of the Vakbl energy in CSR form
 
   // profiling
   bool prof = false;
@@ -2114,6 +2114,22 @@ int maybe_vx3(afqmc_ctx* c, const zd* Lt64)
   });
 }
 
+// The dense Vakbl product Y = Vakbl G as S partial products over chunks of its
+// sum, and the workspace that holds them (from the upload on, where the CSR
+// form allocates its Y).
+int vakbl_split(afqmc_ctx* c, long* chunk)
+{
+  const long NAK = 2L * c->N * c->M;
+  *chunk = f64_chunk(c->nw, NAK, NAK, 1, 16);
+  return (int)((NAK + *chunk - 1) / *chunk);
+}
+int vakbl_work(afqmc_ctx* c)
+{
+  long chunk;
+  const int S = vakbl_split(c, &chunk);
+  return need_work(c, c->ews, sizeof(zd) * (size_t)S * c->nw * 2 * c->N * c->M);
+}
+
 int do_energy(afqmc_ctx* c, double* eav_out)
 {
   const int nw = c->nw, N = c->N, M = c->M;
@@ -2121,10 +2137,10 @@ int do_energy(afqmc_ctx* c, double* eav_out)
   if (c->mode == AFQMC_FP64_CSR) {
     if (c->vkd) {
       // Y(w, i) = sum_j G(w, j) Vakbl(i, j) on FP64 MFMA, split over j
-      const long chunk = f64_chunk(nw, NAK, NAK, 1, 16);
-      const int S = (int)((NAK + chunk - 1) / chunk);
+      long chunk;
+      const int S = vakbl_split(c, &chunk);
       const long gsw = g_wfirst(c) ? NAK : 1, gsi = g_wfirst(c) ? 1 : nw;
-      RET(need_work(c, c->ews, sizeof(zd) * (size_t)S * nw * NAK));
+      RET(vakbl_work(c));
       F64Args a = f64args(nw, (int)NAK, (int)chunk);
       a.ktot = NAK;
       a.bdiv = S;
@@ -2853,8 +2869,10 @@ int afqmc_upload_system(afqmc_ctx* c, const double* trial_alpha, const double* t
         dfree(c, c->v_val);
         c->v_rp = c->v_col = nullptr;
         c->v_val = nullptr;
+        RET(vakbl_work(c));
+      } else {
+        RET(dalloc(c, &c->Gcloc, 2 * NM * c->nw));
       }
-      RET(dalloc(c, &c->Gcloc, 2 * NM * c->nw));
       HIPCHK(c, hipStreamSynchronize(st));
       dfree(c, Lt64);
     } else {
