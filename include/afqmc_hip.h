@@ -116,14 +116,15 @@ typedef enum {
    * over all columns.  May be changed at any time.  No counterpart in the
    * reference (its energy is FP64 throughout). */
   AFQMC_OPT_EXCHANGE_CHUNK = 4,
-  /* (Up to 192 orbitals, 128 in FP64, the propagator runs as one kernel of
-   * its own whatever this option says, unless a GEMM tile is forced or
-   * products take three pieces.)
-   * AFQMC_MIXED_BF16 with M a multiple of 64 up to 512 and N a multiple of
+  /* AFQMC_MIXED_BF16 with M a multiple of 64 up to 512 and N a multiple of
    * 16: 1 runs the whole propagator (P W, the six Taylor terms, P U) as one
-   * kernel per walker and 32 columns, U kept in LDS; 0 (default) runs it as
-   * eight GEMM launches, which measured 2 % faster at 512 orbitals.  Both
-   * give the same walkers bit for bit.  May be changed at any time. */
+   * kernel per walker and 32 columns, U kept in LDS, unless products take
+   * three pieces; 0 (default) runs it as one kernel with V in registers up
+   * to 192 orbitals (128 in FP64) if no GEMM tile is forced, beyond as eight
+   * GEMM launches (13.9 ms per substep at 512 orbitals, 1024 walkers, with
+   * P W and P U in three pieces; the option's kernel 21.3 ms in two pieces
+   * throughout).  All give the same walkers bit for bit.  May be changed at
+   * any time. */
   AFQMC_OPT_FUSED_PROPAGATOR = 5,
   /* AFQMC_MIXED_BF16: 2 (default) runs the GEMMs whose operands are both
    * split-BF16 with k contiguous (vHS, the bias product, the Taylor steps

@@ -31,7 +31,7 @@ REFERENCE_TIMERS = (
     ("Bias Potential", ("vbias_gemm", "vbias_reduce", "csrmm_vbias", "csrmm_vbias_t")),
     ("H-S Potential", ("vhs_gemm", "csrmm_vhs", "vhs_transpose")),
     ("Sigma", ("fields", "set_substep")),
-    ("Propagation", ("prop_pw", "prop_taylor", "prop_ps", "prop_split_w", "prop_fused")),
+    ("Propagation", ("prop_pw", "prop_taylor", "prop_ps", "prop_split_w", "prop_fused", "prop_fused_cols")),
     ("Other", ("save_overlaps", "weights", "branch_select", "branch_gather")),
     ("Overlap", ("ovlp_gemm", "gj_inverse")),
     ("Orthgonalization", ("ortho_gram", "ortho_chol_inv", "ortho_sign", "ortho_apply", "ortho_flags",
@@ -200,7 +200,7 @@ class AfqmcSys:
         self._check(nat.lib.afqmc_set_option(self.ctx, nat.OPT_ORTHO_HOUSEHOLDER, 1.0 if on else 0.0))
 
     def set_fused_propagator(self, on):
-        """Split-BF16 mode: the whole propagator in one kernel (1) or as eight GEMMs (0)."""
+        """Split-BF16 mode: the propagator as one kernel with its terms in LDS (1), or by size (0)."""
         self._check(nat.lib.afqmc_set_option(self.ctx, nat.OPT_FUSED_PROPAGATOR, 1.0 if on else 0.0))
 
     def set_direct_lds(self, level=2):

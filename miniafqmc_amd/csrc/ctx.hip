@@ -1555,7 +1555,7 @@ int propagate_fused(afqmc_ctx* c)
   a.ncb = 2 * c->N / PF_NB;
   const unsigned grid = (unsigned)((long)c->nw * a.ncb);
   // 16 waves of 16 or 32 rows each
-  return launch(c, "prop_fused", [&]() {
+  return launch(c, "prop_fused_cols", [&]() {
     if (c->M <= 256)
       hipLaunchKernelGGL((prop_fused_kernel<1, 16>), dim3(grid), dim3(1024), 0, c->stream, a);
     else
@@ -1568,6 +1568,7 @@ int do_propagate(afqmc_ctx* c)
   c->t1inv_valid = false;
   c->g_fresh = false;
   if (c->three & 4) return propagate_split(c);
+  if (fused_prop_ok(c)) return propagate_fused(c);
   // small systems in one kernel (a forced GEMM tile keeps the GEMM chain)
   const int fmt = c->mode == AFQMC_MIXED_FP32 ? 1 : c->mode == AFQMC_MIXED_BF16 ? 2 : 0;
   if (c->force_cfg == 0 && prop_small_ok(fmt, c->M)) {
@@ -1581,7 +1582,6 @@ int do_propagate(afqmc_ctx* c)
     a.ncb = 0;
     return launch(c, "prop_fused", [&]() { prop_small_launch(c->stream, a, fmt); }, 8);
   }
-  if (fused_prop_ok(c)) return propagate_fused(c);
   if (c->mode == AFQMC_FP64_CSR) return propagate_f64(c, c->vHSw);
   if (c->mode == AFQMC_FP64_DENSE) return propagate_f64(c, (const zd*)c->vHS);
   if (c->mode == AFQMC_MIXED_FP32)
