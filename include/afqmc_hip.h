@@ -356,8 +356,7 @@ const char* afqmc_group_error(const afqmc_group* group);
 /* ---- measurement -------------------------------------------------------- */
 /* Per-kernel timing with HIP events on the context's stream.  While enabled,
  * every launch is bracketed by events; afqmc_kernel_stats fills up to `cap`
- * entries (name, launches, total ms) and returns the count in *count.  The
- * one-kernel propagator of small systems counts as its eight products. */
+ * entries (name, launches, total ms) and returns the count in *count. */
 int afqmc_profile(afqmc_ctx* ctx, int enable);
 int afqmc_kernel_stats(afqmc_ctx* ctx, int cap, char (*names)[64], long long* launches, double* total_ms,
                        int* count);

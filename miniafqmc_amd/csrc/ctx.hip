@@ -42,7 +42,6 @@ struct KStat {
 struct EvPair {
   std::string name;
   hipEvent_t a, b;
-  int count;
 };
 
 } // namespace
@@ -373,9 +372,7 @@ const Roctx& roctx()
   return r;
 }
 
-// count: what the statistics count it as (a kernel that runs several products
-// of the call-by-call form counts each).
-template <class F> int launch(afqmc_ctx* c, const char* name, F&& f, int count = 1)
+template <class F> int launch(afqmc_ctx* c, const char* name, F&& f)
 {
   const Roctx& rx = roctx();
   if (rx.push) rx.push(c->tuning ? (std::string("tune/") + name).c_str() : name);
@@ -397,7 +394,7 @@ template <class F> int launch(afqmc_ctx* c, const char* name, F&& f, int count =
   if (e != hipSuccess) return fail(c, AFQMC_ERR_HIP, std::string(name) + ": " + hipGetErrorString(e));
   if (c->prof) {
     (void)hipEventRecord(b, c->stream);
-    c->pending.push_back({name, a, b, count});
+    c->pending.push_back({name, a, b});
   }
   return AFQMC_OK;
 }
@@ -410,7 +407,7 @@ void collect_events(afqmc_ctx* c)
     float ms = 0.f;
     (void)hipEventElapsedTime(&ms, p.a, p.b);
     auto& s = c->stats[p.name];
-    s.n += p.count;
+    s.n++;
     s.ms += ms;
     c->evpool.push_back(p.a);
     c->evpool.push_back(p.b);
@@ -1580,7 +1577,7 @@ int do_propagate(afqmc_ctx* c)
     a.N = c->N;
     a.nw = c->nw;
     a.ncb = 0;
-    return launch(c, "prop_fused", [&]() { prop_small_launch(c->stream, a, fmt); }, 8);
+    return launch(c, "prop_fused", [&]() { prop_small_launch(c->stream, a, fmt); });
   }
   if (c->mode == AFQMC_FP64_CSR) return propagate_f64(c, c->vHSw);
   if (c->mode == AFQMC_FP64_DENSE) return propagate_f64(c, (const zd*)c->vHS);

@@ -57,3 +57,13 @@ def test_fused_option_leaves_other_shapes(require_gpu, M, N, mode):
     a, sa = walk(M, N, 6, mode, fused=True)
     b, sb = walk(M, N, 6, mode)
     assert set(sa) == set(sb) == {"prop_fused"} and np.array_equal(a, b)
+
+
+@pytest.mark.parametrize("mode", ["fp64_dense", "mixed_fp32", "mixed_bf16"])
+def test_statistics_count_launches(require_gpu, mode):
+    """One kernel is one launch in the statistics, whatever it runs; the
+    timers count its eight products."""
+    _, st = walk(64, 16, 6, mode)
+    assert st["prop_fused"][0] == 1
+    calls, ms = m.reference_timers(st)["Propagation"]
+    assert calls == 8 and ms == st["prop_fused"][1]
