@@ -6,9 +6,9 @@ import sys
 
 import numpy as np
 import pytest
-import torch
 
 import miniafqmc_amd as m
+import hip_rt
 
 pytestmark = pytest.mark.gpu
 
@@ -46,15 +46,16 @@ class Neighbours:
 
     def __init__(self, s, nw):
         n = 32 * nw * s.nchol * 2
-        self.t = [torch.full((n // k,), float("nan"), dtype=torch.float64, device="cuda") for k in (1, 2, 4, 16)
-                  for _ in range(8)]
+        r = np.random.default_rng(nw)
+        self.t = [hip_rt.Buffer(r.standard_normal(n // k)) for k in (1, 2, 4, 16) for _ in range(8)]
         self.g = m.AfqmcSys(s, nw, "fp64_csr" if s.vakbl is not None else "fp64_dense")
         self.g.init_walkers()
         energy(self.g)
-        torch.cuda.synchronize()
 
     def check(self):
-        assert all(bool(torch.isnan(t).all()) for t in self.t), "another allocation was written"
+        assert all(t.unchanged() for t in self.t), "another allocation was written"
+        for t in self.t:
+            t.free()
         self.g.close()
 
 

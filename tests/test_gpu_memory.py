@@ -2,9 +2,9 @@
 import sys
 
 import pytest
-import torch
 
 import miniafqmc_amd as m
+from hip_rt import free_bytes
 
 pytestmark = pytest.mark.gpu
 MB = 1 << 20
@@ -13,11 +13,6 @@ MB = 1 << 20
 def say(*a):
     print(*a, flush=True)
     sys.stdout.flush()
-
-
-def free_bytes():
-    torch.cuda.synchronize()
-    return torch.cuda.mem_get_info()[0]
 
 
 def test_dense_vakbl_allocates_at_upload_only(require_gpu):
