@@ -113,6 +113,7 @@ struct afqmc_ctx {
   zd* gjwork = nullptr;   // N > 128: [nw][2][N][N] working matrices of the batched inverse
   bool t1inv_valid = false;  // T1 holds the inverses for the current walkers
   bool g_fresh = false;      // G was built from T1 and W as they are now
+  bool g_early = false;      // G was written before the system was uploaded
   zd* Wbr = nullptr;         // population control: gathered walkers [nw][2][M][N]
   zd* Wdbr = nullptr;        // and W_data rows [nw][8]
   zd* Wlbr = nullptr;        // and log-overlaps [nw][4]
@@ -855,10 +856,11 @@ ZGemmArgs gc_args(const afqmc_ctx* c)
 
 // G is held walker-first, [nw][2NM], where only GEMMs read it (written in
 // rows of M instead of single values nw apart: gc_gemm 316 -> 105 us at 256
-// walkers of 64 x 256); the CSR products read it walker-last.
+// walkers of 64 x 256); the CSR products read it walker-last, and so it is in
+// the CSR mode until the upload has settled which they are.
 bool g_wfirst(const afqmc_ctx* c)
 {
-  return c->mode != AFQMC_FP64_CSR || (c->sptd && !c->v_rp);
+  return c->mode != AFQMC_FP64_CSR || (c->have_system && c->sptd && !c->v_rp);
 }
 
 // FP64 copy of G in [nw][2NM] for the energy of the mixed modes: rebuilt
@@ -959,6 +961,24 @@ int need_work(afqmc_ctx* c, Work& w, size_t bytes)
         return AFQMC_OK;
       },
       [&](void** p, size_t n) { return dalloc_bytes(c, p, n); }, [&](void* p) { dfree(c, p); });
+}
+
+// G walker-last (rows = 2NM) or walker-first (rows = nw) from `in` to the
+// other layout in `out`
+int turn_g(afqmc_ctx* c, const zd* in, zd* out, long rows)
+{
+  const long cols = 2L * c->N * c->M * c->nw / rows;
+  return launch(c, "g_transpose", [&]() {
+    hipLaunchKernelGGL((ztranspose_kernel<zd, zd>), dim3((unsigned)((cols + 31) / 32), (unsigned)((rows + 31) / 32)),
+                       dim3(256), 0, c->stream, in, out, (int)rows, (int)cols, cols, rows);
+  });
+}
+// room for G turned: Gtmp or the energy's workspace
+int turn_room(afqmc_ctx* c, zd** t)
+{
+  if (!c->Gtmp) RET(need_work(c, c->ews, sizeof(zd) * 2 * c->N * c->M * (size_t)c->nw));
+  *t = c->Gtmp ? c->Gtmp : (zd*)c->ews.p;
+  return AFQMC_OK;
 }
 
 // Chunks of a k sum of length kt whose output is m x n: enough 64 x 64 tiles
@@ -2173,11 +2193,7 @@ int do_energy(afqmc_ctx* c, double* eav_out)
     } else {
       const void* G = c->G;
       if (!g_wfirst(c)) {
-        dim3 grid((nw + 31) / 32, (unsigned)((NAK + 31) / 32));
-        RET(launch(c, "g_transpose", [&]() {
-          hipLaunchKernelGGL((ztranspose_kernel<zd, zd>), grid, dim3(256), 0, c->stream, (const zd*)c->G, c->Gtmp,
-                             (int)NAK, nw, (long)nw, NAK);
-        }));
+        RET(turn_g(c, (const zd*)c->G, c->Gtmp, NAK));
         G = c->Gtmp;
       }
       RET((energy_cholesky<CP_F64, double, CP_F64, double, double, double, double>(c, G, c->Lt, c->Lt)));
@@ -2940,8 +2956,20 @@ int afqmc_upload_system(afqmc_ctx* c, const double* trial_alpha, const double* t
       c->Lt = Lt64;
     }
   }
-  HIPCHK(c, hipStreamSynchronize(st));
   c->have_system = true;
+  if (c->g_early && c->mode == AFQMC_FP64_CSR && g_wfirst(c)) {
+    // G was written before its layout was settled
+    zd* t;
+    int r = turn_room(c, &t);
+    if (r == AFQMC_OK) r = turn_g(c, (const zd*)c->G, t, 2 * NM);
+    if (r == AFQMC_OK && hipMemcpyAsync(c->G, t, sizeof(zd) * 2 * NM * c->nw, hipMemcpyDeviceToDevice, st) != hipSuccess)
+      r = AFQMC_ERR_HIP;
+    if (r != AFQMC_OK) {
+      c->have_system = false;
+      return r;
+    }
+  }
+  HIPCHK(c, hipStreamSynchronize(st));
   return AFQMC_OK;
 }
 
@@ -3042,19 +3070,14 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
   // FP64 G of the CSR mode held walker-first: turned on the device (134 MB
   // read in 4.7 ms and written in 5; 94 and 112 turned by a host thread)
   auto turned = [&]() -> int {
-    zd* t = c->Gtmp;
-    if (!t) {
-      RET(need_work(c, c->ews, sizeof(zd) * NAK * nw));
-      t = (zd*)c->ews.p;
+    zd* t;
+    RET(turn_room(c, &t));
+    if (to_device) {
+      RET(raw(t, sizeof(zd) * NAK * nw));
+      return turn_g(c, t, (zd*)c->G, NAK);
     }
-    if (to_device) RET(raw(t, sizeof(zd) * NAK * nw));
-    const long R = to_device ? NAK : nw, C = to_device ? nw : NAK;  // of the input
-    RET(launch(c, "g_transpose", [&]() {
-      hipLaunchKernelGGL((ztranspose_kernel<zd, zd>), dim3((unsigned)((C + 31) / 32), (unsigned)((R + 31) / 32)),
-                         dim3(256), 0, st, to_device ? t : (const zd*)c->G, to_device ? (zd*)c->G : t, (int)R, (int)C,
-                         C, R);
-    }));
-    return to_device ? AFQMC_OK : raw(t, sizeof(zd) * NAK * nw);
+    RET(turn_g(c, (const zd*)c->G, t, nw));
+    return raw(t, sizeof(zd) * NAK * nw);
   };
   const bool d = dense_layout(c);
   if (to_device && buffer == AFQMC_BUF_W) c->t1inv_valid = false;
@@ -3071,6 +3094,7 @@ int afqmc_copy(afqmc_ctx* c, int buffer, int to_device, double* host)
     return AFQMC_OK;
   case AFQMC_BUF_HYBRIDW: return raw(c->hybridW, sizeof(zd) * nw);
   case AFQMC_BUF_G:
+    if (to_device && !c->have_system) c->g_early = true;
     if (d) return wlast(c->G, NAK, c->mixed, c->tp_G);
     return g_wfirst(c) ? turned() : raw(c->G, sizeof(zd) * NAK * nw);
   case AFQMC_BUF_VBIAS: return d ? wlast(c->vbias, K, false) : raw(c->vbias, sizeof(zd) * K * nw);
