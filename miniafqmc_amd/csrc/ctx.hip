@@ -2088,7 +2088,9 @@ template <class OT> int build_vx(afqmc_ctx* c, const zd* Lt64)
 
 // Build Vx when it fits in device memory with room to spare; otherwise the
 // energy uses the Cholesky form.
-// ZT: storage of Vx; the exchange GEMM writes Z [nw][NM] of zsize bytes per element.
+// ZT: storage of Vx.  The form in chunks of products writes Z [nw][NM] of
+// zsize bytes per element: room is left for it, but only a call that takes that
+// form allocates it (the one-launch form needs a partial per tile and walker).
 template <class ZT> int maybe_vx(afqmc_ctx* c, const zd* Lt64, size_t zsize)
 {
   if (!c->allow_vx) return AFQMC_OK;
@@ -2100,7 +2102,6 @@ template <class ZT> int maybe_vx(afqmc_ctx* c, const zd* Lt64, size_t zsize)
   const size_t need = bytes + ybytes + ((size_t)8 << 30);
   if (need > fr) return AFQMC_OK;
   RET(dalloc_bytes(c, &c->Vx, bytes));
-  RET(need_work(c, c->ybuf, ybytes));
   if (std::is_same<ZT, zd>::value) return build_vx<double>(c, Lt64);
   if (std::is_same<ZT, zb>::value) return build_vx<bfs>(c, Lt64);
   return build_vx<float>(c, Lt64);
@@ -2123,7 +2124,6 @@ int maybe_vx3(afqmc_ctx* c, const zd* Lt64)
   RET(dalloc(c, &c->Vx3, 2 * (size_t)NM * NM));
   RET(dalloc(c, &c->G3, 2 * (size_t)NM * nw));
   RET(dalloc(c, &c->G3l, 2 * (size_t)NM * nw));
-  RET(need_work(c, c->ybuf, ybytes));
   RET(build_vx<float>(c, Lt64));
   return launch(c, "vx_split3", [&]() {
     hipLaunchKernelGGL((split3_kernel<zf>), dim3(nblk(2 * NM * NM, 256)), dim3(256), 0, c->stream, (const zf*)c->Vx,

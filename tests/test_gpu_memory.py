@@ -40,3 +40,28 @@ def test_dense_vakbl_allocates_at_upload_only(require_gpu):
     dense = 16 * v + 2 * 16 * nw * 2 * N * M + 16 * K * 2 * N * M  # Vakbl, workspace, SpvnT
     csr = 20 * s.vakbl.nnz + 16 * nw * 2 * N * M                   # Vakbl, Y
     assert abs(used[True][0] - used[False][0] - (dense - csr)) < 12 * MB, (used, dense, csr)
+
+
+@pytest.mark.parametrize("mode,zs", [("fp64_dense", 16), ("mixed_fp32", 8), ("mixed_bf16", 8)])
+def test_dense_exchange_holds_its_block_only(require_gpu, mode, zs):
+    """The dense exchange block costs its own size at the upload, not the
+    product's [walkers][N M] output beside it (33 or 17 MB here), which only
+    the form in chunks writes: that one allocates it when it runs."""
+    M, N, K, nw = 256, 4, 4, 2048
+    s = m.make_system(M, N, K, density=1.0, sigma_L=0.02, sigma_h=1.0, dt=0.005, seed=4)
+    used = {}
+    for block in (True, False, True):  # the first one loads the kernels
+        say("dense exchange", mode, block)
+        f0 = free_bytes()
+        g = m.AfqmcSys(s, nw, mode, dense_exchange=block)
+        used[block] = f0 - free_bytes()
+        g.init_walkers()
+        g.calculate_mixed_density_matrix()
+        e = [g.calculate_energy()]
+        if block and mode != "fp64_dense":
+            g.set_direct_lds(0)  # the form in chunks
+            e.append(g.calculate_energy())
+            assert abs(e[1] - e[0]) <= 1e-4 * abs(e[0])
+        g.close()
+    say(used)
+    assert abs(used[True] - used[False] - 2 * zs * (N * M) ** 2) < 6 * MB, used
