@@ -1794,13 +1794,13 @@ int do_ortho(afqmc_ctx* c)
 // 4.46 -> 0.80 ms.
 constexpr long kF64ExchChunk = 2048;
 
+// whether the dense block's exchange runs in one launch: always in FP64 and in
+// three pieces (whose block is only built where N M is a multiple of 16); FP32
+// and two pieces take whole 16-byte chunks through the ring
 template <int CP> bool exch_one_ok(const afqmc_ctx* c)
 {
-  if (CP == CP_F64) return true;
-  const long NM = (long)c->N * c->M;
-  if (CP == CP_F32) return NM % 2 == 0 && c->gemm_adma && c->gemm_ring;
-  if (CP == CP_BF16X6) return NM % 16 == 0;
-  return CP == CP_BF16X3 && NM % 2 == 0 && c->exch_chunk % 2 == 0 && c->gemm_adma && c->gemm_ring;
+  if (CP == CP_F64 || CP == CP_BF16X6) return true;
+  return (long)c->N * c->M % 2 == 0 && c->gemm_adma && c->gemm_ring;
 }
 
 // G: FP64 [nw][2NM]; Gs (and Gs3): its split forms
@@ -1907,8 +1907,9 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     RET((dense_contract_vbias<CPV, GT, LVT>(c, c->ews, Gp, Lv, c->e_v, "energy_v_gemm", nullptr, nullptr,
                                             "energy_v_reduce")));
   }
+  constexpr bool G64 = std::is_same<GT, double>::value;
   bool one = false;
-  if constexpr (std::is_same<GT, double>::value && (CP == CP_F64 || CP == CP_F32 || CP == CP_BF16X3 || CP == CP_BF16X6)) {
+  if constexpr (G64) {
     one = c->Vx && exch_one_ok<CP>(c);
     if (one) {
       if (CP == CP_BF16X3) {
@@ -1930,8 +1931,9 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
       RET(exch_one<CP>(c, (const zd*)Gp, c->G3, c->G3l));
     }
   }
-  if (one) {
-  } else if (c->Vx) {
+  if (c->Vx) {
+    if constexpr (G64 && (CP == CP_F64 || CP == CP_BF16X6)) {  // always in one launch
+    } else if (!one) {
     // exchange from the dense same-spin block of Vakbl held in HBM as its
     // lower triangle with the strictly lower part doubled:
     // Z(w, p) = sum_{q <= p} G_s(w, q) Vx'_s(p, q);  e_x(w, s) = sum_p G_s(w, p) Z(w, p)
@@ -1960,21 +1962,14 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
         a.k = (int)kc;
         a.ar = inv_dt;
         a.ktri = 1;
-        if constexpr (CP == CP_BF16X6) {
-          // the product reads the three-piece G; the dot below keeps the FP64 G
-          a.A = c->G3 + sp * NM + q0;
-          a.A3 = c->G3l + sp * NM + q0;
-          a.B3 = c->Vx3 + sp * NM * NM + q0 * NM + q0;
-          RET((zgemm<CP, bfs, VXT, YT, true, true>(c, "energy_vx_gemm", a, 1)));
-        } else {
-          RET((zgemm<CP, GT, VXT, YT, true, true>(c, "energy_vx_gemm", a, 1)));
-        }
+        RET((zgemm<CP, GT, VXT, YT, true, true>(c, "energy_vx_gemm", a, 1)));
         RET(launch(c, "energy_exch_dot", [&]() {
           hipLaunchKernelGGL((coldot_kernel<typename ztype<GT>::type, ZT>), dim3(nw), dim3(256), 0, c->stream,
                              (int)(NM - q0), (const typename ztype<GT>::type*)Gp + sp * NM + q0, 1L, 2 * NM,
                              (const ZT*)c->ybuf.p + q0, 1L, NM, c->e_exch_part + sp, 2L, 1.0, q0 > 0 ? 1 : 0);
         }));
       }
+    }
     }
   } else {
   // exchange: Y_n,s = Lt_s(n) G_s^T (N x N), sum_ab Y_ab Y_ba, for all
