@@ -83,17 +83,16 @@ def csr_flops(name, nw, nnz_spvn, nnz_spvnT):
     return None if c is None else 8.0 * c
 
 
-def contraction_spins_per_launch(M, N, K, nw, mode=None):
+def contraction_spins_per_launch(*shape):
     """Spin blocks per launch of the bias-shaped contraction (G against the
-    K Cholesky rows, the bias and the Coulomb term): both, as batch items,
-    however the sum over N*M is split."""
+    K Cholesky rows, the bias and the Coulomb term): both, as batch items, at
+    every shape and however the sum over N*M is split."""
     return 2
 
 
 def kernel_flops(name, M, N, K, nw, mode=None):
-    """Algorithmic real flops per launch (8 per complex multiply-add).  The
-    FP64 CSR mode's dense bias product contracts both spins in one launch."""
-    sp = 2 if mode == "fp64_csr" else contraction_spins_per_launch(M, N, K, nw, mode)
+    """Algorithmic real flops per launch (8 per complex multiply-add)."""
+    sp = contraction_spins_per_launch(M, N, K, nw)
     c = {
         "vhs_gemm": nw * M * M * K,
         "prop_taylor": 2 * nw * M * M * N,

@@ -109,6 +109,21 @@ __device__ inline zd load_z(const zf* p)
   return {(double)v.re, (double)v.im};
 }
 
+// Direct global -> LDS staging
+namespace dma {
+
+// s_waitcnt with only vmcnt = n (expcnt and lgkmcnt at their maxima), gfx9
+// encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14
+template <int N> __device__ __forceinline__ void wait_vmcnt()
+{
+  static_assert(N >= 0 && N < 64, "vmcnt out of range");
+  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
+}
+// 16-byte chunk c of a 128-byte tile row R sits at c ^ swz(R)
+__device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
+
+} // namespace dma
+
 // The exchange energy as one launch (XD mode of the GEMM kernels).  The
 // lower-triangular block of each spin is cut into chunks of xch columns
 // (AFQMC_OPT_EXCHANGE_CHUNK), chunk c holding the rows p >= c * xch; a work

@@ -586,13 +586,12 @@ F64Args f64args(int m, int n, int k)
 // few waves to cover the LDS reads and reaches about 0.7 of it.
 int f64_default(const F64Args& a, int batch)
 {
-  constexpr double rate[kNF64] = {57.4, 62.7, 63.9};
   int best = 0;
   double tb = 1e300;
   for (int i = 0; i < kNF64; i++) {
     const double tiles = (double)((a.m + kF64[i].BM - 1) / kF64[i].BM) * ((a.n + kF64[i].BN - 1) / kF64[i].BN) * batch;
     const double percu = std::ceil(tiles / 256.0);
-    const double t = percu * kF64[i].BM * kF64[i].BN / (rate[i] * (percu < 2.0 ? 0.7 : 1.0));
+    const double t = percu * kF64[i].BM * kF64[i].BN / (kF64Rate[i] * (percu < 2.0 ? 0.7 : 1.0));
     if (t < tb) {
       tb = t;
       best = i;
@@ -1818,7 +1817,6 @@ template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const void* Gs, const 
   double tb = 1e300;
   constexpr int NP = CP == CP_BF16X6 ? 3 : CP == CP_F32 ? 0 : 2;
   constexpr int n = CP == CP_F64 ? kNF64 : NP == 0 ? ring_count<NP>() : kNExch;
-  constexpr double rate64[] = {57.4, 62.7, 63.9};
   constexpr double rateb[] = {0.86, 1.0, 1.0, 0.9, 0.55};
   auto dims = [&](int i, int& BM, int& BN) {
     BM = CP == CP_F64 ? kF64[i % kNF64].BM : ring_cfg<NP>(i).BM;
@@ -1829,7 +1827,7 @@ template <int CP> int exch_one(afqmc_ctx* c, const zd* G, const void* Gs, const 
     dims(i, BM, BN);
     const double tiles = 2.0 * ((nw + BM - 1) / BM) * exch_items(NM, x.xch, BN);
     const double percu = std::ceil(tiles / 256.0);
-    const double t = percu * BM * BN / ((CP == CP_F64 ? rate64[i % kNF64] : NP == 0 ? ring_rate<NP>(i) : rateb[i]) * (percu < 2.0 ? 0.7 : 1.0));
+    const double t = percu * BM * BN / ((CP == CP_F64 ? kF64Rate[i % kNF64] : NP == 0 ? ring_rate<NP>(i) : rateb[i]) * (percu < 2.0 ? 0.7 : 1.0));
     if (t < tb) {
       tb = t;
       best = i;
@@ -2850,7 +2848,7 @@ int afqmc_upload_system(afqmc_ctx* c, const double* trial_alpha, const double* t
       c->v_nnz = vn;
       // as SpvnT: rows at least half full make a dense product (not when
       // entries repeat, which csrmm adds up), which reads no more bytes and
-      // runs on MFMA: 1024 x 1024, 16 walkers 288 -> 43 us.  The dense form
+      // runs on MFMA: 2048 x 2048, 16 walkers 288 -> 43 us.  The dense form
       // takes the CSR form's place, so that little more memory is held.
       bool dense = c->csr_dense && 2.0 * vn >= (double)vr * vr;
       for (long r = 0; r < vr && dense; r++)

@@ -69,20 +69,6 @@
 #pragma once
 #include "gemm.hpp"
 
-namespace b16 {
-
-// s_waitcnt with only vmcnt = n (expcnt and lgkmcnt at their maxima), gfx9
-// encoding: vmcnt[3:0] | expcnt[6:4] | lgkmcnt[11:8] | vmcnt[5:4] << 14
-template <int N> __device__ __forceinline__ void wait_vmcnt()
-{
-  static_assert(N >= 0 && N < 64, "vmcnt out of range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-
-__device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
-
-} // namespace b16
-
 // BM rows x BN complex columns per workgroup, WM x WN waves, STAGES k-tiles
 // of 16 complex in LDS.  OT: output element (double, float, or bfs for split
 // output).  Launch conditions (checked by the host): A and B split-BF16, unit
@@ -166,21 +152,21 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
 #pragma unroll
   for (int i = 0; i < AL; i++) {
     const int u = i * NT + tid, row = u / CH, pc = u % CH;
-    pa[i] = A + (long)min(m0 + row, p.m - 1) * p.sam + 2 * (pc ^ b16::swz(row));
+    pa[i] = A + (long)min(m0 + row, p.m - 1) * p.sam + 2 * (pc ^ dma::swz(row));
   }
 #pragma unroll
   for (int i = 0; i < BL; i++) {
     const int u = i * NT + tid, row = u / CH, pc = u % CH;
-    pb[i] = B + (long)min(n0 + row, pn - 1) * p.sbn + 2 * (pc ^ b16::swz(row));
+    pb[i] = B + (long)min(n0 + row, pn - 1) * p.sbn + 2 * (pc ^ dma::swz(row));
   }
   // third pieces: unit u is slot u % 8 of LDS row u / 8 = 16q + r, which
   // holds chunk x / 2 (four complex) of tile row 32q + 16 (x & 1) + r, where
   // x = (u % 8) ^ swz(r)
   auto row3 = [](int u) {
-    const int sr = u >> 3, x = (u & 7) ^ b16::swz(sr & 15);
+    const int sr = u >> 3, x = (u & 7) ^ dma::swz(sr & 15);
     return 32 * (sr >> 4) + 16 * (x & 1) + (sr & 15);
   };
-  auto chunk3 = [](int u) { return ((u & 7) ^ b16::swz((u >> 3) & 15)) >> 1; };
+  auto chunk3 = [](int u) { return ((u & 7) ^ dma::swz((u >> 3) & 15)) >> 1; };
   const uint32_t* pa3[AL3 > 0 ? AL3 : 1];
   const uint32_t* pb3[BL3 > 0 ? BL3 : 1];
 #pragma unroll
@@ -196,7 +182,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
   const int w0 = __builtin_amdgcn_readfirstlane(wave);
   // largest k0 whose chunk of two starts inside (the same chunk of every row
   // is a thread's, as NT / 8 rows are a multiple of 16)
-  const int klast = ((kend - 1) & ~1) - 2 * ((tid & 7) ^ b16::swz(tid >> 3));
+  const int klast = ((kend - 1) & ~1) - 2 * ((tid & 7) ^ dma::swz(tid >> 3));
   auto issue = [&](uint2* st, int k0) __attribute__((always_inline)) {
     if constexpr (ANYK) k0 = min(k0, klast);
 #pragma unroll
@@ -234,7 +220,7 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
       }
 
   // fragment rows: this lane's rows are 16-aligned blocks + r, so swz = swz(r)
-  const int sw = b16::swz(r);
+  const int sw = dma::swz(r);
   const int c0 = (2 * g) ^ sw, c1 = (2 * g + 1) ^ sw;
   const int arow = wm * WTM + r, brow = BM + wn * WTN + r;
   // third pieces: LDS rows of the wave tile's first block pair (A, then B
@@ -410,9 +396,9 @@ __global__ __launch_bounds__(64 * WM * WN, WPE) void zgemm_b16dma_kernel(ZGemmAr
     Frags f;
     if (c >= 0) {
       const int ahead = min(nk - 1 - c, STAGES - 2);  // tiles issued after c
-      if (ahead >= 2) b16::wait_vmcnt<(STAGES > 3 ? 2 * LPT : 0)>();
-      else if (ahead == 1) b16::wait_vmcnt<(STAGES > 2 ? LPT : 0)>();
-      else b16::wait_vmcnt<0>();
+      if (ahead >= 2) dma::wait_vmcnt<(STAGES > 3 ? 2 * LPT : 0)>();
+      else if (ahead == 1) dma::wait_vmcnt<(STAGES > 2 ? LPT : 0)>();
+      else dma::wait_vmcnt<0>();
       // a bare barrier: a workgroup fence here would wait for the later
       // tiles' loads too
       __builtin_amdgcn_s_barrier();

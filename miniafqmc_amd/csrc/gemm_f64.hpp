@@ -8,9 +8,10 @@
 // runs as one tall product without a partial tile per batch item.
 //
 // Bound: the matrix cores.  One MFMA takes 64 cycles of its SIMD for 2048
-// flops, so a 64 x 32 complex wave tile has 4096 cycles of MFMA per k-tile of
-// 8 against 12 LDS reads of 16 bytes per lane; what the kernel has to get
-// right is that no wave ever waits on memory.  Each k-tile (8 complex = 128
+// flops, so a 32 x 32 complex wave tile has 2048 cycles of MFMA per k-tile of
+// 8 against 8 LDS reads of 16 bytes per lane (16 x 16, for outputs that would
+// leave CUs idle: 512 against 4); what the kernel has to get right is that no
+// wave ever waits on memory.  Each k-tile (8 complex = 128
 // bytes per row) goes from global memory straight into LDS
 // (global_load_lds_dwordx4, one complex per lane, any operand order since
 // every lane has an address of its own), STAGES k-tiles in a ring: the loads
@@ -67,13 +68,6 @@ struct F64Args {
 };
 
 namespace f64g {
-
-template <int N> __device__ __forceinline__ void wait_vmcnt()
-{
-  static_assert(N >= 0 && N < 64, "vmcnt out of range");
-  __builtin_amdgcn_s_waitcnt((N & 15) | (7 << 4) | (15 << 8) | ((N >> 4) << 14));
-}
-__device__ __forceinline__ int swz(int row) { return (row & 7) ^ ((row >> 3) & 1); }
 
 __device__ __forceinline__ void put(zd* p, long o, double re, double im) { p[o] = zd{re, im}; }
 __device__ __forceinline__ void put(zf* p, long o, double re, double im) { p[o] = zf{(float)re, (float)im}; }
@@ -146,7 +140,7 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_f64_kernel(F64Args p)
 
   // unit u = i * NT + tid of a tile is (row u / 8, slot u % 8) and holds the
   // row's k = slot ^ swz(row), which is the same for all of a thread's units
-  const int kc = (tid & 7) ^ f64g::swz(tid >> 3);
+  const int kc = (tid & 7) ^ dma::swz(tid >> 3);
   const zd* pa[AL];
   const zd* pb[BL];
 #pragma unroll
@@ -192,7 +186,7 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_f64_kernel(F64Args p)
 
   // fragment rows are 16-aligned blocks + r, so swz(row) = swz(r); lane group
   // g takes k = 4 kq + g
-  const int sw = f64g::swz(r);
+  const int sw = dma::swz(r);
   const int arow = wm * WTM + r, brow = BM + wn * WTN + r;
   const unsigned long long sa_ = p.conja ? 0x8000000000000000ull : 0ull, sb_ = p.conjb ? 0x8000000000000000ull : 0ull;
   auto flip = [](double x, unsigned long long s) __attribute__((always_inline)) {
@@ -254,9 +248,9 @@ __global__ __launch_bounds__(64 * WM * WN) void zgemm_f64_kernel(F64Args p)
     if (c >= 0) {
       if constexpr (DMA) {
         const int ahead = min(nk - 1 - c, STAGES - 2);  // tiles issued after c
-        if (ahead >= 2) f64g::wait_vmcnt<(STAGES > 3 ? 2 * LPT : 0)>();
-        else if (ahead == 1) f64g::wait_vmcnt<(STAGES > 2 ? LPT : 0)>();
-        else f64g::wait_vmcnt<0>();
+        if (ahead >= 2) dma::wait_vmcnt<(STAGES > 3 ? 2 * LPT : 0)>();
+        else if (ahead == 1) dma::wait_vmcnt<(STAGES > 2 ? LPT : 0)>();
+        else dma::wait_vmcnt<0>();
         __builtin_amdgcn_s_barrier();
       } else {
         __syncthreads();

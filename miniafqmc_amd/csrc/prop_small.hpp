@@ -16,6 +16,6 @@ struct PropSmallArgs {
 constexpr int PS_MMAX = 192;      // FP32 and split-BF16
 constexpr int PS_MMAX_F64 = 128;  // FP64
 
-// whether the format has a kernel for M (launches it on `st` when go is set)
-bool prop_small_ok(int mode_format, int M);  // 0 zd, 1 zf, 2 zb
+// format: 0 zd, 1 zf, 2 zb
+bool prop_small_ok(int mode_format, int M);  // whether it has a kernel for M
 void prop_small_launch(hipStream_t st, PropSmallArgs a, int mode_format);
