@@ -175,10 +175,10 @@ struct afqmc_ctx {
   bool allow_vx = true;
   zd* Gtmp = nullptr;     // FP64 G [nw][2NM] for the energy (CSR: transposed; mixed: FP64 copy)
   // split-k partials of the bias contraction; captured substeps hold its
-  // address, so it is theirs alone and growing it drops them
+  // address: growing it drops them, and an energy never grows it (split_work)
   Work vws;
   int vws_pending = 0;    // slices there that the next fields kernel sums into vbias
-  Work ews;               // partial sums of the energy (never captured)
+  Work ews;               // partial sums of the energy that vws does not hold (never captured)
   double* xtmp = nullptr; // draws passed to afqmc_fields, [K][nw] (allocated at the first such call)
   // orthogonalisation: Cholesky QR scratch (allocated at the first call)
   bool ortho_householder = false;  // always use the blocked Householder kernel
@@ -962,6 +962,14 @@ int need_work(afqmc_ctx* c, Work& w, size_t bytes)
       [&](void** p, size_t n) { return dalloc_bytes(c, p, n); }, [&](void* p) { dfree(c, p); });
 }
 
+// Where partial sums of `bytes` go: the bias's in vws; an energy's there too if
+// they fit (nothing is kept in it between calls), so that it never moves for
+// them and no second buffer is held, else in ews.
+Work& split_work(afqmc_ctx* c, bool energy, size_t bytes)
+{
+  return energy && c->vws.bytes < bytes ? c->ews : c->vws;
+}
+
 // G walker-last (rows = 2NM) or walker-first (rows = nw) from `in` to the
 // other layout in `out`
 int turn_g(afqmc_ctx* c, const zd* in, zd* out, long rows)
@@ -995,13 +1003,15 @@ long f64_chunk(long m, long n, long kt, int items, int smax)
 // products (spin, chunk of j) run as one batch into a workspace, summed in
 // chunk order.  (200 walkers, 999 vectors, N M = 15250: 12.6 ms unsplit in
 // 32 workgroups per spin.)
-int dense_contract_f64(afqmc_ctx* c, Work& ws, const zd* G, const zd* Lt, zd* out, const char* name,
+int dense_contract_f64(afqmc_ctx* c, bool energy, const zd* G, const zd* Lt, zd* out, const char* name,
                        const char* rname, bool defer)
 {
   const long NM = (long)c->N * c->M, nw = c->nw, K = c->K;
   const long chunk = f64_chunk(nw, K, NM, 2, 16);
   const int S = (int)((NM + chunk - 1) / chunk);
-  RET(need_work(c, ws, sizeof(zd) * 2 * S * nw * K));
+  const size_t need = sizeof(zd) * 2 * S * nw * K;
+  Work& ws = split_work(c, energy, need);
+  RET(need_work(c, ws, need));
   F64Args a = f64args((int)nw, (int)K, (int)chunk);
   a.ktot = NM;
   a.A = G;  // batch (spin, chunk)
@@ -1036,13 +1046,13 @@ int dense_contract_f64(afqmc_ctx* c, Work& ws, const zd* G, const zd* Lt, zd* ou
 // the 2S partial products (spin, chunk) run as one batched GEMM into a
 // workspace and are then summed in FP64.
 template <int CP, class GT, class LT_>
-int dense_contract_vbias(afqmc_ctx* c, Work& ws, const void* Gp, const void* Lt, zd* out, const char* name,
+int dense_contract_vbias(afqmc_ctx* c, bool energy, const void* Gp, const void* Lt, zd* out, const char* name,
                          const uint32_t* G3 = nullptr, const uint32_t* Lt3 = nullptr,
                          const char* rname = "vbias_reduce", bool defer = false)
 {
   const long NM = (long)c->N * c->M, nw = c->nw, K = c->K;
   if constexpr (CP == CP_F64) {
-    if (NM >= 512) return dense_contract_f64(c, ws, (const zd*)Gp, (const zd*)Lt, out, name, rname, defer);
+    if (NM >= 512) return dense_contract_f64(c, energy, (const zd*)Gp, (const zd*)Lt, out, name, rname, defer);
   }
   const long tiles = ((nw + 127) / 128) * ((K + 63) / 64);
   int S = 1;
@@ -1050,7 +1060,9 @@ int dense_contract_vbias(afqmc_ctx* c, Work& ws, const void* Gp, const void* Lt,
   // partials in FP32 for the FP32/BF16 contractions, FP64 otherwise
   using PT = typename std::conditional<CP == CP_F64, double, float>::type;
   using PZ = typename ztype<PT>::type;
-  RET(need_work(c, ws, sizeof(PZ) * 2 * S * nw * K));
+  const size_t need = sizeof(PZ) * 2 * S * nw * K;
+  Work& ws = split_work(c, energy, need);
+  RET(need_work(c, ws, need));
   const long chunk = NM / S;
   ZGemmArgs a = gargs();
   a.A = Gp;  // batch b = (spin, chunk): A offset spin*NM + chunk*NM/S
@@ -1183,15 +1195,15 @@ int do_vbias(afqmc_ctx* c, bool defer = false)
                    (long)nw, c->vbias, (long)nw, one, zero, true);
   }
   if (c->mode == AFQMC_FP64_DENSE)
-    return dense_contract_vbias<CP_F64, double, double>(c, c->vws, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr,
+    return dense_contract_vbias<CP_F64, double, double>(c, false, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr,
                                                         nullptr, rn, defer);
   if (c->mode == AFQMC_MIXED_FP32)
-    return dense_contract_vbias<CP_F32, float, float>(c, c->vws, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr,
+    return dense_contract_vbias<CP_F32, float, float>(c, false, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr,
                                                       rn, defer);
   if (c->three & 1)
-    return dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, c->vws, c->G, c->Lt, c->vbias, "vbias_gemm", c->tp_G, c->tp_Lt,
+    return dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, false, c->G, c->Lt, c->vbias, "vbias_gemm", c->tp_G, c->tp_Lt,
                                                      rn, defer);
-  return dense_contract_vbias<CP_BF16X3, bfs, bfs>(c, c->vws, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
+  return dense_contract_vbias<CP_BF16X3, bfs, bfs>(c, false, c->G, c->Lt, c->vbias, "vbias_gemm", nullptr, nullptr, rn,
                                                    defer);
 }
 
@@ -1899,10 +1911,10 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
   // direct term: v(w,n) = sum Lt G ; direct = sum_n v^2 / dt
   if constexpr (CPV == CP_BF16X6) {
     // three pieces of the split G (built for the exchange) and of Lt
-    RET((dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, c->ews, c->G3, Lv, c->e_v, "energy_v_gemm", c->G3l, c->tp_Lt,
+    RET((dense_contract_vbias<CP_BF16X6, bfs, bfs>(c, true, c->G3, Lv, c->e_v, "energy_v_gemm", c->G3l, c->tp_Lt,
                                                    "energy_v_reduce")));
   } else {
-    RET((dense_contract_vbias<CPV, GT, LVT>(c, c->ews, Gp, Lv, c->e_v, "energy_v_gemm", nullptr, nullptr,
+    RET((dense_contract_vbias<CPV, GT, LVT>(c, true, Gp, Lv, c->e_v, "energy_v_gemm", nullptr, nullptr,
                                             "energy_v_reduce")));
   }
   constexpr bool G64 = std::is_same<GT, double>::value;
@@ -2030,11 +2042,13 @@ int energy_cholesky(afqmc_ctx* c, const void* Gp, const void* Lv, const void* Lx
     }
     // partials per walker-spin: enough workgroups for eight per CU
     const int ngrp = (int)std::max<long>(1, std::min<long>(cnt, 2048 / (2L * nw)));
-    RET(need_work(c, c->ews, sizeof(zd) * (size_t)ngrp * 2 * nw));
+    const size_t need = sizeof(zd) * (size_t)ngrp * 2 * nw;
+    Work& ws = split_work(c, true, need);
+    RET(need_work(c, ws, need));
     RET(launch(c, "energy_trace", [&]() {
       hipLaunchKernelGGL((trace_sq_kernel<typename ztype<YT>::type>), dim3(2 * nw, ngrp), dim3(256), 0, c->stream,
-                         (const typename ztype<YT>::type*)c->ybuf.p, N, cnt, (long)cnt * per_item, (zd*)c->ews.p, ngrp);
-      hipLaunchKernelGGL(add_parts_kernel, dim3((2 * nw + 255) / 256), dim3(256), 0, c->stream, (const zd*)c->ews.p,
+                         (const typename ztype<YT>::type*)c->ybuf.p, N, cnt, (long)cnt * per_item, (zd*)ws.p, ngrp);
+      hipLaunchKernelGGL(add_parts_kernel, dim3((2 * nw + 255) / 256), dim3(256), 0, c->stream, (const zd*)ws.p,
                          ngrp, c->e_exch_part, 2 * nw);
     }));
   }
@@ -2381,7 +2395,7 @@ int capture_prep(afqmc_ctx* c, int ortho)
   if (!c->transposed && !c->Gfull) RET(dalloc(c, &c->Gfull, 2L * c->M * c->M * c->nw));
   if (c->mode != AFQMC_FP64_CSR || c->sptd) {
     // the bias contraction's split-k workspace at its largest (at most 32
-    // chunks, also for the dense copy of SpvnT); nothing else uses it
+    // chunks, also for the dense copy of SpvnT), so that it stays where it is
     RET(need_work(c, c->vws, sizeof(zd) * 32 * (size_t)c->nw * c->K));
   }
   if (!c->t1inv_valid) RET(do_overlaps(c));

@@ -65,3 +65,33 @@ def test_dense_exchange_holds_its_block_only(require_gpu, mode, zs):
         g.close()
     say(used)
     assert abs(used[True] - used[False] - 2 * zs * (N * M) ** 2) < 6 * MB, used
+
+
+@pytest.mark.parametrize("mode", ["fp64_dense", "fp64_csr", "mixed_bf16"])
+@pytest.mark.parametrize("block", [True, False])
+def test_energy_after_capture_allocates_nothing(require_gpu, mode, block):
+    """The workspace of captured substeps (34 MB here) holds the energy's
+    partial sums too: one energy after another, none takes memory."""
+    M, N, K, nw = 96, 24, 128, 512
+    s = m.make_system(M, N, K, density=0.3, sigma_L=0.02, sigma_h=1.0, dt=0.005, seed=4)
+    took = {}
+    for i in range(2):  # the first one loads the kernels
+        say("energy after capture", mode, block, i)
+        g = m.AfqmcSys(s, nw, mode, dense_exchange=block)
+        g.init_walkers()
+        g.stage_fields(m.fields_block(4, K, nw, 0, 4))
+        g.use_graphs(True)
+        for t in range(2):
+            g.substep(t, False, s.dt)
+        g.calculate_mixed_density_matrix()
+        f0 = free_bytes()
+        g.calculate_energy()
+        g.substep(2, False, s.dt)
+        g.calculate_mixed_density_matrix()
+        g.calculate_energy()
+        took[i] = f0 - free_bytes()
+        g.close()
+    say(took)
+    # split-BF16's block has its two-piece G (19 MB) from the first energy on
+    extra = 8 * 2 * N * M * nw if block and mode == "mixed_bf16" else 0
+    assert abs(took[1] - extra) < 4 * MB, took
