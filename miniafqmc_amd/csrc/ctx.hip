@@ -3,8 +3,9 @@
 // Device layouts (HBM):
 //   AFQMC_FP64_CSR: the reference's own layouts (walker index last for
 //     G [2NM][W], vbias/X [K][W], vHS [M*M][W]) so every csrmm reads rows of
-//     walkers contiguously; vHS is transposed once per substep to [W][M*M]
-//     for the per-walker propagation.
+//     walkers contiguously; G is [W][2NM] where only dense products read it
+//     (g_wfirst); vHS is transposed once per substep to [W][M*M] for the
+//     per-walker propagation.
 //   dense modes: walker index first everywhere (G [W][2][N][M],
 //     vbias/X [W][K], vHS [W][M][M]) so each contraction is a GEMM whose
 //     operands are contiguous along the summed index; the Cholesky vectors
@@ -120,7 +121,7 @@ struct afqmc_ctx {
   double* brcum = nullptr;   // cumulative weights [nw]
   int* brparent = nullptr;   // parent of each new walker [nw]
   double* brw = nullptr;     // common weight after the comb
-  void* G = nullptr;      // CSR: zd [2NM][nw]; FP64_DENSE: zd [nw][2NM]; mixed: zf [nw][2NM]
+  void* G = nullptr;      // CSR: zd [2NM][nw] or [nw][2NM] (g_wfirst); FP64_DENSE: zd [nw][2NM]; mixed: zf [nw][2NM]
   zd* vbias = nullptr;    // CSR: [K][nw]; dense: [nw][K]
   void* X = nullptr;      // CSR: zd [K][nw]; dense: [nw][K] (zd / zf)
   void* vHS = nullptr;    // CSR: zd [M*M][nw]; dense: [nw][M*M] (zd / zf)
